@@ -1,0 +1,55 @@
+"""float32 products formed on the bfloat16 matrix pipe from three-term splits (MfmaX3): operands of any magnitude,
+the largest float32, infinities, and tile and k-chunk edges.
+
+Bound: S = sum of D products, the split keeping each to 2^-26 and the accumulator rounding at most once per term:
+|S - S64| <= (D + 8) 2^-24 sum |q| |k|, float32's own bound for a sum of D terms in any order."""
+
+import pytest
+import torch
+
+from theria_amd import _ops
+from theria_amd.attention.scores import triton_qk
+
+pytestmark = pytest.mark.gpu
+
+# k chunks of 16, subtiles of 32, tiles of 64 and blocks of 128 rows: one below, at and above
+SHAPES = [(1, 1, 1), (31, 33, 15), (32, 32, 16), (33, 64, 17), (128, 65, 32), (129, 63, 33), (64, 130, 64), (70, 40, 100),
+          (33, 31, 127), (130, 129, 128)]
+
+
+@pytest.mark.parametrize("T,M,D", SHAPES)
+def test_scores_of_operands_over_many_magnitudes(T, M, D):
+    print(f"float32 split scores T{T} M{M} D{D}", flush=True)
+    g = torch.Generator().manual_seed(T * 1000 + M * 10 + D)
+
+    def wide(rows):  # magnitudes 2^-20 .. 2^20 within every row
+        return torch.randn(1, 2, rows, D, generator=g) * torch.exp2(torch.randint(-20, 21, (1, 2, rows, D), generator=g).float())
+
+    q, k = wide(T), wide(M)
+    s = triton_qk(q.cuda(), k.cuda()).double().cpu()
+    ref = q.double() @ k.double().transpose(-2, -1)
+    bound = (D + 8) * 2.0**-24 * (q.double().abs() @ k.double().abs().transpose(-2, -1))
+    assert ((s - ref).abs() <= bound).all(), float(((s - ref).abs() / bound).max())
+
+
+@pytest.mark.parametrize("D", [16, 64, 128])
+def test_largest_values_and_infinities(D):
+    """The lowest float32 and -infinity in a key mask it (its scores are far below the others), the largest one in
+    V stays finite in O, and an infinite V reaches O's column and no other, as in float32."""
+    print(f"float32 split extremes D{D}", flush=True)
+    g = torch.Generator().manual_seed(D)
+    q = torch.rand(1, 1, 40, D, generator=g) + 0.5  # positive: every score of a masked key is negative
+    k, v = (torch.randn(1, 1, 70, D, generator=g) for _ in range(2))
+    big = torch.finfo(torch.float32).max
+    k[0, 0, 3, 0] = -big
+    k[0, 0, 68, 1] = -float("inf")
+    v[0, 0, 5, 2] = big
+    v[0, 0, 7, 4] = float("inf")
+    o = _ops.fwd(q.cuda(), k.cuda(), v.cuda(), D**-0.5, False)[0].cpu()
+    keep = [j for j in range(70) if j not in (3, 68)]
+    p = torch.softmax(q.double() @ k[:, :, keep].double().transpose(-2, -1) * D**-0.5, -1)
+    ref = p @ v[:, :, keep].double()
+    assert torch.isinf(o[..., 4]).all() and (o[..., 4] > 0).all()
+    cols = [d for d in range(D) if d not in (2, 4)]
+    torch.testing.assert_close(o[..., cols].double(), ref[..., cols], rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(o[..., 2].double(), ref[..., 2], rtol=1e-4, atol=0.0)  # P of one key, scaled by 3.4e38

@@ -43,13 +43,14 @@
 
 namespace theria {
 
-template <typename T, int DP, bool CAUSAL, int QT>
+// X3: float32 products by three-term bfloat16 splits (MfmaX3).
+template <typename T, int DP, bool CAUSAL, int QT, bool X3>
 __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const DqParams p) {
-  using MM = Mfma<T>;
-  using F = typename MM::frag_t;
-  constexpr int KC = MM::KC;
+  using OP = Ops<T, DP, X3>;
+  using F = typename OP::F;
+  constexpr int KC = OP::KC;
   constexpr int NW = 4, BM = 32 * NW * QT, BN = 32, NT = 64 * NW;
-  constexpr int PITCH = DP + 16 / (int)sizeof(T);
+  constexpr int PITCH = OP::PITCH;
   constexpr int NDT = DP / 32, NKC = DP / KC, NPC = 32 / KC;
   __shared__ __attribute__((aligned(16))) T sK[BN * PITCH];
   __shared__ __attribute__((aligned(16))) T sV[BN * PITCH];
@@ -78,8 +79,8 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
     const bool qvalid = myq < s.T;
 #pragma unroll
     for (int c = 0; c < NKC; ++c) {
-      qf[j][c] = gload_frag<T>(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
-      of[j][c] = gload_frag<T>(dO, p.dout.sr, myq, s.T, c, s.D, s.vec);
+      qf[j][c] = OP::gload(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
+      of[j][c] = OP::gload(dO, p.dout.sr, myq, s.T, c, s.D, s.vec);
     }
     const float lse = qvalid ? p.lse[rowbase + myq] : THERIA_INF;
     lse2[j] = lse == -THERIA_INF ? THERIA_INF : lse * kLog2e;  // a row without visible keys has P = 0
@@ -145,8 +146,8 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
       pK.load(K, p.k.sr, k0, s.M, s.D, s.vec);
       pV.load(V, p.v.sr, k0, s.M, s.D, s.vec);
       __syncthreads();
-      pK.store(sK, PITCH);
-      pV.store(sV, PITCH);
+      OP::store(pK, sK);
+      OP::store(pV, sV);
       __syncthreads();
       if (CAUSAL && k0 > q0w + 32 * QT - 1) continue;
       f32x16_t sc[QT], dpp[QT];
@@ -154,12 +155,12 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
       for (int j = 0; j < QT; ++j) sc[j] = dpp[j] = zero16();
 #pragma unroll
       for (int c = 0; c < NKC; ++c) {
-        const F kfr = lds_cols<T, KLIN>(sK, PITCH, li, 0, c);
-        const F vfr = lds_cols<T, KLIN>(sV, PITCH, li, 0, c);
+        const F kfr = OP::cols(sK, li, c);
+        const F vfr = OP::cols(sV, li, c);
 #pragma unroll
         for (int j = 0; j < QT; ++j) {
-          sc[j] = MM::mma(kfr, qf[j][c], sc[j]);
-          dpp[j] = MM::mma(vfr, of[j][c], dpp[j]);
+          sc[j] = OP::mma(kfr, qf[j][c], sc[j]);
+          dpp[j] = OP::mma(vfr, of[j][c], dpp[j]);
         }
       }
 #pragma unroll
@@ -240,8 +241,8 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
   for (int kt = 0; kt < nkt; ++kt) {
     const int k0 = kt * BN;
     __syncthreads();
-    stK.store(sK, PITCH);
-    stV.store(sV, PITCH);
+    OP::store(stK, sK);
+    OP::store(stV, sV);
     __syncthreads();
     if (kt + 1 < nkt) {
       stK.load(K, p.k.sr, k0 + BN, s.M, s.D, s.vec);
@@ -262,12 +263,12 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
     }
 #pragma unroll
     for (int c = 0; c < NKC; ++c) {
-      const F kfr = lds_cols<T, KLIN>(sK, PITCH, li, 0, c);
-      const F vfr = lds_cols<T, KLIN>(sV, PITCH, li, 0, c);
+      const F kfr = OP::cols(sK, li, c);
+      const F vfr = OP::cols(sV, li, c);
 #pragma unroll
       for (int j = 0; j < QT; ++j) {
-        sc[j] = MM::mma(kfr, qf[j][c], sc[j]);
-        dp[j] = MM::mma(vfr, of[j][c], dp[j]);
+        sc[j] = OP::mma(kfr, qf[j][c], sc[j]);
+        dp[j] = OP::mma(vfr, of[j][c], dp[j]);
       }
     }
     // Boundary tiles only (a uniform branch): masked scores become -inf, so P = 0 there.
@@ -293,16 +294,16 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
         if constexpr (SPLIT) {
           split_frag<T>(sc[j], cc, dsf[j], dsl[j]);
         } else {
-          dsf[j] = acc_frag<T>(sc[j], cc);
+          dsf[j] = OP::acc(sc[j], cc);
         }
       }
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt) {
-        const F ktf = lds_rows<T, KACC>(sK, PITCH, 0, cc, dt * 32);
+        const F ktf = OP::rows(sK, 0, cc, dt * 32);
 #pragma unroll
         for (int j = 0; j < QT; ++j) {
-          acc[j][dt] = MM::mma(ktf, dsf[j], acc[j][dt]);
-          if constexpr (SPLIT) acc[j][dt] = MM::mma(ktf, dsl[j], acc[j][dt]);
+          acc[j][dt] = OP::mma(ktf, dsf[j], acc[j][dt]);
+          if constexpr (SPLIT) acc[j][dt] = OP::mma(ktf, dsl[j], acc[j][dt]);
         }
       }
     }
@@ -335,12 +336,12 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
 
 template <typename T, int DP, bool CAUSAL, int KT, bool DV_ONLY>
 __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(const DkdvParams p) {
-  using MM = Mfma<T>;
-  using F = typename MM::frag_t;
-  constexpr int KC = MM::KC;
+  using OP = Ops<T, DP, sizeof(T) == 4>;
+  using F = typename OP::F;
+  constexpr int KC = OP::KC;
   constexpr int NW = 4, BN = 32 * NW * KT, NT = 64 * NW;
   constexpr int BM = sizeof(T) == 2 ? 64 : 32;
-  constexpr int PITCH = DP + 16 / (int)sizeof(T);
+  constexpr int PITCH = OP::PITCH;
   constexpr int NDT = DP / 32, NKC = DP / KC, NPC = 32 / KC, NQT = BM / 32;
   __shared__ __attribute__((aligned(16))) T sQ[BM * PITCH];
   __shared__ __attribute__((aligned(16))) T sdO[BM * PITCH];
@@ -368,7 +369,7 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(c
   for (int t = 0; t < KT; ++t)
 #pragma unroll
     for (int c = 0; c < NKC; ++c) {
-      kf[t][c] = gload_frag<T>(K, p.k.sr, kw0 + 32 * t + li, s.M, c, s.D, s.vec);
+      kf[t][c] = OP::gload(K, p.k.sr, kw0 + 32 * t + li, s.M, c, s.D, s.vec);
       vf[t][c] = F{};
     }
   if constexpr (!DV_ONLY) {
@@ -376,7 +377,7 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(c
 #pragma unroll
     for (int t = 0; t < KT; ++t)
 #pragma unroll
-      for (int c = 0; c < NKC; ++c) vf[t][c] = gload_frag<T>(V, p.v.sr, kw0 + 32 * t + li, s.M, c, s.D, s.vec);
+      for (int c = 0; c < NKC; ++c) vf[t][c] = OP::gload(V, p.v.sr, kw0 + 32 * t + li, s.M, c, s.D, s.vec);
   }
   f32x16_t dv[KT][NDT], dk[KT][NDT];
 #pragma unroll
@@ -420,13 +421,13 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(c
     }
 #pragma unroll
     for (int c = 0; c < NKC; ++c) {
-      const F qfr = lds_cols<T, KLIN>(sQ, PITCH, qr0 + li, 0, c);
+      const F qfr = OP::cols(sQ, qr0 + li, c);
 #pragma unroll
-      for (int t = 0; t < KT; ++t) sc[t] = MM::mma(qfr, kf[t][c], sc[t]);
+      for (int t = 0; t < KT; ++t) sc[t] = OP::template mma<true>(qfr, kf[t][c], sc[t]);
       if constexpr (!DV_ONLY) {
-        const F ofr = lds_cols<T, KLIN>(sdO, PITCH, qr0 + li, 0, c);
+        const F ofr = OP::cols(sdO, qr0 + li, c);
 #pragma unroll
-        for (int t = 0; t < KT; ++t) dp[t] = MM::mma(ofr, vf[t][c], dp[t]);
+        for (int t = 0; t < KT; ++t) dp[t] = OP::template mma<true>(ofr, vf[t][c], dp[t]);
       }
     }
     // Boundary sub-tiles only (a uniform branch): masked scores become -inf, so P = 0 there.
@@ -444,8 +445,8 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(c
   for (int it = 0; it < nqt; ++it) {
     const int q0 = qbeg + it * BM;
     __syncthreads();
-    stQ.store(sQ, PITCH);
-    stO.store(sdO, PITCH);
+    OP::store(stQ, sQ);
+    OP::store(stO, sdO);
     if (tid < BM) {
       sLse[tid] = pre_lse;
       sDel[tid] = pre_del;
@@ -481,21 +482,21 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(c
       for (int cc = 0; cc < NPC; ++cc) {
         F ot[NDT], qtr[NDT];
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) ot[dt] = lds_rows<T, KACC>(sdO, PITCH, qr0, cc, dt * 32);
+        for (int dt = 0; dt < NDT; ++dt) ot[dt] = OP::rows(sdO, qr0, cc, dt * 32);
 #pragma unroll
         for (int t = 0; t < KT; ++t) {
-          const F pa = acc_frag<T>(sc[t], cc);
+          const F pa = OP::acc(sc[t], cc);
 #pragma unroll
-          for (int dt = 0; dt < NDT; ++dt) dv[t][dt] = MM::mma(pa, ot[dt], dv[t][dt]);
+          for (int dt = 0; dt < NDT; ++dt) dv[t][dt] = OP::mma(pa, ot[dt], dv[t][dt]);
         }
         if constexpr (!DV_ONLY) {
 #pragma unroll
-          for (int dt = 0; dt < NDT; ++dt) qtr[dt] = lds_rows<T, KACC>(sQ, PITCH, qr0, cc, dt * 32);
+          for (int dt = 0; dt < NDT; ++dt) qtr[dt] = OP::rows(sQ, qr0, cc, dt * 32);
 #pragma unroll
           for (int t = 0; t < KT; ++t) {
-            const F da = acc_frag<T>(dp[t], cc);
+            const F da = OP::acc(dp[t], cc);
 #pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) dk[t][dt] = MM::mma(da, qtr[dt], dk[t][dt]);
+            for (int dt = 0; dt < NDT; ++dt) dk[t][dt] = OP::mma(da, qtr[dt], dk[t][dt]);
           }
         }
       }
@@ -529,8 +530,8 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(c
               }
 #pragma unroll
               for (int dt = 0; dt < NDT; ++dt) {
-                dv[t][dt] = MM::mma(pl, lds_rows<T, KACC>(sdO, PITCH, qr0, cc, dt * 32), dv[t][dt]);
-                if constexpr (!DV_ONLY) dk[t][dt] = MM::mma(dl, lds_rows<T, KACC>(sQ, PITCH, qr0, cc, dt * 32), dk[t][dt]);
+                dv[t][dt] = OP::mma(pl, OP::rows(sdO, qr0, cc, dt * 32), dv[t][dt]);
+                if constexpr (!DV_ONLY) dk[t][dt] = OP::mma(dl, OP::rows(sQ, qr0, cc, dt * 32), dk[t][dt]);
               }
             }
           }
@@ -578,11 +579,20 @@ struct DqLauncher {
     if (nblk == 0) return hipSuccess;
     if constexpr (DP <= 64 && sizeof(T) == 2) {
       if (qt == 2) {
-        hipLaunchKernelGGL((dq_kernel<T, DP, CAUSAL, 2>), dim3((unsigned)nblk), dim3(256), 0, st, p);
+        hipLaunchKernelGGL((dq_kernel<T, DP, CAUSAL, 2, false>), dim3((unsigned)nblk), dim3(256), 0, st, p);
         return hipGetLastError();
       }
     }
-    hipLaunchKernelGGL((dq_kernel<T, DP, CAUSAL, 1>), dim3((unsigned)nblk), dim3(256), 0, st, p);
+    // The row statistics of the double backward must come from the same products as its row and column kernels
+    // form (kRowOwnStats): native float32 ones at head dim 128, where the split fragments would not fit theirs.
+    if constexpr (sizeof(T) == 4) {
+      if (!(DP == 128 && p.row_term == kRowOwnStats)) {
+        hipLaunchKernelGGL((dq_kernel<T, DP, CAUSAL, 1, true>), dim3((unsigned)nblk), dim3(256), 0, st, p);
+        return hipGetLastError();
+      }
+    }
+    if constexpr (sizeof(T) == 2 || DP == 128)
+      hipLaunchKernelGGL((dq_kernel<T, DP, CAUSAL, 1, false>), dim3((unsigned)nblk), dim3(256), 0, st, p);
     return hipGetLastError();
   }
 };

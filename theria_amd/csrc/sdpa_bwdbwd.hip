@@ -51,13 +51,13 @@ namespace theria {
 // registers and schedule.
 template <typename T, int DP, bool CAUSAL, bool DMA, bool EXACT>
 __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdParams& p, const int blk, const int nblk) {
-  using MM = Mfma<T>;
-  using F = typename MM::frag_t;
-  constexpr int KC = MM::KC;
+  using OP = Ops<T, DP, (sizeof(T) == 4 && DP <= 64)>;
+  using F = typename OP::F;
+  constexpr int KC = OP::KC;
   constexpr int NW = 4, BM = 32 * NW, NT = 64 * NW;
   // keys per tile: two 32-key subtiles per tile where the registers allow (one wave per SIMD)
   constexpr int BN = (DP == 128 || sizeof(T) == 4 || DMA) ? 32 : 64;
-  constexpr int PITCH = DP + 16 / (int)sizeof(T);
+  constexpr int PITCH = OP::PITCH;
   constexpr int NDT = DP / 32, NKC = DP / KC, NPC = 32 / KC, NST = BN / 32;
   constexpr int TB = DMA ? BN * DP * 2 : BN * PITCH * (int)sizeof(T);  // bytes per tile
   constexpr int TB2 = DMA ? TB : 16;                                    // second set (DMA only)
@@ -108,9 +108,9 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
   F qf[NKC], dof[NKC], gqf[NKC];
 #pragma unroll
   for (int c = 0; c < NKC; ++c) {
-    qf[c] = gload_frag<T>(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
-    dof[c] = gload_frag<T>(dO, p.dout.sr, myq, s.T, c, s.D, s.vec);
-    gqf[c] = has_gq ? gload_frag<T>(GQ, p.gq.sr, myq, s.T, c, s.D, s.vec) : F{};
+    qf[c] = OP::gload(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
+    dof[c] = OP::gload(dO, p.dout.sr, myq, s.T, c, s.D, s.vec);
+    gqf[c] = has_gq ? OP::gload(GQ, p.gq.sr, myq, s.T, c, s.D, s.vec) : F{};
   }
   f32x16_t x13[NDT], x2[NDT], x4[NDT], yk[NDT];
 #pragma unroll
@@ -147,13 +147,13 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
     if constexpr (DMA)
       return swz_cols<T, DP>(t, row, c);
     else
-      return lds_cols<T, KLIN>((const T*)t, PITCH, row, 0, c);
+      return OP::cols((const T*)t, row, c);
   };
   auto rowsf = [&](const char* t, int kbase, int c, int col0) -> F {
     if constexpr (DMA)
       return swz_rows<T, DP>(t, kbase, c, col0);
     else
-      return lds_rows<T, KACC>((const T*)t, PITCH, kbase, c, col0);
+      return OP::rows((const T*)t, kbase, c, col0);
   };
 
   // The key tile kt held in (tK, tV, tgK, tgV), as 32-key subtiles.
@@ -175,11 +175,11 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
 #pragma unroll
       for (int c = 0; c < NKC; ++c) {
         const F kfr = colsf(tK, 32 * st + li, c);
-        sc = MM::mma(kfr, qf[c], sc);
-        dpz = MM::mma(colsf(tV, 32 * st + li, c), dof[c], dpz);
-        if (has_gq) gm = MM::mma(kfr, gqf[c], gm);
-        if (has_gk) gm = MM::mma(colsf(tgK, 32 * st + li, c), qf[c], gm);
-        if (has_gv) w = MM::mma(colsf(tgV, 32 * st + li, c), dof[c], w);
+        sc = OP::mma(kfr, qf[c], sc);
+        dpz = OP::mma(colsf(tV, 32 * st + li, c), dof[c], dpz);
+        if (has_gq) gm = OP::mma(kfr, gqf[c], gm);
+        if (has_gk) gm = OP::mma(colsf(tgK, 32 * st + li, c), qf[c], gm);
+        if (has_gv) w = OP::mma(colsf(tgV, 32 * st + li, c), dof[c], w);
       }
       const bool need_mask = (k0s + 32 > s.M) || (CAUSAL && k0s + 31 > q0w);
 #pragma unroll
@@ -220,12 +220,12 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
 #pragma unroll
           for (int dt = 0; dt < NDT; ++dt) {
             const F kr = rowsf(tK, 32 * st, cc, dt * 32);
-            x13[dt] = MM::mma(kr, gh, x13[dt]);
-            x13[dt] = MM::mma(kr, gl, x13[dt]);
+            x13[dt] = OP::mma(kr, gh, x13[dt]);
+            x13[dt] = OP::mma(kr, gl, x13[dt]);
             if (has_gk) {
               const F gkr = rowsf(tgK, 32 * st, cc, dt * 32);
-              yk[dt] = MM::mma(gkr, dh, yk[dt]);
-              yk[dt] = MM::mma(gkr, dl, yk[dt]);
+              yk[dt] = OP::mma(gkr, dh, yk[dt]);
+              yk[dt] = OP::mma(gkr, dl, yk[dt]);
             }
           }
         }
@@ -233,17 +233,17 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
       }
 #pragma unroll
       for (int cc = 0; cc < NPC; ++cc) {
-        const F pf = acc_frag<T>(sc, cc);
-        const F pe1f = acc_frag<T>(gm, cc);
-        const F dsf = acc_frag<T>(dpz, cc);
+        const F pf = OP::acc(sc, cc);
+        const F pe1f = OP::acc(gm, cc);
+        const F dsf = OP::acc(dpz, cc);
         if constexpr (sizeof(T) == 2) t_frag = frag_sum<T>(pe1f, t_frag);
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) {
           const F kr = rowsf(tK, 32 * st, cc, dt * 32);
-          x13[dt] = MM::mma(kr, pe1f, x13[dt]);
-          x2[dt] = MM::mma(kr, dsf, x2[dt]);
-          x4[dt] = MM::mma(kr, pf, x4[dt]);
-          if (has_gk) yk[dt] = MM::mma(rowsf(tgK, 32 * st, cc, dt * 32), dsf, yk[dt]);
+          x13[dt] = OP::mma(kr, pe1f, x13[dt]);
+          x2[dt] = OP::mma(kr, dsf, x2[dt]);
+          x4[dt] = OP::mma(kr, pf, x4[dt]);
+          if (has_gk) yk[dt] = OP::mma(rowsf(tgK, 32 * st, cc, dt * 32), dsf, yk[dt]);
         }
       }
     }
@@ -342,10 +342,10 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
     auto sweep = [&](auto pass_tag) __attribute__((always_inline)) {
       for (int kt = 0; kt < nkt; ++kt) {
         __syncthreads();
-        gsK.store((T*)sK0, PITCH);
-        gsV.store((T*)sV0, PITCH);
-        if (has_gk) gsgK.store((T*)sgK0, PITCH);
-        if (has_gv) gsgV.store((T*)sgV0, PITCH);
+        OP::store(gsK, (T*)sK0);
+        OP::store(gsV, (T*)sV0);
+        if (has_gk) OP::store(gsgK, (T*)sgK0);
+        if (has_gv) OP::store(gsgV, (T*)sgV0);
         __syncthreads();
         if (kt + 1 < nkt) prefetch((kt + 1) * BN);
         compute(pass_tag, kt, sK0, sV0, sgK0, sgV0);
@@ -364,10 +364,10 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
     } else {
       if (sizeof(T) == 2 && nkt > 0) {
         // centre pre-pass over tile 0 (the loop stages the same registers again)
-        gsK.store((T*)sK0, PITCH);
-        gsV.store((T*)sV0, PITCH);
-        if (has_gk) gsgK.store((T*)sgK0, PITCH);
-        if (has_gv) gsgV.store((T*)sgV0, PITCH);
+        OP::store(gsK, (T*)sK0);
+        OP::store(gsV, (T*)sV0);
+        if (has_gk) OP::store(gsgK, (T*)sgK0);
+        if (has_gv) OP::store(gsgV, (T*)sgV0);
         __syncthreads();
         compute(pre_pass, 0, sK0, sV0, sgK0, sgV0);
         set_centre();
@@ -412,13 +412,13 @@ __global__ __launch_bounds__(256) void bwdbwd_rows_kernel(const BwdBwdParams p) 
 // first BM threads and written beside them one tile ahead).
 template <typename T, int DP, bool CAUSAL, bool DMA>
 __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdParams& p, const int blk, const int nblk) {
-  using MM = Mfma<T>;
-  using F = typename MM::frag_t;
-  constexpr int KC = MM::KC;
+  using OP = Ops<T, DP, (sizeof(T) == 4 && DP <= 64)>;
+  using F = typename OP::F;
+  constexpr int KC = OP::KC;
   constexpr int NW = 4, BN = 32 * NW, NT = 64 * NW;
   // queries per tile: two 32-query subtiles per tile where the registers allow
   constexpr int BM = (DP == 128 || sizeof(T) == 4 || DMA) ? 32 : 64;
-  constexpr int PITCH = DP + 16 / (int)sizeof(T);
+  constexpr int PITCH = OP::PITCH;
   constexpr int NDT = DP / 32, NKC = DP / KC, NPC = 32 / KC, NSQ = BM / 32;
   constexpr int TB = DMA ? BM * DP * 2 : BM * PITCH * (int)sizeof(T);  // bytes per tile
   constexpr int TB2 = DMA ? TB : 16;                                    // second set (DMA only)
@@ -462,10 +462,10 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
   F kf[NKC], vf[NKC], gkf[NKC], gvf[NKC];
 #pragma unroll
   for (int c = 0; c < NKC; ++c) {
-    kf[c] = gload_frag<T>(K, p.k.sr, mykey, s.M, c, s.D, s.vec);
-    vf[c] = gload_frag<T>(V, p.v.sr, mykey, s.M, c, s.D, s.vec);
-    gkf[c] = has_gk ? gload_frag<T>(GK, p.gk.sr, mykey, s.M, c, s.D, s.vec) : F{};
-    gvf[c] = has_gv ? gload_frag<T>(GV, p.gv.sr, mykey, s.M, c, s.D, s.vec) : F{};
+    kf[c] = OP::gload(K, p.k.sr, mykey, s.M, c, s.D, s.vec);
+    vf[c] = OP::gload(V, p.v.sr, mykey, s.M, c, s.D, s.vec);
+    gkf[c] = has_gk ? OP::gload(GK, p.gk.sr, mykey, s.M, c, s.D, s.vec) : F{};
+    gvf[c] = has_gv ? OP::gload(GV, p.gv.sr, mykey, s.M, c, s.D, s.vec) : F{};
   }
   f32x16_t accV[NDT], accK[NDT];
 #pragma unroll
@@ -482,13 +482,13 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
     if constexpr (DMA)
       return swz_cols<T, DP>(t, row, c);
     else
-      return lds_cols<T, KLIN>((const T*)t, PITCH, row, 0, c);
+      return OP::cols((const T*)t, row, c);
   };
   auto rowsf = [&](const char* t, int kbase, int c, int col0) -> F {
     if constexpr (DMA)
       return swz_rows<T, DP>(t, kbase, c, col0);
     else
-      return lds_rows<T, KACC>((const T*)t, PITCH, kbase, c, col0);
+      return OP::rows((const T*)t, kbase, c, col0);
   };
 
   // Row terms of a tile for thread tid < BM, held raw (rows past the end: lse = +inf) and converted when
@@ -547,11 +547,11 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
       for (int c = 0; c < NKC; ++c) {
         const F qfr = colsf(tQ, 32 * sq + li, c);
         const F ofr = colsf(tO, 32 * sq + li, c);
-        sc = MM::mma(qfr, kf[c], sc);
-        dpz = MM::mma(ofr, vf[c], dpz);
-        if (has_gq) gm = MM::mma(colsf(tgQ, 32 * sq + li, c), kf[c], gm);
-        if (has_gk) gm = MM::mma(qfr, gkf[c], gm);
-        if (has_gv) w = MM::mma(ofr, gvf[c], w);
+        sc = OP::template mma<true>(qfr, kf[c], sc);
+        dpz = OP::template mma<true>(ofr, vf[c], dpz);
+        if (has_gq) gm = OP::template mma<true>(colsf(tgQ, 32 * sq + li, c), kf[c], gm);
+        if (has_gk) gm = OP::template mma<true>(qfr, gkf[c], gm);
+        if (has_gv) w = OP::template mma<true>(ofr, gvf[c], w);
       }
       const bool diag = CAUSAL && (kw0 + 31 > q0s);
       f32x16_t gdp, gs;
@@ -579,29 +579,29 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
 #pragma unroll
           for (int dt = 0; dt < NDT; ++dt) {
             const F ro = rowsf(tO, 32 * sq, cc, dt * 32);
-            accV[dt] = MM::mma(gdph, ro, accV[dt]);
-            accV[dt] = MM::mma(gdpl, ro, accV[dt]);
+            accV[dt] = OP::mma(gdph, ro, accV[dt]);
+            accV[dt] = OP::mma(gdpl, ro, accV[dt]);
             const F rq = rowsf(tQ, 32 * sq, cc, dt * 32);
-            accK[dt] = MM::mma(gsh, rq, accK[dt]);
-            accK[dt] = MM::mma(gsl, rq, accK[dt]);
+            accK[dt] = OP::mma(gsh, rq, accK[dt]);
+            accK[dt] = OP::mma(gsl, rq, accK[dt]);
             if (has_gq) {
               const F rg = rowsf(tgQ, 32 * sq, cc, dt * 32);
-              accK[dt] = MM::mma(dsh, rg, accK[dt]);
-              accK[dt] = MM::mma(dsl, rg, accK[dt]);
+              accK[dt] = OP::mma(dsh, rg, accK[dt]);
+              accK[dt] = OP::mma(dsl, rg, accK[dt]);
             }
           }
         }
       } else {
 #pragma unroll
         for (int cc = 0; cc < NPC; ++cc) {
-          const F gdpf = acc_frag<T>(gdp, cc);
-          const F gsf = acc_frag<T>(gs, cc);
-          const F dsf = acc_frag<T>(dpz, cc);
+          const F gdpf = OP::acc(gdp, cc);
+          const F gsf = OP::acc(gs, cc);
+          const F dsf = OP::acc(dpz, cc);
 #pragma unroll
           for (int dt = 0; dt < NDT; ++dt) {
-            accV[dt] = MM::mma(gdpf, rowsf(tO, 32 * sq, cc, dt * 32), accV[dt]);
-            accK[dt] = MM::mma(gsf, rowsf(tQ, 32 * sq, cc, dt * 32), accK[dt]);
-            if (has_gq) accK[dt] = MM::mma(dsf, rowsf(tgQ, 32 * sq, cc, dt * 32), accK[dt]);
+            accV[dt] = OP::mma(gdpf, rowsf(tO, 32 * sq, cc, dt * 32), accV[dt]);
+            accK[dt] = OP::mma(gsf, rowsf(tQ, 32 * sq, cc, dt * 32), accK[dt]);
+            if (has_gq) accK[dt] = OP::mma(dsf, rowsf(tgQ, 32 * sq, cc, dt * 32), accK[dt]);
           }
         }
       }
@@ -710,9 +710,9 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
     if (nqt > 0) prefetch(0);
     for (int it = 0; it < nqt; ++it) {
       __syncthreads();
-      gsQ.store((T*)sQ0, PITCH);
-      gsO.store((T*)sdO0, PITCH);
-      if (has_gq) gsgQ.store((T*)sgQ0, PITCH);
+      OP::store(gsQ, (T*)sQ0);
+      OP::store(gsO, (T*)sdO0);
+      if (has_gq) OP::store(gsgQ, (T*)sgQ0);
       store_rows(sRow0);
       __syncthreads();
       if (it + 1 < nqt) prefetch(it + 1);
@@ -721,9 +721,9 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
     if (pk_any)
       peaked_tiles([&](int it) __attribute__((always_inline)) {
         prefetch(it);
-        gsQ.store((T*)sQ0, PITCH);
-        gsO.store((T*)sdO0, PITCH);
-        if (has_gq) gsgQ.store((T*)sgQ0, PITCH);
+        OP::store(gsQ, (T*)sQ0);
+        OP::store(gsO, (T*)sdO0);
+        if (has_gq) OP::store(gsgQ, (T*)sgQ0);
         store_rows(sRow0);
       });
   }

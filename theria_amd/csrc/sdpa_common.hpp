@@ -2,8 +2,9 @@
 //
 // Tiling vocabulary used by every kernel:
 //  * All matrix products use 32x32 MFMA output tiles. For 16-bit inputs the instruction is
-//    v_mfma_f32_32x32x16_{bf16,f16} (k extent 16, 8 elements per lane); for float32 inputs it is
-//    v_mfma_f32_32x32x2_f32 (k extent 2, 1 element per lane). Accumulation is float32 in both.
+//    v_mfma_f32_32x32x16_{bf16,f16} (k extent 16, 8 elements per lane); for float32 inputs it is either
+//    v_mfma_f32_32x32x2_f32 (k extent 2, 1 element per lane) or six v_mfma_f32_32x32x16_bf16 over operands split
+//    into three bfloat16 terms (MfmaX3 below). Accumulation is float32 in all.
 //  * Operand fragment of lane l (li = l % 32, g = l / 32): the row (A) or column (B) index is li, and
 //    the k elements depend on g. Output ("accumulator") layout: register r of lane l holds the element
 //    at row acc_row(r, g) = 8*(r/4) + 4*g + r%4 and column li. These layouts were checked bit-exactly
@@ -73,6 +74,35 @@ template <> struct Mfma<float> {
   static constexpr int EPL = 1;
   __device__ __forceinline__ static f32x16_t mma(frag_t a, frag_t b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+  }
+};
+
+// float32 products on the bfloat16 matrix pipe. Each operand is split into three bfloat16 terms, h = bf16(x),
+// m = bf16(x - h), l = bf16(x - h - m), which hold all 24 bits of it (rounding to nearest leaves |m| <= 2^-9 |x|
+// and |l| <= 2^-18 |x|), and a b is summed as the six products down to 2^-18: the three dropped ones (m l, l m,
+// l l) are below 2^-26 of it, under float32's own rounding. One 16-wide k chunk then takes 6 x 32 cycles of the
+// matrix pipe where eight v_mfma_f32_32x32x2_f32 take 8 x 64, and rounds the accumulator fewer times.
+// Measured against the native float32 products: forward + backward of B2 H16 T1000 D64 460 -> 310 us, the HVP of
+// B8 H8 T512 D64 783 -> 554 us; relative error against float64 7.4e-7 -> 6.4e-7 and 7.4e-7 -> 6.3e-7, and not
+// larger in any of 25 float32 calls over B 1..468, T and M 6..3638, D 16..128.
+struct X3Frag {
+  bf16x8_t h, m, l;
+};
+struct MfmaX3 {
+  using frag_t = X3Frag;
+  static constexpr int KC = 16;
+  static constexpr int EPL = 8;
+  // Smallest products first. SW: the roles of a and b exchanged in that order, so that a product formed with its
+  // operands swapped (S and S^T) rounds identically.
+  template <bool SW = false>
+  __device__ __forceinline__ static f32x16_t mma(const frag_t& a, const frag_t& b, f32x16_t c) {
+    using M = Mfma<__bf16>;
+    c = M::mma(a.m, b.m, c);
+    c = SW ? M::mma(a.h, b.l, c) : M::mma(a.l, b.h, c);
+    c = SW ? M::mma(a.l, b.h, c) : M::mma(a.h, b.l, c);
+    c = SW ? M::mma(a.h, b.m, c) : M::mma(a.m, b.h, c);
+    c = SW ? M::mma(a.m, b.h, c) : M::mma(a.h, b.m, c);
+    return M::mma(a.h, b.h, c);
   }
 };
 
@@ -217,9 +247,8 @@ __device__ __forceinline__ typename Mfma<T>::frag_t scaled_frag(const typename M
 // Two-term 16-bit split of accumulator chunk c (16-bit T only): hi = round(x), lo = round(x - hi), so
 // hi + lo carries x to ~2^-16 relative and an MFMA pair over (hi, lo) sums x-weighted products with no
 // operand rounding of consequence.
-template <typename T>
-__device__ __forceinline__ void split_frag(const f32x16_t& a, int c, typename Mfma<T>::frag_t& hi,
-                                           typename Mfma<T>::frag_t& lo) {
+template <typename T, typename F>
+__device__ __forceinline__ void split_frag(const f32x16_t& a, int c, F& hi, F& lo) {
   static_assert(sizeof(T) == 2, "split_frag is for 16-bit operands");
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
@@ -406,5 +435,140 @@ __device__ __forceinline__ f32x4_t load4(const T* base, int64_t rs, int row, int
   }
   return out;
 }
+
+// ----------------------------------------------------------------------------------------------
+// float32 as three bfloat16 terms (MfmaX3)
+// ----------------------------------------------------------------------------------------------
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+
+// Element i of a register array of 8 floats -> element i of the three terms. CLAMP: values beyond bfloat16's
+// largest (a finite float32 there would round to infinity) take that value as their first term; an infinity then
+// ends up in l, which only meets the other operand's h, so that products with it stay infinite (NaN against 0)
+// as in float32, and a NaN reaches l the same way.
+template <bool CLAMP>
+__device__ __forceinline__ X3Frag split3(const float (&x)[8]) {
+  constexpr float kBig = 3.3895313892515355e38f;  // the largest finite bfloat16
+  X3Frag f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float xh = CLAMP ? __builtin_amdgcn_fmed3f(x[e], -kBig, kBig) : x[e];
+    f.h[e] = (__bf16)xh;
+    const float r1 = x[e] - (float)f.h[e];
+    const float xm = CLAMP ? __builtin_amdgcn_fmed3f(r1, -kBig, kBig) : r1;
+    f.m[e] = (__bf16)xm;
+    f.l[e] = (__bf16)(r1 - (float)f.m[e]);
+  }
+  return f;
+}
+
+// Tile layout, fragment access and product of a kernel over elements T at padded head dim DP. X3: float32 with
+// the split products; its LDS tiles hold each row as three bfloat16 planes of DP columns (h | m | l), split once
+// when the tile is staged, so that fragments are read as a 16-bit tile's are (ds_read_b128, ds_read_b64_tr_b16).
+template <typename T, int DP, bool X3>
+struct Ops {
+  using MM = Mfma<T>;
+  using F = typename MM::frag_t;
+  static constexpr int KC = MM::KC;
+  static constexpr int PITCH = DP + 16 / (int)sizeof(T);  // elements T between rows
+  __device__ __forceinline__ static F cols(const T* tile, int row, int c) {
+    return lds_cols<T, KLIN>(tile, PITCH, row, 0, c);
+  }
+  __device__ __forceinline__ static F rows(const T* tile, int kbase, int c, int col0) {
+    return lds_rows<T, KACC>(tile, PITCH, kbase, c, col0);
+  }
+  __device__ __forceinline__ static F gload(const T* base, int64_t rs, int row, int nrows, int c, int D, bool vec) {
+    return gload_frag<T>(base, rs, row, nrows, c, D, vec);
+  }
+  __device__ __forceinline__ static F acc(const f32x16_t& a, int c) { return acc_frag<T>(a, c); }
+  template <bool SW = false>
+  __device__ __forceinline__ static f32x16_t mma(const F& a, const F& b, f32x16_t c) {
+    return MM::mma(a, b, c);
+  }
+  template <int ROWS, int NT>
+  __device__ __forceinline__ static void store(const TileStage<T, ROWS, DP, NT>& st, T* lds) {
+    st.store(lds, PITCH);
+  }
+};
+
+template <int DP>
+struct Ops<float, DP, true> {
+  using MM = MfmaX3;
+  using F = X3Frag;
+  static constexpr int KC = MM::KC;
+  // 3 DP bfloat16 and padding to 52, 100 or 228 words: 16 consecutive rows start in 16 distinct groups of 4 banks
+  static constexpr int PITCH = DP == 128 ? 228 : 3 * DP / 2 + 4;
+  __device__ __forceinline__ static F cols(const float* tile, int row, int c) {
+    const int g = (threadIdx.x >> 5) & 1;
+    const char* p = reinterpret_cast<const char*>(tile + row * PITCH) + (16 * c + 8 * g) * 2;
+    F f;
+    f.h = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const i16x8_t*>(p));
+    f.m = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const i16x8_t*>(p + 2 * DP));
+    f.l = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const i16x8_t*>(p + 4 * DP));
+    return f;
+  }
+  __device__ __forceinline__ static F rows(const float* tile, int kbase, int c, int col0) {
+    F f;
+    const short* t = reinterpret_cast<const short*>(tile);
+    f.h = __builtin_bit_cast(bf16x8_t, lds_rows<__bf16, KACC>((const __bf16*)t, 2 * PITCH, kbase, c, col0));
+    f.m = __builtin_bit_cast(bf16x8_t, lds_rows<__bf16, KACC>((const __bf16*)t + DP, 2 * PITCH, kbase, c, col0));
+    f.l = __builtin_bit_cast(bf16x8_t, lds_rows<__bf16, KACC>((const __bf16*)t + 2 * DP, 2 * PITCH, kbase, c, col0));
+    return f;
+  }
+  __device__ __forceinline__ static F gload(const float* base, int64_t rs, int row, int nrows, int c, int D, bool vec) {
+    const int col = 16 * c + 8 * ((threadIdx.x >> 5) & 1);
+    float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (row < nrows) {
+      const float* p = base + (int64_t)row * rs + col;
+      if (vec && col + 8 <= D) {
+        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(p), b = *reinterpret_cast<const f32x4_t*>(p + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[e] = a[e];
+          x[4 + e] = b[e];
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (col + e < D) x[e] = p[e];
+      }
+    }
+    return split3<true>(x);
+  }
+  __device__ __forceinline__ static F acc(const f32x16_t& a, int c) {
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = a[8 * c + e];
+    return split3<false>(x);
+  }
+  template <bool SW = false>
+  __device__ __forceinline__ static f32x16_t mma(const F& a, const F& b, f32x16_t c) {
+    return MM::template mma<SW>(a, b, c);
+  }
+  template <int ROWS, int NT>
+  __device__ __forceinline__ static void store(const TileStage<float, ROWS, DP, NT>& st, float* lds) {
+    using S = TileStage<float, ROWS, DP, NT>;
+    constexpr float kBig = 3.3895313892515355e38f;
+#pragma unroll
+    for (int i = 0; i < S::PER; ++i) {
+      const int ch = (int)threadIdx.x + i * NT;
+      if (S::NCH % NT == 0 || ch < S::NCH) {
+        const int row = ch / S::CPR, col = (ch % S::CPR) * S::VEC;
+        const f32x4_t x = __builtin_bit_cast(f32x4_t, st.r[i]);
+        bf16x4_t h, m, l;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {  // as split3<true>
+          h[e] = (__bf16)__builtin_amdgcn_fmed3f(x[e], -kBig, kBig);
+          const float r1 = x[e] - (float)h[e];
+          m[e] = (__bf16)__builtin_amdgcn_fmed3f(r1, -kBig, kBig);
+          l[e] = (__bf16)(r1 - (float)m[e]);
+        }
+        char* p = reinterpret_cast<char*>(lds + row * PITCH) + 2 * col;
+        *reinterpret_cast<i16x4_t*>(p) = __builtin_bit_cast(i16x4_t, h);
+        *reinterpret_cast<i16x4_t*>(p + 2 * DP) = __builtin_bit_cast(i16x4_t, m);
+        *reinterpret_cast<i16x4_t*>(p + 4 * DP) = __builtin_bit_cast(i16x4_t, l);
+      }
+    }
+  }
+};
 
 }  // namespace theria

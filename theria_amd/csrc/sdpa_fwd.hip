@@ -25,11 +25,11 @@ namespace theria {
 
 template <typename T, int DP, bool CAUSAL, int QT, int BN>
 __global__ __launch_bounds__(256, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel(const FwdParams p) {
-  using MM = Mfma<T>;
-  using F = typename MM::frag_t;
-  constexpr int KC = MM::KC;
+  using OP = Ops<T, DP, sizeof(T) == 4>;
+  using F = typename OP::F;
+  constexpr int KC = OP::KC;
   constexpr int NW = 4, BM = 32 * NW * QT, NT = 64 * NW;
-  constexpr int PITCH = DP + 16 / (int)sizeof(T);
+  constexpr int PITCH = OP::PITCH;
   constexpr int NDT = DP / 32, NKC = DP / KC, NPC = 32 / KC, NST = BN / 32;
   __shared__ __attribute__((aligned(16))) T sK[BN * PITCH];
   __shared__ __attribute__((aligned(16))) T sV[BN * PITCH];
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(256, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel(con
   for (int j = 0; j < QT; ++j) {
     const int myq = q0w + 32 * j + li;
 #pragma unroll
-    for (int c = 0; c < NKC; ++c) qf[j][c] = gload_frag<T>(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
+    for (int c = 0; c < NKC; ++c) qf[j][c] = OP::gload(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) o[j][dt] = zero16();
     m_use[j] = -THERIA_INF;  // offset of P in the log2 domain
@@ -75,8 +75,8 @@ __global__ __launch_bounds__(256, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel(con
   for (int kt = 0; kt < nkt; ++kt) {
     const int k0 = kt * BN;
     __syncthreads();
-    stK.store(sK, PITCH);
-    stV.store(sV, PITCH);
+    OP::store(stK, sK);
+    OP::store(stV, sV);
     __syncthreads();
     if (kt + 1 < nkt) {
       stK.load_any(K, p.k.sr, k0 + BN, s.M, s.D, s.vec);
@@ -91,9 +91,9 @@ __global__ __launch_bounds__(256, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel(con
       for (int j = 0; j < QT; ++j) sc[j][t] = zero16();
 #pragma unroll
       for (int c = 0; c < NKC; ++c) {
-        const F kfr = lds_cols<T, KLIN>(sK, PITCH, t * 32 + li, 0, c);
+        const F kfr = OP::cols(sK, t * 32 + li, c);
 #pragma unroll
-        for (int j = 0; j < QT; ++j) sc[j][t] = MM::mma(kfr, qf[j][c], sc[j][t]);
+        for (int j = 0; j < QT; ++j) sc[j][t] = OP::mma(kfr, qf[j][c], sc[j][t]);
       }
     }
     // Boundary tiles only (a uniform branch): masked scores become -inf, so P = 0 there. Interior
@@ -149,12 +149,12 @@ __global__ __launch_bounds__(256, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel(con
       for (int cc = 0; cc < NPC; ++cc) {
         F pf[QT];
 #pragma unroll
-        for (int j = 0; j < QT; ++j) pf[j] = acc_frag<T>(sc[j][t], cc);
+        for (int j = 0; j < QT; ++j) pf[j] = OP::acc(sc[j][t], cc);
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) {
-          const F vfr = lds_rows<T, KACC>(sV, PITCH, t * 32, cc, dt * 32);
+          const F vfr = OP::rows(sV, t * 32, cc, dt * 32);
 #pragma unroll
-          for (int j = 0; j < QT; ++j) o[j][dt] = MM::mma(vfr, pf[j], o[j][dt]);
+          for (int j = 0; j < QT; ++j) o[j][dt] = OP::mma(vfr, pf[j], o[j][dt]);
         }
       }
   }

@@ -38,12 +38,12 @@ namespace theria {
 // tile with the next tile's copies in flight; otherwise they pass through registers into padded LDS rows.
 template <typename T, int DP, bool CAUSAL, bool HAS_O, bool DMA>
 __global__ __launch_bounds__(256) void jvp_kernel(const JvpParams p) {
-  using MM = Mfma<T>;
-  using F = typename MM::frag_t;
-  constexpr int KC = MM::KC;
+  using OP = Ops<T, DP, (sizeof(T) == 4 && DP <= 64)>;
+  using F = typename OP::F;
+  constexpr int KC = OP::KC;
   constexpr int NW = 4, BM = 32 * NW, NT = 64 * NW;
   constexpr int BN = (DP == 128 || sizeof(T) == 4) ? 32 : 64;  // keys per tile (register budget)
-  constexpr int PITCH = DP + 16 / (int)sizeof(T);
+  constexpr int PITCH = OP::PITCH;
   constexpr int NDT = DP / 32, NKC = DP / KC, NPC = 32 / KC, NST = BN / 32;
   constexpr int TB = DMA ? BN * DP * 2 : BN * PITCH * (int)sizeof(T);  // bytes per tile
   constexpr int TB2 = DMA ? TB : 16;                                    // second set (DMA only)
@@ -79,8 +79,8 @@ __global__ __launch_bounds__(256) void jvp_kernel(const JvpParams p) {
   F qf[NKC], tqf[NKC];
 #pragma unroll
   for (int c = 0; c < NKC; ++c) {
-    qf[c] = gload_frag<T>(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
-    tqf[c] = has_tq ? gload_frag<T>(TQ, p.tq.sr, myq, s.T, c, s.D, s.vec) : F{};
+    qf[c] = OP::gload(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
+    tqf[c] = has_tq ? OP::gload(TQ, p.tq.sr, myq, s.T, c, s.D, s.vec) : F{};
   }
   f32x16_t accA[NDT], accC[NDT], accO[NDT];
 #pragma unroll
@@ -103,13 +103,13 @@ __global__ __launch_bounds__(256) void jvp_kernel(const JvpParams p) {
     if constexpr (DMA)
       return swz_cols<T, DP>(t, row, c);
     else
-      return lds_cols<T, KLIN>((const T*)t, PITCH, row, 0, c);
+      return OP::cols((const T*)t, row, c);
   };
   auto rowsf = [&](const char* t, int kbase, int c, int col0) -> F {
     if constexpr (DMA)
       return swz_rows<T, DP>(t, kbase, c, col0);
     else
-      return lds_rows<T, KACC>((const T*)t, PITCH, kbase, c, col0);
+      return OP::rows((const T*)t, kbase, c, col0);
   };
 
   // The key tile kt held in (tK, tV, ttK, ttV).
@@ -125,9 +125,9 @@ __global__ __launch_bounds__(256) void jvp_kernel(const JvpParams p) {
 #pragma unroll
       for (int c = 0; c < NKC; ++c) {
         const F kfr = colsf(tK, t * 32 + li, c);
-        sc[t] = MM::mma(kfr, qf[c], sc[t]);
-        if (has_tq) gm[t] = MM::mma(kfr, tqf[c], gm[t]);
-        if (has_tk) gm[t] = MM::mma(colsf(ttK, t * 32 + li, c), qf[c], gm[t]);
+        sc[t] = OP::mma(kfr, qf[c], sc[t]);
+        if (has_tq) gm[t] = OP::mma(kfr, tqf[c], gm[t]);
+        if (has_tk) gm[t] = OP::mma(colsf(ttK, t * 32 + li, c), qf[c], gm[t]);
       }
     }
     const bool need_mask = (k0 + BN > s.M) || (CAUSAL && k0 + BN - 1 > q0w);
@@ -155,17 +155,17 @@ __global__ __launch_bounds__(256) void jvp_kernel(const JvpParams p) {
           split_frag<T>(sc[t], cc, pf, pf_lo);
           split_frag<T>(gm[t], cc, pgf, pgf_lo);
         } else {
-          pf = acc_frag<T>(sc[t], cc);
-          pgf = acc_frag<T>(gm[t], cc);
+          pf = OP::acc(sc[t], cc);
+          pgf = OP::acc(gm[t], cc);
         }
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) {
           const F vfr = rowsf(tV, t * 32, cc, dt * 32);
-          accA[dt] = MM::mma(vfr, pgf, accA[dt]);
-          if (SPLIT) accA[dt] = MM::mma(vfr, pgf_lo, accA[dt]);
-          if (REBUILD) accO[dt] = MM::mma(vfr, pf, accO[dt]);
-          if (REBUILD && SPLIT) accO[dt] = MM::mma(vfr, pf_lo, accO[dt]);
-          if (has_tv) accC[dt] = MM::mma(rowsf(ttV, t * 32, cc, dt * 32), pf, accC[dt]);
+          accA[dt] = OP::mma(vfr, pgf, accA[dt]);
+          if (SPLIT) accA[dt] = OP::mma(vfr, pgf_lo, accA[dt]);
+          if (REBUILD) accO[dt] = OP::mma(vfr, pf, accO[dt]);
+          if (REBUILD && SPLIT) accO[dt] = OP::mma(vfr, pf_lo, accO[dt]);
+          if (has_tv) accC[dt] = OP::mma(rowsf(ttV, t * 32, cc, dt * 32), pf, accC[dt]);
         }
       }
   };
@@ -220,10 +220,10 @@ __global__ __launch_bounds__(256) void jvp_kernel(const JvpParams p) {
     if (nkt > 0) prefetch(0);
     for (int kt = 0; kt < nkt; ++kt) {
       __syncthreads();
-      gK.store((T*)sK0, PITCH);
-      gV.store((T*)sV0, PITCH);
-      if (has_tk) gtK.store((T*)stK0, PITCH);
-      if (has_tv) gtV.store((T*)stV0, PITCH);
+      OP::store(gK, (T*)sK0);
+      OP::store(gV, (T*)sV0);
+      if (has_tk) OP::store(gtK, (T*)stK0);
+      if (has_tv) OP::store(gtV, (T*)stV0);
       __syncthreads();
       if (kt + 1 < nkt) prefetch((kt + 1) * BN);
       compute(kt, sK0, sV0, stK0, stV0);

@@ -44,11 +44,11 @@ constexpr bool scores_wide() {
 
 template <typename T, int DP, int MODE>
 __global__ __launch_bounds__(256, (scores_wide<T, DP>() || DP > 64) ? 2 : 4) void scores_kernel(const ScoresParams p) {
-  using MM = Mfma<T>;
-  using F = typename MM::frag_t;
-  constexpr int NKC = DP / MM::KC;
+  using Tile = Ops<T, DP, sizeof(T) == 4>;
+  using F = typename Tile::F;
+  constexpr int NKC = DP / Tile::KC;
   constexpr int NW = 4, NT = 64 * NW, BN = 64, NU = BN / 32;
-  constexpr int PITCH = DP + 16 / (int)sizeof(T);  // K tile rows (padded)
+  constexpr int PITCH = Tile::PITCH;  // K tile rows (padded)
   constexpr int SW = scores_wide<T, DP>() ? 4 : 1;  // 32-key subtiles staged per store round
   constexpr int OP = 32 * SW + 4;                   // output staging rows, in floats (padded against bank conflicts)
   __shared__ __attribute__((aligned(16))) T sK[BN * PITCH];
@@ -68,14 +68,14 @@ __global__ __launch_bounds__(256, (scores_wide<T, DP>() || DP > 64) ? 2 : 4) voi
 
   F qf[NKC];
 #pragma unroll
-  for (int c = 0; c < NKC; ++c) qf[c] = gload_frag<T>(Q, p.q.sr, q0w + li, s.T, c, s.D, s.vec);
+  for (int c = 0; c < NKC; ++c) qf[c] = Tile::gload(Q, p.q.sr, q0w + li, s.T, c, s.D, s.vec);
 
   const int nkt = (s.M + BN - 1) / BN;
   TileStage<T, BN, DP, NT> stK;
   // Stages key tile kt (two barriers) and prefetches the next one.
   auto stage = [&](int kt) {
     __syncthreads();  // every wave is done with the previous tile
-    stK.store(sK, PITCH);
+    Tile::store(stK, sK);
     __syncthreads();
     if (kt + 1 < nkt) stK.load_any(K, p.k.sr, (kt + 1) * BN, s.M, s.D, s.vec);
   };
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256, (scores_wide<T, DP>() || DP > 64) ? 2 : 4) voi
   auto sub_scores = [&](int kt, int u) {
     f32x16_t st = zero16();
 #pragma unroll
-    for (int c = 0; c < NKC; ++c) st = MM::mma(lds_cols<T, KLIN>(sK, PITCH, 32 * u + li, 0, c), qf[c], st);
+    for (int c = 0; c < NKC; ++c) st = Tile::mma(Tile::cols(sK, 32 * u + li, c), qf[c], st);
     if (kt * BN + 32 * u + 32 > s.M) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)
