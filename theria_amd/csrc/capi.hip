@@ -300,6 +300,22 @@ THERIA_API int theria_sdpa_bwd(const theria_sdpa_problem_t* p, const theria_tens
   if (!c.err.empty()) return fail(THERIA_ERR_CONTRACT, c.err);
   s.vec = c.vec;
   const hipStream_t st = (hipStream_t)stream;
+  if (c.q_rows && c.k_rows && theria::small_problem(s)) {
+    theria::SmallBwdParams sp{};
+    sp.s = s;
+    sp.q = cv(q);
+    sp.k = cv(k);
+    sp.v = cv(v);
+    sp.dout = cv(dout);
+    sp.o = cv(o);
+    sp.o_f32 = o_is_f32 != 0;
+    sp.lse = lse;
+    sp.delta = delta_out;
+    sp.dq = mv(dq);
+    sp.dk = mv(dk);
+    sp.dv = mv(dv);
+    return hip_status(theria::launch_small_bwd(sp, st), "theria_sdpa_bwd (small)");
+  }
   if (c.q_rows) {
     int rc = run_dq(s, q, k, v, o, o_is_f32 != 0, theria::kRowFromO, dout, lse, delta_out, dq, st,
                     "theria_sdpa_bwd (dq)");
@@ -434,6 +450,13 @@ static int run_bwd_bwd(const theria_sdpa_problem_t* p, const theria_tensor_t* q,
   bp.row_l2 = nullptr;
   bp.r_row = row_ws;
   bp.t_row = row_ws + nrows;
+  if (theria::small_problem(s)) {  // one launch, from the rows' own statistics
+    bp.out_gq = mv(out_gq);
+    bp.out_gk = mv(out_gk);
+    bp.out_gv = mv(out_gv);
+    bp.out_gdo = mv(out_gdout);
+    return hip_status(theria::launch_small_bwdbwd(bp, st), "theria_sdpa_bwd_bwd (small)");
+  }
   if (s.dtype == THERIA_DTYPE_F32 && s.T > 0) {
     // float32: a pass over the keys forms each row's own statistics from its float32 scores, m2 = max_j fl(S c),
     // L2 = log2 sum_j exp2(fl(S c) - m2) (c = scale log2 e), and the row term z = sum_j P dP / sum_j P with dP

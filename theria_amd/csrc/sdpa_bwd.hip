@@ -77,12 +77,18 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
   for (int j = 0; j < QT; ++j) {
     const int myq = q0w + 32 * j + li;
     const bool qvalid = myq < s.T;
+    typename OP::Raw qraw[NKC], oraw[NKC];
 #pragma unroll
     for (int c = 0; c < NKC; ++c) {
-      qf[j][c] = OP::gload(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
-      of[j][c] = OP::gload(dO, p.dout.sr, myq, s.T, c, s.D, s.vec);
+      qraw[c] = OP::raw(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
+      oraw[c] = OP::raw(dO, p.dout.sr, myq, s.T, c, s.D, s.vec);
     }
     const float lse = qvalid ? p.lse[rowbase + myq] : THERIA_INF;
+#pragma unroll
+    for (int c = 0; c < NKC; ++c) {
+      qf[j][c] = OP::frag(qraw[c]);
+      of[j][c] = OP::frag(oraw[c]);
+    }
     lse2[j] = lse == -THERIA_INF ? THERIA_INF : lse * kLog2e;  // a row without visible keys has P = 0
     peaked |= qvalid && lse_peaked(lse);
     del[j] = 0.f;
@@ -366,18 +372,22 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(c
 
   F kf[KT][NKC], vf[KT][NKC];
 #pragma unroll
-  for (int t = 0; t < KT; ++t)
+  for (int t = 0; t < KT; ++t) {
+    typename OP::Raw kraw[NKC], vraw[NKC];
+    const T* V = DV_ONLY ? nullptr : (const T*)p.v.p + b * p.v.sb + h * p.v.sh;
 #pragma unroll
     for (int c = 0; c < NKC; ++c) {
-      kf[t][c] = OP::gload(K, p.k.sr, kw0 + 32 * t + li, s.M, c, s.D, s.vec);
-      vf[t][c] = F{};
+      kraw[c] = OP::raw(K, p.k.sr, kw0 + 32 * t + li, s.M, c, s.D, s.vec);
+      if constexpr (!DV_ONLY) vraw[c] = OP::raw(V, p.v.sr, kw0 + 32 * t + li, s.M, c, s.D, s.vec);
     }
-  if constexpr (!DV_ONLY) {
-    const T* V = (const T*)p.v.p + b * p.v.sb + h * p.v.sh;
 #pragma unroll
-    for (int t = 0; t < KT; ++t)
-#pragma unroll
-      for (int c = 0; c < NKC; ++c) vf[t][c] = OP::gload(V, p.v.sr, kw0 + 32 * t + li, s.M, c, s.D, s.vec);
+    for (int c = 0; c < NKC; ++c) {
+      kf[t][c] = OP::frag(kraw[c]);
+      if constexpr (!DV_ONLY)
+        vf[t][c] = OP::frag(vraw[c]);
+      else
+        vf[t][c] = F{};
+    }
   }
   f32x16_t dv[KT][NDT], dk[KT][NDT];
 #pragma unroll

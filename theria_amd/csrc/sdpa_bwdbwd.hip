@@ -106,11 +106,20 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
   if (EXACT && !exact) return;
 
   F qf[NKC], dof[NKC], gqf[NKC];
+  {
+    typename OP::Raw r0[NKC], r1[NKC], r2[NKC];
 #pragma unroll
-  for (int c = 0; c < NKC; ++c) {
-    qf[c] = OP::gload(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
-    dof[c] = OP::gload(dO, p.dout.sr, myq, s.T, c, s.D, s.vec);
-    gqf[c] = has_gq ? OP::gload(GQ, p.gq.sr, myq, s.T, c, s.D, s.vec) : F{};
+    for (int c = 0; c < NKC; ++c) {
+      r0[c] = OP::raw(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
+      r1[c] = OP::raw(dO, p.dout.sr, myq, s.T, c, s.D, s.vec);
+      r2[c] = has_gq ? OP::raw(GQ, p.gq.sr, myq, s.T, c, s.D, s.vec) : typename OP::Raw{};
+    }
+#pragma unroll
+    for (int c = 0; c < NKC; ++c) {
+      qf[c] = OP::frag(r0[c]);
+      dof[c] = OP::frag(r1[c]);
+      gqf[c] = OP::frag(r2[c]);
+    }
   }
   f32x16_t x13[NDT], x2[NDT], x4[NDT], yk[NDT];
 #pragma unroll
@@ -460,12 +469,22 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
   const bool kvalid = mykey < s.M;
 
   F kf[NKC], vf[NKC], gkf[NKC], gvf[NKC];
+  {
+    typename OP::Raw r0[NKC], r1[NKC], r2[NKC], r3[NKC];
 #pragma unroll
-  for (int c = 0; c < NKC; ++c) {
-    kf[c] = OP::gload(K, p.k.sr, mykey, s.M, c, s.D, s.vec);
-    vf[c] = OP::gload(V, p.v.sr, mykey, s.M, c, s.D, s.vec);
-    gkf[c] = has_gk ? OP::gload(GK, p.gk.sr, mykey, s.M, c, s.D, s.vec) : F{};
-    gvf[c] = has_gv ? OP::gload(GV, p.gv.sr, mykey, s.M, c, s.D, s.vec) : F{};
+    for (int c = 0; c < NKC; ++c) {
+      r0[c] = OP::raw(K, p.k.sr, mykey, s.M, c, s.D, s.vec);
+      r1[c] = OP::raw(V, p.v.sr, mykey, s.M, c, s.D, s.vec);
+      r2[c] = has_gk ? OP::raw(GK, p.gk.sr, mykey, s.M, c, s.D, s.vec) : typename OP::Raw{};
+      r3[c] = has_gv ? OP::raw(GV, p.gv.sr, mykey, s.M, c, s.D, s.vec) : typename OP::Raw{};
+    }
+#pragma unroll
+    for (int c = 0; c < NKC; ++c) {
+      kf[c] = OP::frag(r0[c]);
+      vf[c] = OP::frag(r1[c]);
+      gkf[c] = OP::frag(r2[c]);
+      gvf[c] = OP::frag(r3[c]);
+    }
   }
   f32x16_t accV[NDT], accK[NDT];
 #pragma unroll

@@ -476,9 +476,13 @@ struct Ops {
   __device__ __forceinline__ static F rows(const T* tile, int kbase, int c, int col0) {
     return lds_rows<T, KACC>(tile, PITCH, kbase, c, col0);
   }
-  __device__ __forceinline__ static F gload(const T* base, int64_t rs, int row, int nrows, int c, int D, bool vec) {
+  // A fragment from global memory in two steps, raw (the loads) and frag (what the registers need after them), so
+  // that a caller can have the loads of all its operands in flight before the first frag waits for one.
+  using Raw = F;
+  __device__ __forceinline__ static Raw raw(const T* base, int64_t rs, int row, int nrows, int c, int D, bool vec) {
     return gload_frag<T>(base, rs, row, nrows, c, D, vec);
   }
+  __device__ __forceinline__ static F frag(const Raw& r) { return r; }
   __device__ __forceinline__ static F acc(const f32x16_t& a, int c) { return acc_frag<T>(a, c); }
   template <bool SW = false>
   __device__ __forceinline__ static f32x16_t mma(const F& a, const F& b, f32x16_t c) {
@@ -514,24 +518,29 @@ struct Ops<float, DP, true> {
     f.l = __builtin_bit_cast(bf16x8_t, lds_rows<__bf16, KACC>((const __bf16*)t + 2 * DP, 2 * PITCH, kbase, c, col0));
     return f;
   }
-  __device__ __forceinline__ static F gload(const float* base, int64_t rs, int row, int nrows, int c, int D, bool vec) {
+  struct Raw {
+    f32x4_t a, b;
+  };
+  __device__ __forceinline__ static Raw raw(const float* base, int64_t rs, int row, int nrows, int c, int D, bool vec) {
     const int col = 16 * c + 8 * ((threadIdx.x >> 5) & 1);
-    float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    Raw r = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
     if (row < nrows) {
       const float* p = base + (int64_t)row * rs + col;
       if (vec && col + 8 <= D) {
-        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(p), b = *reinterpret_cast<const f32x4_t*>(p + 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          x[e] = a[e];
-          x[4 + e] = b[e];
-        }
+        r.a = *reinterpret_cast<const f32x4_t*>(p);
+        r.b = *reinterpret_cast<const f32x4_t*>(p + 4);
       } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (col + e < D) x[e] = p[e];
+        for (int e = 0; e < 4; ++e) {
+          if (col + e < D) r.a[e] = p[e];
+          if (col + 4 + e < D) r.b[e] = p[4 + e];
+        }
       }
     }
+    return r;
+  }
+  __device__ __forceinline__ static F frag(const Raw& r) {
+    const float x[8] = {r.a[0], r.a[1], r.a[2], r.a[3], r.b[0], r.b[1], r.b[2], r.b[3]};
     return split3<true>(x);
   }
   __device__ __forceinline__ static F acc(const f32x16_t& a, int c) {

@@ -54,8 +54,11 @@ __global__ __launch_bounds__(256, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel(con
 #pragma unroll
   for (int j = 0; j < QT; ++j) {
     const int myq = q0w + 32 * j + li;
+    typename OP::Raw qraw[NKC];
 #pragma unroll
-    for (int c = 0; c < NKC; ++c) qf[j][c] = OP::gload(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
+    for (int c = 0; c < NKC; ++c) qraw[c] = OP::raw(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
+#pragma unroll
+    for (int c = 0; c < NKC; ++c) qf[j][c] = OP::frag(qraw[c]);
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) o[j][dt] = zero16();
     m_use[j] = -THERIA_INF;  // offset of P in the log2 domain

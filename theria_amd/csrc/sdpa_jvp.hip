@@ -77,10 +77,18 @@ __global__ __launch_bounds__(256) void jvp_kernel(const JvpParams p) {
   const int64_t row_id = (int64_t)bh * s.T + myq;
 
   F qf[NKC], tqf[NKC];
+  {
+    typename OP::Raw qraw[NKC], tqraw[NKC];
 #pragma unroll
-  for (int c = 0; c < NKC; ++c) {
-    qf[c] = OP::gload(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
-    tqf[c] = has_tq ? OP::gload(TQ, p.tq.sr, myq, s.T, c, s.D, s.vec) : F{};
+    for (int c = 0; c < NKC; ++c) {
+      qraw[c] = OP::raw(Q, p.q.sr, myq, s.T, c, s.D, s.vec);
+      tqraw[c] = has_tq ? OP::raw(TQ, p.tq.sr, myq, s.T, c, s.D, s.vec) : typename OP::Raw{};
+    }
+#pragma unroll
+    for (int c = 0; c < NKC; ++c) {
+      qf[c] = OP::frag(qraw[c]);
+      tqf[c] = OP::frag(tqraw[c]);
+    }
   }
   f32x16_t accA[NDT], accC[NDT], accO[NDT];
 #pragma unroll

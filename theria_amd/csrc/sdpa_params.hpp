@@ -106,8 +106,20 @@ struct BwdBwdParams {
   const float* lse_fwd;
   float* z_out;
   float* lse_out;
-  MutView out_gdo;  // the key-split row kernel also writes G_dO (no separate JVP launch)
+  MutView out_gdo;  // the key-split row kernel and the small-problem kernel also write G_dO (no separate JVP launch)
 };
+
+// Whole backward of a small problem (sdpa_small.hip); dq and dk may be null.
+struct SmallBwdParams {
+  Shape s;
+  View q, k, v, dout, o;
+  bool o_f32;
+  const float* lse;
+  float* delta;
+  MutView dq, dk, dv;
+};
+// At most 64 queries and 64 keys, at a head dim the one-workgroup kernels hold.
+bool small_problem(const Shape& s);
 
 // The row kernel of this problem forms the row term and the exact normaliser itself (no row-term pass needed).
 bool bwdbwd_rows_make_row_terms(const BwdBwdParams& p);
@@ -131,6 +143,8 @@ hipError_t launch_bwd_dkdv(const DkdvParams& p, hipStream_t st);
 hipError_t launch_jvp(const JvpParams& p, hipStream_t st);
 hipError_t launch_bwdbwd_rows(const BwdBwdParams& p, hipStream_t st);
 hipError_t launch_bwdbwd_cols(const BwdBwdParams& p, hipStream_t st);
+hipError_t launch_small_bwd(const SmallBwdParams& p, hipStream_t st);
+hipError_t launch_small_bwdbwd(const BwdBwdParams& p, hipStream_t st);
 hipError_t launch_scores(const ScoresParams& p, hipStream_t st);
 
 #ifdef THERIA_TILE_COUNT

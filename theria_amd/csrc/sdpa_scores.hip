@@ -67,8 +67,11 @@ __global__ __launch_bounds__(256, (scores_wide<T, DP>() || DP > 64) ? 2 : 4) voi
   const float c2 = s.scale * kLog2e;
 
   F qf[NKC];
+  typename Tile::Raw qraw[NKC];
 #pragma unroll
-  for (int c = 0; c < NKC; ++c) qf[c] = Tile::gload(Q, p.q.sr, q0w + li, s.T, c, s.D, s.vec);
+  for (int c = 0; c < NKC; ++c) qraw[c] = Tile::raw(Q, p.q.sr, q0w + li, s.T, c, s.D, s.vec);
+#pragma unroll
+  for (int c = 0; c < NKC; ++c) qf[c] = Tile::frag(qraw[c]);
 
   const int nkt = (s.M + BN - 1) / BN;
   TileStage<T, BN, DP, NT> stK;
