@@ -23,12 +23,14 @@
 
 namespace theria {
 
-template <typename T, int DP, bool CAUSAL, int QT, int BN>
-__global__ __launch_bounds__(256, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel(const FwdParams p) {
+// NW waves per workgroup: four, or two for at most 64 queries (QT = 1), where two of four would have no rows (us, four
+// -> two waves: float32 B400 H4 T64 D16 18.6 -> 17.3, B128 H8 T32 D32 12.6 -> 9.5, bfloat16 B64 H8 T64 D128 13.2 -> 9.4).
+template <typename T, int DP, bool CAUSAL, int QT, int BN, int NW = 4>
+__global__ __launch_bounds__(64 * NW, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel(const FwdParams p) {
   using OP = Ops<T, DP, sizeof(T) == 4>;
   using F = typename OP::F;
   constexpr int KC = OP::KC;
-  constexpr int NW = 4, BM = 32 * NW * QT, NT = 64 * NW;
+  constexpr int BM = 32 * NW * QT, NT = 64 * NW;
   constexpr int PITCH = OP::PITCH;
   constexpr int NDT = DP / 32, NKC = DP / KC, NPC = 32 / KC, NST = BN / 32;
   __shared__ __attribute__((aligned(16))) T sK[BN * PITCH];
@@ -224,6 +226,13 @@ struct FwdLauncher {
     }
     // Two query tiles per wave only for 16-bit inputs: with float32 fragments (twice the registers)
     // that variant spills ~150 VGPRs and runs at half the one-tile rate.
+    // Two-wave workgroups where four-wave ones (two of whose waves have no rows) would not all be resident at once;
+    // below that the wider workgroup stages its tiles sooner (float32 D64 B24 H16 T52: 12.0 against 14.5 us).
+    const int64_t nbh = (int64_t)p.s.B * p.s.H;
+    if (p.s.T >= 1 && p.s.T <= 64 && nbh > (int64_t)device_cu_count() * (DP <= 64 ? 2 : 1)) {
+      hipLaunchKernelGGL((fwd_kernel<T, DP, CAUSAL, 1, 64, 2>), dim3((unsigned)nbh), dim3(128), 0, st, p);
+      return hipGetLastError();
+    }
     const int qt = sizeof(T) == 2 ? fwd_qt<DP>(p.s.T) : 1;
     const int bm = 128 * qt;
     const int64_t nblk = (int64_t)((p.s.T + bm - 1) / bm) * p.s.B * p.s.H;

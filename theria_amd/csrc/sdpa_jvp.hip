@@ -36,12 +36,13 @@ namespace theria {
 // DMA: 16-bit inputs with head dim exactly 64 or 128 and 16-byte-aligned rows. The K, tK, V, tV tiles are
 // then filled by LDS DMA into two sets of unpadded, XOR-swizzled buffers (sdpa_lds.hpp), one barrier per
 // tile with the next tile's copies in flight; otherwise they pass through registers into padded LDS rows.
-template <typename T, int DP, bool CAUSAL, bool HAS_O, bool DMA>
-__global__ __launch_bounds__(256) void jvp_kernel(const JvpParams p) {
+// NW: waves per workgroup, four or (without DMA) two for at most 64 queries.
+template <typename T, int DP, bool CAUSAL, bool HAS_O, bool DMA, int NW = 4>
+__global__ __launch_bounds__(64 * NW) void jvp_kernel(const JvpParams p) {
   using OP = Ops<T, DP, (sizeof(T) == 4 && DP <= 64)>;
   using F = typename OP::F;
   constexpr int KC = OP::KC;
-  constexpr int NW = 4, BM = 32 * NW, NT = 64 * NW;
+  constexpr int BM = 32 * NW, NT = 64 * NW;
   constexpr int BN = (DP == 128 || sizeof(T) == 4) ? 32 : 64;  // keys per tile (register budget)
   constexpr int PITCH = OP::PITCH;
   constexpr int NDT = DP / 32, NKC = DP / KC, NPC = 32 / KC, NST = BN / 32;
@@ -555,6 +556,12 @@ struct JvpLauncher {
           hipLaunchKernelGGL((jvp_kernel<T, DP, CAUSAL, HAS_O, true>), dim3((unsigned)nblk), dim3(256), 0, st, p);
         return hipGetLastError();
       }
+    }
+    // at most 64 queries, and more workgroups than CUs (one four-wave workgroup per CU is resident): float32 B400 H4
+    // T64 D16 42 -> 34 us
+    if (p.s.T <= 64 && nblk > device_cu_count()) {
+      hipLaunchKernelGGL((jvp_kernel<T, DP, CAUSAL, HAS_O, false, 2>), dim3((unsigned)nblk), dim3(128), 0, st, p);
+      return hipGetLastError();
     }
     hipLaunchKernelGGL((jvp_kernel<T, DP, CAUSAL, HAS_O, false>), dim3((unsigned)nblk), dim3(256), 0, st, p);
     return hipGetLastError();
