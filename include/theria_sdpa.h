@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define THERIA_SDPA_ABI_VERSION 9
+#define THERIA_SDPA_ABI_VERSION 10
 
 enum theria_dtype { THERIA_DTYPE_F32 = 0, THERIA_DTYPE_F16 = 1, THERIA_DTYPE_BF16 = 2 };
 enum theria_status { THERIA_OK = 0, THERIA_ERR_CONTRACT = 1, THERIA_ERR_HIP = 2 };
@@ -71,6 +71,17 @@ int theria_sdpa_fwd(const theria_sdpa_problem_t* p, const theria_tensor_t* q, co
                     float* row_max, float* row_sum, void* stream);
 
 /*
+ * theria_sdpa_fwd with a workspace: ws_floats float32 of 16-byte-aligned device memory, used until the call's work on
+ * the stream is done. Problems with few query blocks against many keys split the keys over workgroups when ws holds at
+ * least theria_sdpa_fwd_ws_floats(p) floats (0 for every other problem: then, and with ws NULL or smaller, the call is
+ * theria_sdpa_fwd). Same results up to the order in which a row's keys are summed.
+ */
+int theria_sdpa_fwd_ws(const theria_sdpa_problem_t* p, const theria_tensor_t* q, const theria_tensor_t* k,
+                       const theria_tensor_t* v, const theria_tensor_t* o, int32_t o_is_f32, float* lse,
+                       float* row_max, float* row_sum, float* ws, int64_t ws_floats, void* stream);
+int64_t theria_sdpa_fwd_ws_floats(const theria_sdpa_problem_t* p);
+
+/*
  * Explicit backward given the forward output O: dQ, dK, dV.
  * Replaces sdpa_bwd_dq / sdpa_bwd_dk / sdpa_bwd_dv and their kernels
  * (theria/attention/triton_sdpa_backward.py:106-266, 269-462, 505-696) and the backward of
@@ -81,7 +92,8 @@ int theria_sdpa_fwd(const theria_sdpa_problem_t* p, const theria_tensor_t* q, co
  * (on a row whose probability sits on one key, dP - z is then a difference of consistently rounded values;
  * dO . O with the forward's O leaves ~2e-5 in dQ there). dout has the input dtype; o may be float32 (o_is_f32).
  * dq / dk may have data == NULL to skip that output. Deterministic (no atomics, no workspace).
- * theria_sdpa_bwd = theria_sdpa_bwd_dq followed by theria_sdpa_bwd_dkdv on the same stream.
+ * theria_sdpa_bwd = theria_sdpa_bwd_dq followed by theria_sdpa_bwd_dkdv on the same stream, or one launch with the same
+ * results up to rounding (at most 64 queries and 64 keys).
  *
  * 16-bit inputs: the probabilities P and the score gradients dS enter the MFMA products as 16-bit
  * operands. On the rows lse flags as peaked (theria_sdpa_fwd), each is taken as two 16-bit terms (hi + lo,

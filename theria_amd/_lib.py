@@ -18,7 +18,7 @@ import torch  # noqa: F401  (must be imported first: it loads the HIP runtime th
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libtheria_sdpa.so"
 # The counter-enabled build of the same sources (theria_debug_tile_counts counts there), for measurements only.
 TILES_LIB_PATH = LIB_PATH.with_name("libtheria_sdpa_tiles.so")
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 DTYPE_F32, DTYPE_F16, DTYPE_BF16 = 0, 1, 2
 OK, ERR_CONTRACT, ERR_HIP = 0, 1, 2
@@ -61,6 +61,11 @@ SIGNATURES = {
     "theria_abi_version": ([], ctypes.c_int),
     "theria_last_error": ([], ctypes.c_char_p),
     "theria_sdpa_fwd": ([_PR, _TV, _TV, _TV, _TV, ctypes.c_int32, _P, _P, _P, _P], ctypes.c_int),
+    "theria_sdpa_fwd_ws": (
+        [_PR, _TV, _TV, _TV, _TV, ctypes.c_int32, _P, _P, _P, _P, ctypes.c_int64, _P],
+        ctypes.c_int,
+    ),
+    "theria_sdpa_fwd_ws_floats": ([_PR], ctypes.c_int64),
     "theria_sdpa_bwd": (
         [_PR, _TV, _TV, _TV, _TV, ctypes.c_int32, _TV, _P, _P, _TV, _TV, _TV, _P],
         ctypes.c_int,

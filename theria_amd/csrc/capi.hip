@@ -99,6 +99,12 @@ int hip_status(hipError_t e, const char* what) {
   return fail(THERIA_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// Workspace of a forward whose keys are split over workgroups (0: not split).
+int64_t fwd_ws_floats(const theria::Shape& s) {
+  const int n = theria::fwd_splits(s);
+  return n > 1 ? (int64_t)n * s.B * s.H * s.T * theria::fwd_split_row_floats(s.D) : 0;
+}
+
 bool empty_problem(const theria::Shape& s) { return s.B == 0 || s.H == 0 || s.T == 0; }
 
 }  // namespace
@@ -159,9 +165,9 @@ THERIA_API int theria_abi_version(void) { return THERIA_SDPA_ABI_VERSION; }
 
 THERIA_API const char* theria_last_error(void) { return g_last_error.c_str(); }
 
-THERIA_API int theria_sdpa_fwd(const theria_sdpa_problem_t* p, const theria_tensor_t* q, const theria_tensor_t* k,
-                               const theria_tensor_t* v, const theria_tensor_t* o, int32_t o_is_f32, float* lse,
-                               float* row_max, float* row_sum, void* stream) {
+static int run_fwd(const theria_sdpa_problem_t* p, const theria_tensor_t* q, const theria_tensor_t* k,
+                   const theria_tensor_t* v, const theria_tensor_t* o, int32_t o_is_f32, float* lse, float* row_max,
+                   float* row_sum, float* ws, int64_t ws_floats, void* stream) {
   theria::Shape s;
   std::string err;
   if (!shape_from(p, s, err)) return fail(THERIA_ERR_CONTRACT, err);
@@ -185,7 +191,29 @@ THERIA_API int theria_sdpa_fwd(const theria_sdpa_problem_t* p, const theria_tens
   fp.lse = lse;
   fp.row_max = row_max;
   fp.row_sum = row_sum;
+  fp.nsplit = ws && ws_floats > 0 && ws_floats >= fwd_ws_floats(s) ? theria::fwd_splits(s) : 1;
+  fp.ws = ws;
   return hip_status(theria::launch_fwd(fp, (hipStream_t)stream), "theria_sdpa_fwd");
+}
+
+THERIA_API int theria_sdpa_fwd(const theria_sdpa_problem_t* p, const theria_tensor_t* q, const theria_tensor_t* k,
+                               const theria_tensor_t* v, const theria_tensor_t* o, int32_t o_is_f32, float* lse,
+                               float* row_max, float* row_sum, void* stream) {
+  return run_fwd(p, q, k, v, o, o_is_f32, lse, row_max, row_sum, nullptr, 0, stream);
+}
+
+THERIA_API int theria_sdpa_fwd_ws(const theria_sdpa_problem_t* p, const theria_tensor_t* q, const theria_tensor_t* k,
+                                  const theria_tensor_t* v, const theria_tensor_t* o, int32_t o_is_f32, float* lse,
+                                  float* row_max, float* row_sum, float* ws, int64_t ws_floats, void* stream) {
+  if (ws && reinterpret_cast<uintptr_t>(ws) % 16 != 0)
+    return fail(THERIA_ERR_CONTRACT, "theria_sdpa_fwd_ws: ws must be 16-byte aligned");
+  return run_fwd(p, q, k, v, o, o_is_f32, lse, row_max, row_sum, ws, ws_floats, stream);
+}
+
+THERIA_API int64_t theria_sdpa_fwd_ws_floats(const theria_sdpa_problem_t* p) {
+  theria::Shape s;
+  std::string err;
+  return shape_from(p, s, err) ? fwd_ws_floats(s) : 0;
 }
 
 // The dQ kernel; row_term (theria::RowTerm) says how it obtains the row term it writes to (or reads from) delta.

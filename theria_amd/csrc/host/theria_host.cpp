@@ -131,8 +131,11 @@ py::tuple fwd(at::Tensor q, at::Tensor k, at::Tensor v, double scale, bool causa
   if (stats) m = at::empty_like(lse), l = at::empty_like(lse);
   const auto p = problem(q, k, scale, causal);
   const auto tq = view(q), tk = view(k), tv = view(v), to = view(o);
-  check_rc(theria_sdpa_fwd(&p, &tq, &tk, &tv, &to, out_fp32 ? 1 : 0, fptr(lse), fptr(m), fptr(l),
-                           stream_of(q)),
+  // workspace of a forward whose keys are split over workgroups, on the stream that uses it
+  const int64_t nws = theria_sdpa_fwd_ws_floats(&p);
+  const OptT ws = nws > 0 ? OptT(at::empty({nws}, f)) : std::nullopt;
+  check_rc(theria_sdpa_fwd_ws(&p, &tq, &tk, &tv, &to, out_fp32 ? 1 : 0, fptr(lse), fptr(m), fptr(l), fptr(ws), nws,
+                              stream_of(q)),
            "theria_sdpa_fwd");
   return py::make_tuple(o, lse, m ? py::cast(*m) : py::none(), l ? py::cast(*l) : py::none());
 }

@@ -25,6 +25,7 @@
 //    numerator and denominator use the same probabilities.
 #include <type_traits>
 
+#include "fwd_split.hpp"
 #include "sdpa_common.hpp"
 #include "sdpa_lds.hpp"
 #include "tile_count.hpp"
@@ -51,7 +52,8 @@ hipError_t tile_counts_fwd(unsigned long long* fwd, bool reset) {
 }
 #endif
 
-template <typename T, bool CAUSAL, bool STATS, int NW, int DP, int QT, bool FD>
+// SPLIT: one part of the keys per workgroup (FwdParams::nsplit), no causal mask.
+template <typename T, bool CAUSAL, bool STATS, int NW, int DP, int QT, bool FD, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p) {
   using MM = Mfma<T>;
   using F = typename MM::frag_t;
@@ -76,12 +78,15 @@ __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p)
   const bool pair = CAUSAL && !s.unpaired;
   const int nunit = pair ? (nqb + 1) / 2 : nqb;
   const int bid = xcd_remap(blockIdx.x, gridDim.x);
-  const int bh = bid / nunit;
-  const int unit = bid - bh * nunit;
+  const int bhp = bid / nunit;  // (batch, head) and, with SPLIT, the part of its keys
+  const int unit = bid - bhp * nunit;
+  const int bh = SPLIT ? bhp / p.nsplit : bhp, part = SPLIT ? bhp - bh * p.nsplit : 0;
   const int b = bh / s.H, h = bh - b * s.H;
   const T* Q = (const T*)p.q.p + b * p.q.sb + h * p.q.sh;
-  const T* K = (const T*)p.k.p + b * p.k.sb + h * p.k.sh;
-  const T* V = (const T*)p.v.p + b * p.v.sb + h * p.v.sh;
+  const FwdPart kp = fwd_part(s, SPLIT ? p.nsplit : 1, part);
+  const int M = SPLIT ? kp.keys : s.M;  // this workgroup's keys
+  const T* K = (const T*)p.k.p + b * p.k.sb + h * p.k.sh + (SPLIT ? kp.key0 * p.k.sr : 0);
+  const T* V = (const T*)p.v.p + b * p.v.sb + h * p.v.sh + (SPLIT ? kp.key0 * p.v.sr : 0);
   const int64_t rowbase = (int64_t)bh * s.T;
   const float c2 = s.scale * kLog2e;
   THERIA_TILES_DECL;
@@ -94,11 +99,11 @@ __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p)
   }
   const int q0w = qb * BM + wave * 32 * QT;  // query tile j of this wave starts at q0w + 32 j
 
-    int kend = s.M;
-    if (CAUSAL) kend = min(s.M, qb * BM + BM);
+    int kend = M;
+    if (CAUSAL) kend = min(M, qb * BM + BM);
     const int nkt = (kend + BN - 1) / BN;
     // Tiles [0, nfull) have every key in range and visible to every query of the block.
-    int nfull = s.M / BN;
+    int nfull = M / BN;
     if (CAUSAL) nfull = min(nfull, qb * BM / BN);
 
     using Dma = SwzDma<NW, DP>;
@@ -108,15 +113,15 @@ __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p)
     // Byte offsets fit in 32 bits: the host only selects this kernel when every (batch, head) slab of K
     // and V spans less than 2^31 bytes.
     const uint32_t krs = (uint32_t)p.k.sr * 2, vrs = (uint32_t)p.v.sr * 2;
-    const rsrc_t krsrc = make_rsrc(K, (uint32_t)slab_span(s.M, krs, 2 * Dh));
-    const rsrc_t vrsrc = make_rsrc(V, (uint32_t)slab_span(s.M, vrs, 2 * Dh));
+    const rsrc_t krsrc = make_rsrc(K, (uint32_t)slab_span(M, krs, 2 * Dh));
+    const rsrc_t vrsrc = make_rsrc(V, (uint32_t)slab_span(M, vrs, 2 * Dh));
     uint32_t koff[NSLAB], voff[NSLAB];
 #pragma unroll
     for (int i = 0; i < NSLAB; ++i) {
       koff[i] = dma.lane_offset(krs, i);
       voff[i] = dma.lane_offset(vrs, i);
     }
-    if (nkt > 0) dma.template issue_clamped<NSLAB>(krsrc, krs, 0, s.M, sK0);
+    if (nkt > 0) dma.template issue_clamped<NSLAB>(krsrc, krs, 0, M, sK0);
 
     F qf[QT][NKC];
 #pragma unroll
@@ -179,10 +184,10 @@ __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p)
     };
     // Keys out of range, or (causal) after the query, get -inf. Only boundary tiles pay for the test.
     auto mask = [&](f32x16_t (&sc)[QT][2], int k0) {
-      if ((k0 + BN > s.M) || (CAUSAL && k0 + BN - 1 > q0w)) {
+      if ((k0 + BN > M) || (CAUSAL && k0 + BN - 1 > q0w)) {
 #pragma unroll
         for (int j = 0; j < QT; ++j) {
-          const int lim = CAUSAL ? min(s.M, q0w + 32 * j + li + 1) : s.M;  // first key this query cannot see
+          const int lim = CAUSAL ? min(M, q0w + 32 * j + li + 1) : M;  // first key this query cannot see
 #pragma unroll
           for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -279,8 +284,8 @@ __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p)
         dma.template issue<NSLAB>(krsrc, koff, (uint32_t)(k0 + BN) * krs, kn);
         dma.template issue<NSLAB>(vrsrc, voff, (uint32_t)k0 * vrs, vn);
       } else {
-        if (k + 1 < nkt) dma.template issue_clamped<NSLAB>(krsrc, krs, k0 + BN, s.M, kn);
-        dma.template issue_clamped<NSLAB>(vrsrc, vrs, k0, s.M, vn);
+        if (k + 1 < nkt) dma.template issue_clamped<NSLAB>(krsrc, krs, k0 + BN, M, kn);
+        dma.template issue_clamped<NSLAB>(vrsrc, vrs, k0, M, vn);
       }
       F pn[QT][2][2];
       // QT query tiles x two 32-key subtiles, unless every key of the tile follows every query of the wave
@@ -407,7 +412,7 @@ __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p)
       // every buffer is a fixed array; then the boundary tiles.
       step(general, 0, sK0, sV1, sK1, sV0);
       // fast steps: k < nfull and K(k+1) in range
-      const int nfast = min(nfull, s.M / BN - 1);
+      const int nfast = min(nfull, M / BN - 1);
       int k = 1;
       for (; k + 1 < nfast; k += 2) {
         step(fast, k, sK1, sV0, sK0, sV1);      // k odd
@@ -433,8 +438,24 @@ __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p)
       const float l = pair_sum(l_part[j]);
       const float inv = l > 0.f ? 1.f / l : 0.f;
       // cross-lane, so taken by every lane before the per-row branches
-      const bool peaked = pair_max(pk_max[j]) > kPeakedFrac * l;
-      if (myq < s.T) {
+      const float pk_row = pair_max(pk_max[j]);
+      const bool peaked = pk_row > kPeakedFrac * l;
+      if constexpr (SPLIT) {
+        if (myq < s.T) {
+          const int RF = fwd_split_row_floats(s.D);
+          float* w = p.ws + ((int64_t)part * s.B * s.H * s.T + rowbase + myq) * RF;
+#pragma unroll
+          for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd) {
+              const int d0 = dt * 32 + 8 * qd + 4 * g;
+              if (d0 < Dh)
+                *reinterpret_cast<f32x4_t*>(w + d0) =
+                    f32x4_t{o[j][dt][4 * qd], o[j][dt][4 * qd + 1], o[j][dt][4 * qd + 2], o[j][dt][4 * qd + 3]};
+            }
+          if (g == 0) *reinterpret_cast<f32x4_t*>(w + RF - 4) = f32x4_t{m_use[j], l, m_max[j], pk_row};
+        }
+      } else if (myq < s.T) {
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
@@ -487,6 +508,16 @@ static void fwd_pipe_launch(const FwdParams& p0, hipStream_t st) {
   FwdParams p = p0;
   const int64_t bh = (int64_t)p.s.B * p.s.H;
   const int64_t cus = device_cu_count();
+  if constexpr (!CAUSAL) {
+    if (p.nsplit > 1) {  // (the statistics kernel: the parts' row maxima are combined whether or not m is wanted)
+      const dim3 grid((unsigned)((p.s.T + 127) / 128 * bh * p.nsplit)), block(256);
+      if (p.s.D == DP)
+        hipLaunchKernelGGL((fwd_pipe_kernel<T, false, true, 4, DP, 1, true, true>), grid, block, 0, st, p);
+      else
+        hipLaunchKernelGGL((fwd_pipe_kernel<T, false, true, 4, DP, 1, false, true>), grid, block, 0, st, p);
+      return;
+    }
+  }
   // workgroups per (batch, head): query blocks, or (causal) pairs of mirrored query blocks
   auto units = [](int64_t nqb) { return CAUSAL ? (nqb + 1) / 2 : nqb; };
   const int64_t nblk8 = units((p.s.T + 256 * QT - 1) / (256 * QT)) * bh;
@@ -517,7 +548,7 @@ static void fwd_pipe_launch(const FwdParams& p0, hipStream_t st) {
 // otherwise.
 template <typename T, bool CAUSAL>
 bool launch_fwd_pipe(const FwdParams& p, hipStream_t st, hipError_t* err) {
-  if (!(p.s.vec && p.s.D % 8 == 0 && p.s.D >= 8 && p.s.T > 128)) return false;
+  if (!(p.s.vec && p.s.D % 8 == 0 && p.s.D >= 8 && (p.s.T > 128 || p.nsplit > 1))) return false;
   // 32-bit byte offsets inside each (batch, head) slab of K and V
   if (!slab_fits_dma(p.s.M, p.k.sr, p.s.D) || !slab_fits_dma(p.s.M, p.v.sr, p.s.D)) return false;
   if ((int64_t)p.s.B * p.s.H == 0) {

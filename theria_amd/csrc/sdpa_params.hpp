@@ -37,7 +37,15 @@ struct FwdParams {
   float* lse;
   float* row_max;  // optional
   float* row_sum;  // optional
+  // Keys split over nsplit workgroups per query block (1: not split): each writes its part of every row to ws, which
+  // a combining launch turns into the outputs. ws: nsplit parts of B H T rows of fwd_split_row_floats(D) floats.
+  int nsplit;
+  float* ws;
 };
+// Parts of the keys a forward problem is split into where its query blocks alone would leave CUs idle (1: none).
+int fwd_splits(const Shape& s);
+// One row of a part: the unnormalised O (D rounded up to 4), its offset, row sum, row max and peaked bound.
+__host__ __device__ constexpr int fwd_split_row_floats(int D) { return (D + 3) / 4 * 4 + 4; }
 
 // How the dQ kernel obtains the row term delta_i of dS = P o (dP - delta), which it writes to delta (the
 // dK / dV kernel reads it there):
