@@ -1,0 +1,56 @@
+"""The split second-order kernels above head dim 64 (computed at 128): the JVP with two key groups and with one (256 or
+more 128-query blocks), the key-split row and query-split column kernels of the double backward, at the edges of their
+32-row subtiles and 64- or 128-row blocks, against the float64 oracle (bars: tests/bars.py)."""
+
+import pytest
+import torch
+
+import bars
+from oracle import sdpa_oracle as O
+from test_gpu_parity import _check_all_entry_points, make
+from theria_amd import _ops
+
+pytestmark = pytest.mark.gpu
+
+F16, BF16 = torch.float16, torch.bfloat16
+
+
+@pytest.mark.parametrize("dt,D", [(BF16, 72), (F16, 96), (BF16, 128)])
+def test_second_order_of_large_heads_matches_oracle(dt, D, hip_device):
+    for i, (T, M) in enumerate([(65, 63), (64, 65), (1, 129), (129, 1), (127, 32), (128, 128), (200, 33), (97, 300)]):
+        for causal in (False, True):
+            print(f"[split 128] {dt} T{T} M{M} D{D} causal={causal}", flush=True)
+            _check_all_entry_points((dt, 1, 2, T, M, D, causal), hip_device, seed=700 + i)
+
+
+@pytest.mark.parametrize("std", [1.0, 3.0])
+@pytest.mark.parametrize("T,M,causal", [(65, 65, True), (70, 33, False), (130, 64, False), (129, 129, True)])
+def test_jvp_of_many_blocks(T, M, causal, std, hip_device):
+    """256 (batch, head) pairs: one key group per workgroup; every tangent, one of them, and head dims below 128."""
+    for D in (80, 128):
+        print(f"[split 128 jvp] T{T} M{M} D{D} causal={causal} std{std}", flush=True)
+        (q, qc), (k, kc) = make((16, 16, T, D), BF16, hip_device, 1, std), make((16, 16, M, D), BF16, hip_device, 2, std)
+        (v, vc), (tq, tqc) = make((16, 16, M, D), BF16, hip_device, 3), make((16, 16, T, D), BF16, hip_device, 4)
+        (tk, tkc), (tv, tvc) = (make((16, 16, M, D), BF16, hip_device, 5 + i) for i in range(2))
+        s = D**-0.5
+        o, lse = _ops.fwd(q, k, v, s, causal)[:2]
+        for ts, tcs in (((tq, tk, tv), (tqc, tkc, tvc)), ((None, tk, None), (None, tkc, None))):
+            got = _ops.jvp(q, k, v, o, lse, *ts, s, causal)
+            bars.close(got, O.jvp(qc, kc, vc, *tcs, s, causal), what=f"JVP D{D}", **bars.tol(BF16))
+
+
+@pytest.mark.parametrize("D", [80, 128])
+def test_large_heads_on_strided_views(D, hip_device):
+    """Packed-projection views (row stride 3 H D): the same results as on contiguous copies, bit for bit."""
+    B, H, T = 2, 2, 150
+    print(f"[split 128 strided] D{D}", flush=True)
+    g = torch.Generator(device=hip_device).manual_seed(D)
+    q, k, v = torch.randn(B, T, 3, H, D, generator=g, device=hip_device).to(BF16).permute(2, 0, 3, 1, 4)
+    tq, tk, tv = torch.randn(B, T, 3, H, D, generator=g, device=hip_device).to(BF16).permute(2, 0, 3, 1, 4)
+    do = torch.randn(B, T, H, D, generator=g, device=hip_device).to(BF16).transpose(1, 2)
+    got = []
+    for ts in ((q, k, v, do, tq, tk, tv), [t.contiguous() for t in (q, k, v, do, tq, tk, tv)]):
+        o, lse = _ops.fwd(*ts[:3], D**-0.5, True)[:2]
+        got.append([_ops.jvp(*ts[:3], o, lse, *ts[4:], D**-0.5, True),
+                    *_ops.bwd_bwd(*ts[:3], o, ts[3], lse, None, *ts[4:], D**-0.5, True)])
+    assert all(torch.equal(a, b) for a, b in zip(*got))

@@ -33,11 +33,8 @@
 
 namespace theria {
 
-// DMA: 16-bit inputs with head dim exactly 64 or 128 and 16-byte-aligned rows. The K, tK, V, tV tiles are
-// then filled by LDS DMA into two sets of unpadded, XOR-swizzled buffers (sdpa_lds.hpp), one barrier per
-// tile with the next tile's copies in flight; otherwise they pass through registers into padded LDS rows.
-// NW: waves per workgroup, four or (without DMA) two for at most 64 queries.
-template <typename T, int DP, bool CAUSAL, bool HAS_O, bool DMA, int NW = 4>
+// Tiles pass through registers into padded LDS rows. NW: waves per workgroup, four or two (at most 64 queries).
+template <typename T, int DP, bool CAUSAL, bool HAS_O, int NW = 4>
 __global__ __launch_bounds__(64 * NW) void jvp_kernel(const JvpParams p) {
   using OP = Ops<T, DP, (sizeof(T) == 4 && DP <= 64)>;
   using F = typename OP::F;
@@ -46,16 +43,7 @@ __global__ __launch_bounds__(64 * NW) void jvp_kernel(const JvpParams p) {
   constexpr int BN = (DP == 128 || sizeof(T) == 4) ? 32 : 64;  // keys per tile (register budget)
   constexpr int PITCH = OP::PITCH;
   constexpr int NDT = DP / 32, NKC = DP / KC, NPC = 32 / KC, NST = BN / 32;
-  constexpr int TB = DMA ? BN * DP * 2 : BN * PITCH * (int)sizeof(T);  // bytes per tile
-  constexpr int TB2 = DMA ? TB : 16;                                    // second set (DMA only)
-  __shared__ __attribute__((aligned(1024))) char sK0[TB];
-  __shared__ __attribute__((aligned(1024))) char sV0[TB];
-  __shared__ __attribute__((aligned(1024))) char stK0[TB];
-  __shared__ __attribute__((aligned(1024))) char stV0[TB];
-  __shared__ __attribute__((aligned(1024))) char sK1[TB2];
-  __shared__ __attribute__((aligned(1024))) char sV1[TB2];
-  __shared__ __attribute__((aligned(1024))) char stK1[TB2];
-  __shared__ __attribute__((aligned(1024))) char stV1[TB2];
+  __shared__ __attribute__((aligned(16))) T sK0[BN * PITCH], sV0[BN * PITCH], stK0[BN * PITCH], stV0[BN * PITCH];
 
   const Shape& s = p.s;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 31, g = lane >> 5;
@@ -108,21 +96,8 @@ __global__ __launch_bounds__(64 * NW) void jvp_kernel(const JvpParams p) {
   int kend = s.M;
   if (CAUSAL) kend = min(s.M, qb * BM + BM);
   const int nkt = (kend + BN - 1) / BN;
-  auto colsf = [&](const char* t, int row, int c) -> F {
-    if constexpr (DMA)
-      return swz_cols<T, DP>(t, row, c);
-    else
-      return OP::cols((const T*)t, row, c);
-  };
-  auto rowsf = [&](const char* t, int kbase, int c, int col0) -> F {
-    if constexpr (DMA)
-      return swz_rows<T, DP>(t, kbase, c, col0);
-    else
-      return OP::rows((const T*)t, kbase, c, col0);
-  };
-
   // The key tile kt held in (tK, tV, ttK, ttV).
-  auto compute = [&](int kt, const char* tK, const char* tV, const char* ttK, const char* ttV) {
+  auto compute = [&](int kt, const T* tK, const T* tV, const T* ttK, const T* ttV) {
     const int k0 = kt * BN;
     if (CAUSAL && k0 > q0w + 31) return;
 
@@ -133,10 +108,10 @@ __global__ __launch_bounds__(64 * NW) void jvp_kernel(const JvpParams p) {
       gm[t] = zero16();
 #pragma unroll
       for (int c = 0; c < NKC; ++c) {
-        const F kfr = colsf(tK, t * 32 + li, c);
+        const F kfr = OP::cols(tK, t * 32 + li, c);
         sc[t] = OP::mma(kfr, qf[c], sc[t]);
         if (has_tq) gm[t] = OP::mma(kfr, tqf[c], gm[t]);
-        if (has_tk) gm[t] = OP::mma(colsf(ttK, t * 32 + li, c), qf[c], gm[t]);
+        if (has_tk) gm[t] = OP::mma(OP::cols(ttK, t * 32 + li, c), qf[c], gm[t]);
       }
     }
     const bool need_mask = (k0 + BN > s.M) || (CAUSAL && k0 + BN - 1 > q0w);
@@ -169,56 +144,17 @@ __global__ __launch_bounds__(64 * NW) void jvp_kernel(const JvpParams p) {
         }
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) {
-          const F vfr = rowsf(tV, t * 32, cc, dt * 32);
+          const F vfr = OP::rows(tV, t * 32, cc, dt * 32);
           accA[dt] = OP::mma(vfr, pgf, accA[dt]);
           if (SPLIT) accA[dt] = OP::mma(vfr, pgf_lo, accA[dt]);
           if (REBUILD) accO[dt] = OP::mma(vfr, pf, accO[dt]);
           if (REBUILD && SPLIT) accO[dt] = OP::mma(vfr, pf_lo, accO[dt]);
-          if (has_tv) accC[dt] = OP::mma(rowsf(ttV, t * 32, cc, dt * 32), pf, accC[dt]);
+          if (has_tv) accC[dt] = OP::mma(OP::rows(ttV, t * 32, cc, dt * 32), pf, accC[dt]);
         }
       }
   };
 
-  if constexpr (DMA) {
-    using Dma = SwzDma<NW, DP>;
-    constexpr int NSLAB = BN / Dma::SLAB_ROWS;
-    static_assert(NSLAB * Dma::SLAB_ROWS == BN, "key tiles must be whole DMA slabs");
-    const Dma dma(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane);
-    // Byte offsets fit in 32 bits: the host only selects this path when each (batch, head) slab of K, V,
-    // tK and tV spans less than 2^31 bytes.
-    const uint32_t krs = (uint32_t)p.k.sr * 2, vrs = (uint32_t)p.v.sr * 2;
-    const uint32_t tkrs = has_tk ? (uint32_t)p.tk.sr * 2 : 0u, tvrs = has_tv ? (uint32_t)p.tv.sr * 2 : 0u;
-    const rsrc_t krsrc = make_rsrc(K, (uint32_t)slab_span(s.M, krs, 2 * DP)),
-                  vrsrc = make_rsrc(V, (uint32_t)slab_span(s.M, vrs, 2 * DP));
-    const rsrc_t tkrsrc = make_rsrc(has_tk ? (const void*)TK : (const void*)K, (uint32_t)slab_span(s.M, tkrs, 2 * DP));
-    const rsrc_t tvrsrc = make_rsrc(has_tv ? (const void*)TV : (const void*)V, (uint32_t)slab_span(s.M, tvrs, 2 * DP));
-    auto issue = [&](int kt, char* tK, char* tV, char* ttK, char* ttV) {
-      const int k0 = kt * BN;
-      dma.template issue_clamped<NSLAB>(krsrc, krs, k0, s.M, tK);
-      dma.template issue_clamped<NSLAB>(vrsrc, vrs, k0, s.M, tV);
-      if (has_tk) dma.template issue_clamped<NSLAB>(tkrsrc, tkrs, k0, s.M, ttK);
-      if (has_tv) dma.template issue_clamped<NSLAB>(tvrsrc, tvrs, k0, s.M, ttV);
-    };
-    // Tile kt from the set c*; the next tile's copies go to the set n* (read in the previous step, which
-    // every wave has finished at the barrier).
-    auto step = [&](int kt, const char* cK, const char* cV, const char* ctK, const char* ctV, char* nK, char* nV,
-                    char* ntK, char* ntV) {
-      wait_vm_all();
-      __syncthreads();
-      if (kt + 1 < nkt) issue(kt + 1, nK, nV, ntK, ntV);
-      compute(kt, cK, cV, ctK, ctV);
-      __builtin_amdgcn_sched_barrier(0);  // keep the two unrolled steps apart (register pressure)
-    };
-    if (nkt > 0) {
-      issue(0, sK0, sV0, stK0, stV0);
-      int kt = 0;
-      for (; kt + 1 < nkt; kt += 2) {
-        step(kt, sK0, sV0, stK0, stV0, sK1, sV1, stK1, stV1);
-        step(kt + 1, sK1, sV1, stK1, stV1, sK0, sV0, stK0, stV0);
-      }
-      if (kt < nkt) step(kt, sK0, sV0, stK0, stV0, sK1, sV1, stK1, stV1);
-    }
-  } else {
+  {
     TileStage<T, BN, DP, NT> gK, gV, gtK, gtV;
     auto prefetch = [&](int k0) {
       gK.load(K, p.k.sr, k0, s.M, s.D, s.vec);
@@ -229,10 +165,10 @@ __global__ __launch_bounds__(64 * NW) void jvp_kernel(const JvpParams p) {
     if (nkt > 0) prefetch(0);
     for (int kt = 0; kt < nkt; ++kt) {
       __syncthreads();
-      OP::store(gK, (T*)sK0);
-      OP::store(gV, (T*)sV0);
-      if (has_tk) OP::store(gtK, (T*)stK0);
-      if (has_tv) OP::store(gtV, (T*)stV0);
+      OP::store(gK, sK0);
+      OP::store(gV, sV0);
+      if (has_tk) OP::store(gtK, stK0);
+      if (has_tv) OP::store(gtV, stV0);
       __syncthreads();
       if (kt + 1 < nkt) prefetch((kt + 1) * BN);
       compute(kt, sK0, sV0, stK0, stV0);
@@ -272,34 +208,41 @@ __global__ __launch_bounds__(64 * NW) void jvp_kernel(const JvpParams p) {
   }
 }
 
-// 16-bit inputs at head dims up to 64 (a multiple of 8, computed at 64 with the tile columns past D zero) with
-// LDS-DMA tiles: the same JVP with the keys of a query block split between two groups of four waves
+// 16-bit inputs with LDS-DMA tiles (a head dim that is a multiple of 8, computed at DP = 64 or 128 with the tile columns
+// past D zero): the same JVP with the keys of a query block split between two groups. DP = 64: groups of four waves
 // (eight-wave workgroups), so that a SIMD holds two waves at 256 registers each
 // where jvp_kernel holds one at ~380 (config 4: B H T / 32 = 1024 query waves for 1024 SIMDs; 27.1 -> 23.0 us
 // there, same box). Each group streams its own half of the key tiles (64 keys per tile, 128 KB of LDS in
 // all) through its own double-buffered tiles; both groups meet at the same barrier every step (a group
 // whose half is shorter idles through the last step). The float32 partial sums of group 1 (accumulators,
-// row sums) pass to group 0 through LDS at the end. ALL: every tangent is given (the presence tests are then
+// row sums) are exchanged through LDS at the end. DP = 128, whose accumulators take a whole SIMD per wave: G = 2 groups of
+// two waves (64 queries, 32-key tiles) where 128-query workgroups would leave CUs idle, else G = 1 group of four waves
+// (128 queries, no exchange), which reads each tile for twice the queries (us, the one-group kernel it replaced -> G = 2 /
+// G = 1, bfloat16: B2 H8 T1024 86 -> 32 / 46, B2 H16 T1024 90 -> 66 / 56, B1 H4 T8192 605 -> 405 / 356, B64 H8 T1000 M96
+// 250 -> 324 / 221, B2 H8 T1024 causal 86 -> 33). ALL: every tangent is given (the presence tests are then
 // constants, and the loop body has no branches between its products).
-template <typename T, bool CAUSAL, bool HAS_O, bool ALL, bool FD>
-__global__ __launch_bounds__(512, 2) void jvp_ksplit_kernel(const JvpParams p) {
+template <typename T, bool CAUSAL, bool ALL, bool FD, int DP, int G>
+__global__ __launch_bounds__(DP == 64 ? 512 : 256, DP == 64 ? 2 : 1) void jvp_ksplit_kernel(const JvpParams p) {
   using MM = Mfma<T>;
   using F = typename MM::frag_t;
   static_assert(sizeof(T) == 2, "16-bit inputs only");
-  constexpr int DP = 64, NW = 4, BM = 32 * NW, BN = 64, NST = BN / 32;
+  static_assert(G == 2 || DP == 128, "one group only at DP = 128");
+  constexpr int NW = DP == 64 ? 4 : 4 / G, GT = 64 * NW, BM = 32 * NW, BN = DP == 64 ? 64 : 32, NST = BN / 32;
   constexpr int NDT = DP / 32, NKC = DP / MM::KC, NPC = 32 / MM::KC;
   constexpr int TB = BN * DP * 2;  // bytes per tile
-  using Dma = SwzDma<NW, DP>;
+  // DP = 64: each group fills its own tiles; 128: all four waves fill both groups' (a slab is then 16 rows)
+  constexpr bool JOINT = DP == 128 && G == 2;
+  using Dma = SwzDma<4, DP>;
   constexpr int NSLAB = BN / Dma::SLAB_ROWS;
   static_assert(NSLAB * Dma::SLAB_ROWS == BN, "key tiles must be whole DMA slabs");
   // [group][set][K, V, tK, tV]; reused for the partial sums after the key loop
-  __shared__ __attribute__((aligned(1024))) char smem[2 * 2 * 4 * TB];
-  static_assert(sizeof(smem) >= (2 * 3 * 16 + 4) * 256 * 4, "the partial sums fit in the tile memory");
+  __shared__ __attribute__((aligned(1024))) char smem[G * 2 * 4 * TB];
+  static_assert(G == 1 || sizeof(smem) >= (NDT * 3 * 16 + 4) * GT * 4, "the partial sums fit in the tile memory");
 
   const Shape& s = p.s;
   const int lane = threadIdx.x & 63, li = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int grp = wave >> 2, wig = wave & 3;  // key group, wave in group
+  const int grp = (unsigned)wave / NW, wig = (unsigned)wave % NW;  // key group, wave in group
   const int nqb = (s.T + BM - 1) / BM;
   const int bid = xcd_remap(blockIdx.x, gridDim.x);
   const int bh = bid / nqb;
@@ -344,7 +287,7 @@ __global__ __launch_bounds__(512, 2) void jvp_ksplit_kernel(const JvpParams p) {
   int kend = s.M;
   if (CAUSAL) kend = min(s.M, qb * BM + BM);
   const int nkt = (kend + BN - 1) / BN;
-  const int half = (nkt + 1) / 2;
+  const int half = (nkt + G - 1) / G;
   const int kt0 = grp * half, kt1 = min(nkt, kt0 + half);  // this group's tiles [kt0, kt1)
 
   // The key tile kt held in (tK, tV, ttK, ttV): as jvp_kernel, 32-key subtiles one after the other. MASK: the
@@ -410,24 +353,29 @@ __global__ __launch_bounds__(512, 2) void jvp_ksplit_kernel(const JvpParams p) {
     }
   };
 
-  // Head dims below 64 (a multiple of 8): the tiles' columns D .. 63 are filled with zeros by the DMA.
-  const Dma dma(wig, lane, FD ? 8 : s.D / 8);  // FD: head dim 64
+  // Head dims below DP (a multiple of 8): the tiles' columns past D are filled with zeros by the DMA.
+  const Dma dma(JOINT ? wave : wig, lane, FD ? DP / 8 : s.D / 8);  // FD: head dim DP
   // Byte offsets fit in 32 bits: the host only selects this path when each (batch, head) slab of K, V, tK
   // and tV spans less than 2^31 bytes.
   const uint32_t krs = (uint32_t)p.k.sr * 2, vrs = (uint32_t)p.v.sr * 2;
   const uint32_t tkrs = has_tk ? (uint32_t)p.tk.sr * 2 : 0u, tvrs = has_tv ? (uint32_t)p.tv.sr * 2 : 0u;
-  const int64_t rb = 2 * (FD ? 64 : s.D);  // bytes of a row the DMA reads
+  const int64_t rb = 2 * (FD ? DP : s.D);  // bytes of a row the DMA reads
   const rsrc_t krsrc = make_rsrc(K, (uint32_t)slab_span(s.M, krs, rb)),
                vrsrc = make_rsrc(V, (uint32_t)slab_span(s.M, vrs, rb));
   const rsrc_t tkrsrc = make_rsrc(has_tk ? (const void*)TK : (const void*)K, (uint32_t)slab_span(s.M, tkrs, rb));
   const rsrc_t tvrsrc = make_rsrc(has_tv ? (const void*)TV : (const void*)V, (uint32_t)slab_span(s.M, tvrs, rb));
-  auto tile = [&](int set, int a) { return smem + ((grp * 2 + set) * 4 + a) * TB; };  // a: K, V, tK, tV
-  auto issue = [&](int kt, int set) {
+  auto tile_of = [&](int gg, int set, int a) { return smem + ((gg * 2 + set) * 4 + a) * TB; };  // a: K, V, tK, tV
+  auto tile = [&](int set, int a) { return tile_of(grp, set, a); };
+  auto issue_one = [&](int gg, int kt, int set) __attribute__((always_inline)) {
     const int k0 = kt * BN;
-    dma.template issue_clamped<NSLAB>(krsrc, krs, k0, s.M, tile(set, 0));
-    dma.template issue_clamped<NSLAB>(vrsrc, vrs, k0, s.M, tile(set, 1));
-    if (has_tk) dma.template issue_clamped<NSLAB>(tkrsrc, tkrs, k0, s.M, tile(set, 2));
-    if (has_tv) dma.template issue_clamped<NSLAB>(tvrsrc, tvrs, k0, s.M, tile(set, 3));
+    dma.template issue_clamped<NSLAB>(krsrc, krs, k0, s.M, tile_of(gg, set, 0));
+    dma.template issue_clamped<NSLAB>(vrsrc, vrs, k0, s.M, tile_of(gg, set, 1));
+    if (has_tk) dma.template issue_clamped<NSLAB>(tkrsrc, tkrs, k0, s.M, tile_of(gg, set, 2));
+    if (has_tv) dma.template issue_clamped<NSLAB>(tvrsrc, tvrs, k0, s.M, tile_of(gg, set, 3));
+  };
+  auto issue_joint = [&](int i) __attribute__((always_inline)) {  // step i's tiles of both groups
+    if (i < half) issue_one(0, i, i & 1);
+    if (i < half && half + i < nkt) issue_one(1, half + i, i & 1);
   };
   // Step i: tile kt0 + i of this group (if it has one) from set i & 1; the next one's copies go to the other
   // set, read in step i - 1, which every wave has finished at the barrier. The tiles from mask_from on may
@@ -439,7 +387,10 @@ __global__ __launch_bounds__(512, 2) void jvp_ksplit_kernel(const JvpParams p) {
       const int kt = kt0 + i;
       wait_vm_all();
       __syncthreads();
-      if (kt + 1 < kt1) issue(kt + 1, (i + 1) & 1);
+      if constexpr (JOINT)
+        issue_joint(i + 1);
+      else if (kt + 1 < kt1)
+        issue_one(grp, kt + 1, (i + 1) & 1);
       if (kt < kt1) compute(split_tag, mask_tag, kt, tile(i & 1, 0), tile(i & 1, 1), tile(i & 1, 2), tile(i & 1, 3));
     };
     const int isplit = min(half, max(0, mask_from - kt0));
@@ -447,58 +398,20 @@ __global__ __launch_bounds__(512, 2) void jvp_ksplit_kernel(const JvpParams p) {
     for (; i < isplit; ++i) step(std::false_type{}, i);
     for (; i < half; ++i) step(std::true_type{}, i);
   };
-  if (kt0 < kt1) issue(kt0, 0);
+  if constexpr (JOINT)
+    issue_joint(0);
+  else if (kt0 < kt1)
+    issue_one(grp, kt0, 0);
   // The waves of a workgroup may take different copies of the loop: both meet the same barriers.
   if (split)
     sweep(std::integral_constant<bool, true>{});
   else
     sweep(std::integral_constant<bool, false>{});
 
-  // The groups finish one column tile each (group g the tile dt = g): each hands the other tile's partial sums
-  // and its row sums to the other group in one round, 16 bytes per lane per store (elements 4c .. 4c + 3 of
-  // accumulator a of lane l of wave w of group g at words (((g * 3 + a) * 4 + c) * 256 + w * 64 + l) * 4, so one
-  // store instruction covers 1 KiB of consecutive words), then stores its half of the output.
-  static_assert(NDT == 2, "one column tile per group");
-  float* buf = reinterpret_cast<float*>(smem);
-  f32x4_t* buf4 = reinterpret_cast<f32x4_t*>(smem);
-  constexpr int RS = 2 * 3 * 4 * 256 * 4;  // the row sums, [group][l, c]
-  __syncthreads();  // every wave is done with the last tile
-  auto finish = [&](auto keep_tag) __attribute__((always_inline)) {
-    constexpr int KEEP = decltype(keep_tag)::value, GIVE = 1 - KEEP;
-    const int mine = KEEP * 3 * 4 * 256, theirs = GIVE * 3 * 4 * 256;  // group KEEP writes at `mine`
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int i = c * 256 + wig * 64 + lane;
-      buf4[mine + i] = f32x4_t{accA[GIVE][4 * c], accA[GIVE][4 * c + 1], accA[GIVE][4 * c + 2], accA[GIVE][4 * c + 3]};
-      buf4[mine + 4 * 256 + i] =
-          f32x4_t{accO[GIVE][4 * c], accO[GIVE][4 * c + 1], accO[GIVE][4 * c + 2], accO[GIVE][4 * c + 3]};
-      if (has_tv)
-        buf4[mine + 8 * 256 + i] =
-            f32x4_t{accC[GIVE][4 * c], accC[GIVE][4 * c + 1], accC[GIVE][4 * c + 2], accC[GIVE][4 * c + 3]};
-    }
-    buf[RS + KEEP * 512 + wig * 64 + lane] = lpart;
-    buf[RS + KEEP * 512 + 256 + wig * 64 + lane] = cpart;
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int i = c * 256 + wig * 64 + lane;
-      const f32x4_t a = buf4[theirs + i], o4 = buf4[theirs + 4 * 256 + i];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        accA[KEEP][4 * c + e] += a[e];
-        accO[KEEP][4 * c + e] += o4[e];
-      }
-      if (has_tv) {
-        const f32x4_t c4 = buf4[theirs + 8 * 256 + i];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) accC[KEEP][4 * c + e] += c4[e];
-      }
-    }
-    lpart += buf[RS + GIVE * 512 + wig * 64 + lane];
-    cpart += buf[RS + GIVE * 512 + 256 + wig * 64 + lane];
-
-    // Epilogue as jvp_kernel's (O rebuilt from the same P; normalize: P divided by its own row sum), for the
-    // columns of tile KEEP.
+  // Epilogue as jvp_kernel's (O rebuilt from the same P; normalize: P divided by its own row sum), for the N column tiles
+  // from DT0 on.
+  auto store = [&](auto dt0_tag, auto n_tag) __attribute__((always_inline)) {
+    constexpr int DT0 = decltype(dt0_tag)::value, N = decltype(n_tag)::value;
     float inv = 1.f;
     if (p.normalize) {
       const float L = pair_sum(lpart);
@@ -508,17 +421,70 @@ __global__ __launch_bounds__(512, 2) void jvp_ksplit_kernel(const JvpParams p) {
     if (qvalid) {
       T* TO = (T*)p.tout.p + b * p.tout.sb + h * p.tout.sh;
 #pragma unroll
-      for (int qd = 0; qd < 4; ++qd) {
-        const int d0 = KEEP * 32 + 8 * qd + 4 * g;
-        float r4[4];
+      for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int qd = 0; qd < 4; ++qd) {
+          const int dt = DT0 + j, d0 = dt * 32 + 8 * qd + 4 * g;
+          float r4[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float ov = accO[dt][4 * qd + e] * inv;
+            r4[e] = inv * (s.scale * accA[dt][4 * qd + e] + accC[dt][4 * qd + e]) - cval * ov;
+          }
+          store4<T>(TO, p.tout.sr, myq, d0, s.D, r4[0], r4[1], r4[2], r4[3], s.vec);
+        }
+    }
+  };
+  if constexpr (G == 1) {
+    store(std::integral_constant<int, 0>{}, std::integral_constant<int, NDT>{});
+    return;
+  }
+  // The groups finish NH column tiles each (group g the tiles g NH ..): each hands the other's partial sums and its row
+  // sums to the other group in one round, 16 bytes per lane per store (elements 4c .. 4c + 3 of accumulator a of tile j
+  // of lane l of wave w of group g at words ((((g * NH + j) * 3 + a) * 4 + c) * GT + w * 64 + l) * 4, so one store
+  // instruction covers 1 KiB of consecutive words), then stores its part of the output.
+  constexpr int NH = NDT / 2;
+  float* buf = reinterpret_cast<float*>(smem);
+  f32x4_t* buf4 = reinterpret_cast<f32x4_t*>(smem);
+  constexpr int RS = NDT * 3 * 4 * GT * 4;  // the row sums, [group][l, c]
+  __syncthreads();  // every wave is done with the last tile
+  auto finish = [&](auto keep_tag) __attribute__((always_inline)) {
+    constexpr int KEEP = decltype(keep_tag)::value, GIVE = 1 - KEEP;
+    const int me = wig * 64 + lane;
+#pragma unroll
+    for (int j = 0; j < NH; ++j)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int i = ((KEEP * NH + j) * 3 * 4 + c) * GT + me, dt = GIVE * NH + j;
+        auto q4 = [&](const f32x16_t& a) { return f32x4_t{a[4 * c], a[4 * c + 1], a[4 * c + 2], a[4 * c + 3]}; };
+        buf4[i] = q4(accA[dt]);
+        buf4[i + 4 * GT] = q4(accO[dt]);
+        if (has_tv) buf4[i + 8 * GT] = q4(accC[dt]);
+      }
+    buf[RS + KEEP * 2 * GT + me] = lpart;
+    buf[RS + KEEP * 2 * GT + GT + me] = cpart;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NH; ++j)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int i = ((GIVE * NH + j) * 3 * 4 + c) * GT + me, dt = KEEP * NH + j;
+        const f32x4_t a = buf4[i], o4 = buf4[i + 4 * GT];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float ov = accO[KEEP][4 * qd + e] * inv;
-          r4[e] = inv * (s.scale * accA[KEEP][4 * qd + e] + accC[KEEP][4 * qd + e]) - cval * ov;
+          accA[dt][4 * c + e] += a[e];
+          accO[dt][4 * c + e] += o4[e];
         }
-        store4<T>(TO, p.tout.sr, myq, d0, s.D, r4[0], r4[1], r4[2], r4[3], s.vec);
+        if (has_tv) {
+          const f32x4_t c4 = buf4[i + 8 * GT];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) accC[dt][4 * c + e] += c4[e];
+        }
       }
-    }
+    lpart += buf[RS + GIVE * 2 * GT + me];
+    cpart += buf[RS + GIVE * 2 * GT + GT + me];
+
+    store(std::integral_constant<int, KEEP * NH>{}, std::integral_constant<int, NH>{});
   };
   // both branches meet the one barrier inside finish
   if (grp == 0)
@@ -536,34 +502,41 @@ struct JvpLauncher {
     if (nblk == 0) return hipSuccess;
     if constexpr (sizeof(T) == 2) {
       // LDS-DMA tiles: 16-byte-aligned views, each streamed (batch, head) slab < 2^31 bytes, and a head dim that
-      // is a multiple of 8 up to 64 (the key-split kernel, columns past D zero-filled) or exactly 128
-      bool ok = p.s.vec && (DP <= 64 ? p.s.D % 8 == 0 : p.s.D == DP);
+      // is a multiple of 8 (columns past D zero-filled)
+      bool ok = p.s.vec && p.s.D % 8 == 0;
       for (const View* v : {&p.k, &p.v, &p.tk, &p.tv})
         if (v->p && !slab_fits_dma(p.s.M, v->sr, p.s.D)) ok = false;
       if (ok) {
-        if constexpr (DP <= 64) {
-          const bool all = p.tq.p && p.tk.p && p.tv.p, fd = p.s.D == 64;
-          const dim3 grid((unsigned)nblk), block(512);
+        const bool all = p.tq.p && p.tk.p && p.tv.p, fd = p.s.D == (DP <= 64 ? 64 : 128);
+        auto go = [&](auto kp_tag, auto g_tag) {
+          constexpr int KP = decltype(kp_tag)::value, G = decltype(g_tag)::value, BM = KP == 64 ? 128 : 128 / G;
+          const dim3 grid((unsigned)((int64_t)((p.s.T + BM - 1) / BM) * p.s.B * p.s.H)), block(KP == 64 ? 512 : 256);
           if (all && fd)
-            hipLaunchKernelGGL((jvp_ksplit_kernel<T, CAUSAL, HAS_O, true, true>), grid, block, 0, st, p);
+            hipLaunchKernelGGL((jvp_ksplit_kernel<T, CAUSAL, true, true, KP, G>), grid, block, 0, st, p);
           else if (all)
-            hipLaunchKernelGGL((jvp_ksplit_kernel<T, CAUSAL, HAS_O, true, false>), grid, block, 0, st, p);
+            hipLaunchKernelGGL((jvp_ksplit_kernel<T, CAUSAL, true, false, KP, G>), grid, block, 0, st, p);
           else if (fd)
-            hipLaunchKernelGGL((jvp_ksplit_kernel<T, CAUSAL, HAS_O, false, true>), grid, block, 0, st, p);
+            hipLaunchKernelGGL((jvp_ksplit_kernel<T, CAUSAL, false, true, KP, G>), grid, block, 0, st, p);
           else
-            hipLaunchKernelGGL((jvp_ksplit_kernel<T, CAUSAL, HAS_O, false, false>), grid, block, 0, st, p);
-        } else
-          hipLaunchKernelGGL((jvp_kernel<T, DP, CAUSAL, HAS_O, true>), dim3((unsigned)nblk), dim3(256), 0, st, p);
+            hipLaunchKernelGGL((jvp_ksplit_kernel<T, CAUSAL, false, false, KP, G>), grid, block, 0, st, p);
+        };
+        using std::integral_constant;
+        if constexpr (DP <= 64)
+          go(integral_constant<int, 64>{}, integral_constant<int, 2>{});
+        else if (p.s.T > 64 && nblk >= device_cu_count())
+          go(integral_constant<int, 128>{}, integral_constant<int, 1>{});
+        else
+          go(integral_constant<int, 128>{}, integral_constant<int, 2>{});
         return hipGetLastError();
       }
     }
     // at most 64 queries, and more workgroups than CUs (one four-wave workgroup per CU is resident): float32 B400 H4
     // T64 D16 42 -> 34 us
     if (p.s.T <= 64 && nblk > device_cu_count()) {
-      hipLaunchKernelGGL((jvp_kernel<T, DP, CAUSAL, HAS_O, false, 2>), dim3((unsigned)nblk), dim3(128), 0, st, p);
+      hipLaunchKernelGGL((jvp_kernel<T, DP, CAUSAL, HAS_O, 2>), dim3((unsigned)nblk), dim3(128), 0, st, p);
       return hipGetLastError();
     }
-    hipLaunchKernelGGL((jvp_kernel<T, DP, CAUSAL, HAS_O, false>), dim3((unsigned)nblk), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((jvp_kernel<T, DP, CAUSAL, HAS_O>), dim3((unsigned)nblk), dim3(256), 0, st, p);
     return hipGetLastError();
   }
 };

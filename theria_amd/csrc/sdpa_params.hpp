@@ -108,7 +108,7 @@ struct BwdBwdParams {
   float* r_row;
   float* t_row;
   MutView out_gq, out_gk, out_gv;
-  // The key-split row kernel (16-bit, head dim 64) forms the row statistics itself from the forward's lse
+  // The key-split row kernel (16-bit) forms the row statistics itself from the forward's lse
   // (lse_fwd) and writes the row term and the exact normaliser to z_out and lse_out, which the column kernel
   // then reads as delta and lse.
   const float* lse_fwd;
