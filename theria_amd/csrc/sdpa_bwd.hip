@@ -124,6 +124,9 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
   int kend = s.M;
   if (CAUSAL) kend = min(s.M, qb * BM + BM);
   const int nkt = (kend + BN - 1) / BN;
+  // Tiles with every key in range and visible to the block; the others take their own copy of each loop (a mask behind a
+  // uniform branch becomes a compare and a select per score in every tile).
+  const int nfull = min(nkt, CAUSAL ? min(s.M / BN, qb * BM / BN) : s.M / BN);
 
   // The row term from a pass over the key tiles: always for the frozen / normalised forms, and (16-bit) for a
   // workgroup holding a peaked row in place of dO . O, whose 16-bit P rounding in the forward's PV product
@@ -147,15 +150,22 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
       m_run[j] = -THERIA_INF;
     }
     TileStage<T, BN, DP, NT> pK, pV;
-    for (int kt = 0; kt < nkt; ++kt) {
+    if (nkt > 0) {
+      pK.load(K, p.k.sr, 0, s.M, s.D, s.vec);
+      pV.load(V, p.v.sr, 0, s.M, s.D, s.vec);
+    }
+    auto sums = [&](auto mask_tag, int kt) __attribute__((always_inline)) {
+      constexpr bool MASK = decltype(mask_tag)::value;
       const int k0 = kt * BN;
-      pK.load(K, p.k.sr, k0, s.M, s.D, s.vec);
-      pV.load(V, p.v.sr, k0, s.M, s.D, s.vec);
       __syncthreads();
       OP::store(pK, sK);
       OP::store(pV, sV);
       __syncthreads();
-      if (CAUSAL && k0 > q0w + 32 * QT - 1) continue;
+      if (kt + 1 < nkt) {
+        pK.load(K, p.k.sr, k0 + BN, s.M, s.D, s.vec);
+        pV.load(V, p.v.sr, k0 + BN, s.M, s.D, s.vec);
+      }
+      if (CAUSAL && k0 > q0w + 32 * QT - 1) return;
       f32x16_t sc[QT], dpp[QT];
 #pragma unroll
       for (int j = 0; j < QT; ++j) sc[j] = dpp[j] = zero16();
@@ -177,7 +187,7 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
           float mt = m_run[j];
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            t[r] = k0 + acc_row(r, g) < lim ? mul_rn(sc[j][r], c2) : -THERIA_INF;
+            t[r] = !MASK || k0 + acc_row(r, g) < lim ? mul_rn(sc[j][r], c2) : -THERIA_INF;
             mt = fmaxf(mt, t[r]);
           }
           if (mt > m_run[j]) {  // m_run = -inf: the partial sums are still 0
@@ -196,13 +206,16 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const float pv = k0 + acc_row(r, g) < lim ? fast_exp2(fmaf(sc[j][r], c2, -lse2[j])) : 0.f;
+          const float pv = !MASK || k0 + acc_row(r, g) < lim ? fast_exp2(fmaf(sc[j][r], c2, -lse2[j])) : 0.f;
           a_part[j] = fmaf(pv, dpp[j][r], a_part[j]);
           l_part[j] += pv;
           p_mx[j] = fmaxf(p_mx[j], pv);
         }
       }
-    }
+    };
+    int kt = 0;
+    for (; kt < nfull; ++kt) sums(std::false_type{}, kt);
+    for (; kt < nkt; ++kt) sums(std::true_type{}, kt);
 #pragma unroll
     for (int j = 0; j < QT; ++j) {
       float mm = -THERIA_INF;
@@ -244,7 +257,8 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
     stK.load(K, p.k.sr, 0, s.M, s.D, s.vec);
     stV.load(V, p.v.sr, 0, s.M, s.D, s.vec);
   }
-  for (int kt = 0; kt < nkt; ++kt) {
+  auto step = [&](auto mask_tag, int kt) __attribute__((always_inline)) {
+    constexpr bool MASK = decltype(mask_tag)::value;
     const int k0 = kt * BN;
     __syncthreads();
     OP::store(stK, sK);
@@ -254,7 +268,7 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
       stK.load(K, p.k.sr, k0 + BN, s.M, s.D, s.vec);
       stV.load(V, p.v.sr, k0 + BN, s.M, s.D, s.vec);
     }
-    if (CAUSAL && k0 > q0w + 32 * QT - 1) continue;
+    if (CAUSAL && k0 > q0w + 32 * QT - 1) return;
 
     // dP starts from -delta, so the MFMA yields dP - delta; float32 forms dP from zero and subtracts after, so
     // that dP rounds exactly as in the row-term pass and dP - delta keeps only delta's own rounding (a row whose
@@ -277,8 +291,8 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
         dp[j] = OP::mma(vfr, of[j][c], dp[j]);
       }
     }
-    // Boundary tiles only (a uniform branch): masked scores become -inf, so P = 0 there.
-    if ((k0 + BN > s.M) || (CAUSAL && k0 + BN - 1 > q0w)) {
+    // masked scores become -inf, so P = 0 there
+    if constexpr (MASK) {
 #pragma unroll
       for (int j = 0; j < QT; ++j) {
         const int lim = CAUSAL ? min(s.M, q0w + 32 * j + li + 1) : s.M;  // first key this query cannot see
@@ -313,7 +327,10 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
         }
       }
     }
-  }
+  };
+  int kt = 0;
+  for (; kt < nfull; ++kt) step(std::false_type{}, kt);
+  for (; kt < nkt; ++kt) step(std::true_type{}, kt);
 
   };
   if (sizeof(T) == 2 && __any(peaked))
@@ -419,7 +436,8 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(c
   if (nqt > 0) prefetch(qbeg);
 
   // S = Q K^T and dP = dO V^T - delta for the 32-row subtile qr0 of the staged tile (masked scores -inf).
-  auto scores = [&](int qr0, int q0t, f32x16_t (&sc)[KT], f32x16_t (&dp)[KT]) {
+  auto scores = [&](auto mask_tag, int qr0, int q0t, f32x16_t (&sc)[KT], f32x16_t (&dp)[KT]) __attribute__((always_inline)) {
+    constexpr bool MASK = decltype(mask_tag)::value;
     f32x4_t del4[4];
 #pragma unroll
     for (int qd = 0; qd < 4; ++qd) del4[qd] = *reinterpret_cast<const f32x4_t*>(sDel + qr0 + 8 * qd + 4 * g);
@@ -440,19 +458,20 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(c
         for (int t = 0; t < KT; ++t) dp[t] = OP::template mma<true>(ofr, vf[t][c], dp[t]);
       }
     }
-    // Boundary sub-tiles only (a uniform branch): masked scores become -inf, so P = 0 there.
-    if ((kw0 + 32 * KT > s.M) || (CAUSAL && kw0 + 32 * KT - 1 > q0t)) {
+    // Causal, on the diagonal: masked scores become -inf, so P = 0 there. (Keys past the end need none: their lane's
+    // results are not stored.)
+    if constexpr (MASK) {
 #pragma unroll
       for (int t = 0; t < KT; ++t) {
         const int mykey = kw0 + 32 * t + li;
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          if (mykey >= s.M || (CAUSAL && mykey > q0t + acc_row(r, g))) sc[t][r] = -THERIA_INF;
+          if (mykey > q0t + acc_row(r, g)) sc[t][r] = -THERIA_INF;
       }
     }
   };
 
-  for (int it = 0; it < nqt; ++it) {
+  auto step = [&](auto mask_tag, int it) __attribute__((always_inline)) {
     const int q0 = qbeg + it * BM;
     __syncthreads();
     OP::store(stQ, sQ);
@@ -479,7 +498,7 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(c
 #pragma unroll
       for (int qd = 0; qd < 4; ++qd) lse4[qd] = *reinterpret_cast<const f32x4_t*>(sLse + qr0 + 8 * qd + 4 * g);
       f32x16_t sc[KT], dp[KT];
-      scores(qr0, q0t, sc, dp);
+      scores(mask_tag, qr0, q0t, sc, dp);
 #pragma unroll
       for (int t = 0; t < KT; ++t)
 #pragma unroll
@@ -525,7 +544,7 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(c
 #pragma unroll
           for (int qd = 0; qd < 4; ++qd) lse4[qd] = *reinterpret_cast<const f32x4_t*>(sLse + qr0 + 8 * qd + 4 * g);
           f32x16_t sc[KT], dp[KT];
-          scores(qr0, q0t, sc, dp);
+          scores(mask_tag, qr0, q0t, sc, dp);
 #pragma unroll
           for (int cc = 0; cc < NPC; ++cc) {
 #pragma unroll
@@ -548,7 +567,12 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(c
         }
       }
     }
-  }
+  };
+  // causal: the tiles before the block's last key, then the unmasked ones
+  const int ndiag = CAUSAL ? min(nqt, (key0 + BN - 1 - qbeg + BM - 1) / BM) : 0;
+  int it = 0;
+  for (; it < ndiag; ++it) step(std::integral_constant<bool, CAUSAL>{}, it);
+  for (; it < nqt; ++it) step(std::false_type{}, it);
 
   // Epilogue: lane holds column d = dt*32 + li of rows (keys) kw0 + 32 t + acc_row(r, g).
   T* DV = (T*)p.dv.p + b * p.dv.sb + h * p.dv.sh;

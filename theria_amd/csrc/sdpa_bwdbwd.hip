@@ -76,6 +76,8 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
   int kend = s.M;
   if (CAUSAL) kend = min(s.M, qb * BM + BM);
   const int nkt = (kend + BN - 1) / BN;
+  // tiles that need no mask (their own copy of the loops; at float32 head dim 128, whose loop spills, only one copy)
+  const int nfull = sizeof(T) == 4 && DP == 128 ? 0 : min(nkt, CAUSAL ? min(s.M / BN, qb * BM / BN) : s.M / BN);
   // 16-bit workgroups holding a row flagged peaked in lse take the exact form (uniform). Causal ones with at
   // most half the longest workgroup's key tiles run both of its passes in the first launch, inside that
   // launch's slack (every head's first query block holds such rows); the others are the second pass's.
@@ -137,9 +139,10 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
   // The key tile kt held in (tK, tV, tgK, tgV), as 32-key subtiles.
   // PASS: 0 the pre-pass (sums only: for the centres over the first tile, or for r and t over every tile),
   // 1 the common pass, 3 the exact pass (Gbar_S from exact row terms r, t; 16-bit only).
-  auto compute = [&](auto pass_tag, int kt, const T* tK, const T* tV, const T* tgK,
+  auto compute = [&](auto pass_tag, auto mask_tag, int kt, const T* tK, const T* tV, const T* tgK,
                      const T* tgV) __attribute__((always_inline)) {
     constexpr int PASS = decltype(pass_tag)::value;
+    constexpr bool MASK = decltype(mask_tag)::value;  // the tile reaches past the last key or past the block's first query
     constexpr bool PRE = PASS == 0;
     const int k0 = kt * BN;
 #pragma unroll
@@ -159,12 +162,11 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
         if (has_gk) gm = OP::mma(OP::cols(tgK, 32 * st + li, c), qf[c], gm);
         if (has_gv) w = OP::mma(OP::cols(tgV, 32 * st + li, c), dof[c], w);
       }
-      const bool need_mask = (k0s + 32 > s.M) || (CAUSAL && k0s + 31 > q0w);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         if constexpr (OWN) dpz[r] -= z;
         float pv = OWN ? own_prob(sc[r], c2, m2, l2) : fast_exp2(fmaf(sc[r], c2, -moff));
-        if (need_mask) {
+        if constexpr (MASK) {
           const int key = k0s + acc_row(r, g);
           if (key >= s.M || (CAUSAL && key > myq)) pv = 0.f;
         }
@@ -259,7 +261,7 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
     };
     // every key tile once, from tile 0 already prefetched
     auto sweep = [&](auto pass_tag) __attribute__((always_inline)) {
-      for (int kt = 0; kt < nkt; ++kt) {
+      auto step = [&](auto mask_tag, int kt) __attribute__((always_inline)) {
         __syncthreads();
         OP::store(gsK, sK0);
         OP::store(gsV, sV0);
@@ -267,8 +269,11 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
         if (has_gv) OP::store(gsgV, sgV0);
         __syncthreads();
         if (kt + 1 < nkt) prefetch((kt + 1) * BN);
-        compute(pass_tag, kt, sK0, sV0, sgK0, sgV0);
-      }
+        compute(pass_tag, mask_tag, kt, sK0, sV0, sgK0, sgV0);
+      };
+      int kt = 0;
+      for (; kt < nfull; ++kt) step(std::false_type{}, kt);
+      for (; kt < nkt; ++kt) step(std::true_type{}, kt);
     };
     if (nkt > 0) prefetch(0);
     if (exact) {
@@ -288,7 +293,7 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
         if (has_gk) OP::store(gsgK, sgK0);
         if (has_gv) OP::store(gsgV, sgV0);
         __syncthreads();
-        compute(pre_pass, 0, sK0, sV0, sgK0, sgV0);
+        compute(pre_pass, std::true_type{}, 0, sK0, sV0, sgK0, sgV0);
         set_centre();
       }
       sweep(full_pass);
@@ -366,7 +371,6 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
   const int key0 = kb * BN;
   const int kw0 = key0 + wave * 32;
   const int mykey = kw0 + li;
-  const bool kvalid = mykey < s.M;
 
   F kf[NKC], vf[NKC], gkf[NKC], gvf[NKC];
   {
@@ -426,9 +430,10 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
 
   // The query tile it held in (tQ, tO, tgQ) with its row terms in sr, as 32-query subtiles. SPLIT: Gbar_dP,
   // Gbar_S and dS enter the products as two 16-bit terms each.
-  auto tile = [&](auto split_tag, int it, const T* tQ, const T* tO, const T* tgQ,
+  auto tile = [&](auto split_tag, auto diag_tag, int it, const T* tQ, const T* tO, const T* tgQ,
                   const float* sr) __attribute__((always_inline)) {
     constexpr bool SPLIT = decltype(split_tag)::value;
+    constexpr bool DIAG = decltype(diag_tag)::value;  // causal: the tile starts before the block's last key
     const int q0 = qbeg + it * BM;
     if (CAUSAL && kw0 > q0 + BM - 1) return;
 #pragma unroll
@@ -459,15 +464,14 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
         if (has_gk) gm = OP::template mma<true>(qfr, gkf[c], gm);
         if (has_gv) w = OP::template mma<true>(ofr, gvf[c], w);
       }
-      const bool diag = CAUSAL && (kw0 + 31 > q0s);
       f32x16_t gdp, gs;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int qd = r >> 2, e = r & 3;
         if constexpr (OWN) dpz[r] -= z4[qd][e];
         float pv = OWN ? own_prob(sc[r], c2, l4[qd][e], lo4[qd][e]) : fast_exp2(fmaf(sc[r], c2, -l4[qd][e]));
-        if (!kvalid) pv = 0.f;
-        if (diag && mykey > q0s + acc_row(r, g)) pv = 0.f;
+        if constexpr (DIAG)  // (a key past the end needs no mask: its lane's results are not stored)
+          if (mykey > q0s + acc_row(r, g)) pv = 0.f;
         const float gam = s.scale * gm[r];
         const float ds = pv * dpz[r];
         const float e1 = fmaf(gam, dpz[r], w[r]);
@@ -516,12 +520,12 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
   const std::integral_constant<bool, true> with_split;
   const std::integral_constant<bool, false> no_split;
   bool pk_any = false;  // uniform: a tile holding a peaked row was skipped (16-bit)
-  auto compute = [&](int it, const T* tQ, const T* tO, const T* tgQ,
+  auto compute = [&](auto diag_tag, int it, const T* tQ, const T* tO, const T* tgQ,
                      const float* sr) __attribute__((always_inline)) {
     // uniform: every thread reads the same flag
     const bool pk = sizeof(T) == 2 && __builtin_amdgcn_readfirstlane(__float_as_uint(sr[FLAG])) != 0u;
     pk_any |= pk;  // run after the loop, so the loop's schedule holds only the one-term products
-    if (!pk) tile(no_split, it, tQ, tO, tgQ, sr);
+    if (!pk) tile(no_split, diag_tag, it, tQ, tO, tgQ, sr);
   };
   // The tiles holding a peaked row, found 64 at a time from the lse flags and run one after the other with
   // the split products, from stage(it) (loads tile it into sQ0, sdO0, sgQ0 and its row terms into sRow0).
@@ -548,7 +552,7 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
         if (!sPk[i]) continue;  // uniform: every thread reads the same flag
         stage(t0 + i);
         __syncthreads();
-        tile(with_split, t0 + i, sQ0, sdO0, sgQ0, sRow0);
+        tile(with_split, std::integral_constant<bool, CAUSAL>{}, t0 + i, sQ0, sdO0, sgQ0, sRow0);
         __syncthreads();  // the tile buffers are free again
       }
     }
@@ -564,7 +568,7 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
       load_rows(it);
     };
     if (nqt > 0) prefetch(0);
-    for (int it = 0; it < nqt; ++it) {
+    auto step = [&](auto diag_tag, int it) __attribute__((always_inline)) {
       __syncthreads();
       OP::store(gsQ, sQ0);
       OP::store(gsO, sdO0);
@@ -572,8 +576,12 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
       store_rows(sRow0);
       __syncthreads();
       if (it + 1 < nqt) prefetch(it + 1);
-      compute(it, sQ0, sdO0, sgQ0, sRow0);
-    }
+      compute(diag_tag, it, sQ0, sdO0, sgQ0, sRow0);
+    };
+    const int ndiag = CAUSAL ? min(nqt, (key0 + BN - 1 - qbeg + BM - 1) / BM) : 0;
+    int it = 0;
+    for (; it < ndiag; ++it) step(std::integral_constant<bool, CAUSAL>{}, it);
+    for (; it < nqt; ++it) step(std::false_type{}, it);
     if (pk_any)
       peaked_tiles([&](int it) __attribute__((always_inline)) {
         prefetch(it);

@@ -82,8 +82,8 @@ template <> struct Mfma<float> {
 // and |l| <= 2^-18 |x|), and a b is summed as the six products down to 2^-18: the three dropped ones (m l, l m,
 // l l) are below 2^-26 of it, under float32's own rounding. One 16-wide k chunk then takes 6 x 32 cycles of the
 // matrix pipe where eight v_mfma_f32_32x32x2_f32 take 8 x 64, and rounds the accumulator fewer times.
-// Measured against the native float32 products: forward + backward of B2 H16 T1000 D64 460 -> 310 us, the HVP of
-// B8 H8 T512 D64 783 -> 554 us; relative error against float64 7.4e-7 -> 6.4e-7 and 7.4e-7 -> 6.3e-7, and not
+// Measured against the native float32 products: forward + backward of B2 H16 T1000 D64 460 -> 297 us, the HVP of
+// B8 H8 T512 D64 783 -> 524 us; relative error against float64 7.4e-7 -> 6.4e-7 and 7.4e-7 -> 6.3e-7, and not
 // larger in any of 25 float32 calls over B 1..468, T and M 6..3638, D 16..128.
 struct X3Frag {
   bf16x8_t h, m, l;
@@ -445,18 +445,31 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 // largest (a finite float32 there would round to infinity) take that value as their first term; an infinity then
 // ends up in l, which only meets the other operand's h, so that products with it stay infinite (NaN against 0)
 // as in float32, and a NaN reaches l the same way.
+// Two elements at a time, so that one v_cvt_pk_bf16_f32 rounds both and the rounded values are read back from its result
+// (element by element the compiler converts each value a second time for the residual: 56 conversions instead of 24 for
+// 16 elements).
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+template <bool CLAMP>
+__device__ __forceinline__ void split3_pair(float x0, float x1, bf16x2_t& h, bf16x2_t& m, bf16x2_t& l) {
+  constexpr float kBig = 3.3895313892515355e38f;  // the largest finite bfloat16
+  auto big = [](float x) { return CLAMP ? __builtin_amdgcn_fmed3f(x, -kBig, kBig) : x; };
+  auto lo = [](bf16x2_t p) { return __uint_as_float(__builtin_bit_cast(uint32_t, p) << 16); };
+  auto hi = [](bf16x2_t p) { return __uint_as_float(__builtin_bit_cast(uint32_t, p) & 0xffff0000u); };
+  h = __builtin_convertvector((f32x2_t{big(x0), big(x1)}), bf16x2_t);
+  const float r0 = x0 - lo(h), r1 = x1 - hi(h);
+  m = __builtin_convertvector((f32x2_t{big(r0), big(r1)}), bf16x2_t);
+  l = __builtin_convertvector((f32x2_t{r0 - lo(m), r1 - hi(m)}), bf16x2_t);
+}
 template <bool CLAMP>
 __device__ __forceinline__ X3Frag split3(const float (&x)[8]) {
-  constexpr float kBig = 3.3895313892515355e38f;  // the largest finite bfloat16
   X3Frag f;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float xh = CLAMP ? __builtin_amdgcn_fmed3f(x[e], -kBig, kBig) : x[e];
-    f.h[e] = (__bf16)xh;
-    const float r1 = x[e] - (float)f.h[e];
-    const float xm = CLAMP ? __builtin_amdgcn_fmed3f(r1, -kBig, kBig) : r1;
-    f.m[e] = (__bf16)xm;
-    f.l[e] = (__bf16)(r1 - (float)f.m[e]);
+  for (int e = 0; e < 8; e += 2) {
+    bf16x2_t h, m, l;
+    split3_pair<CLAMP>(x[e], x[e + 1], h, m, l);
+    f.h[e] = h[0], f.h[e + 1] = h[1];
+    f.m[e] = m[0], f.m[e + 1] = m[1];
+    f.l[e] = l[0], f.l[e + 1] = l[1];
   }
   return f;
 }
@@ -556,7 +569,6 @@ struct Ops<float, DP, true> {
   template <int ROWS, int NT>
   __device__ __forceinline__ static void store(const TileStage<float, ROWS, DP, NT>& st, float* lds) {
     using S = TileStage<float, ROWS, DP, NT>;
-    constexpr float kBig = 3.3895313892515355e38f;
 #pragma unroll
     for (int i = 0; i < S::PER; ++i) {
       const int ch = (int)threadIdx.x + i * NT;
@@ -565,11 +577,12 @@ struct Ops<float, DP, true> {
         const f32x4_t x = __builtin_bit_cast(f32x4_t, st.r[i]);
         bf16x4_t h, m, l;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {  // as split3<true>
-          h[e] = (__bf16)__builtin_amdgcn_fmed3f(x[e], -kBig, kBig);
-          const float r1 = x[e] - (float)h[e];
-          m[e] = (__bf16)__builtin_amdgcn_fmed3f(r1, -kBig, kBig);
-          l[e] = (__bf16)(r1 - (float)m[e]);
+        for (int e = 0; e < 4; e += 2) {
+          bf16x2_t h2, m2, l2;
+          split3_pair<true>(x[e], x[e + 1], h2, m2, l2);
+          h[e] = h2[0], h[e + 1] = h2[1];
+          m[e] = m2[0], m[e + 1] = m2[1];
+          l[e] = l2[0], l[e + 1] = l2[1];
         }
         char* p = reinterpret_cast<char*>(lds + row * PITCH) + 2 * col;
         *reinterpret_cast<i16x4_t*>(p) = __builtin_bit_cast(i16x4_t, h);

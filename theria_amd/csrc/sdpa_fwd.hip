@@ -86,7 +86,10 @@ __global__ __launch_bounds__(64 * NW, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel
     stK.load_any(K, p.k.sr, 0, M, s.D, s.vec);
     stV.load_any(V, p.v.sr, 0, M, s.D, s.vec);
   }
-  for (int kt = 0; kt < nkt; ++kt) {
+  // MASK: the tile reaches past the last key or (causal) past the block's first query; those tiles take their own copy of
+  // the loop (a mask behind a uniform branch becomes a compare and a select per score in every tile).
+  auto step = [&](auto mask_tag, int kt) __attribute__((always_inline)) {
+    constexpr bool MASK = decltype(mask_tag)::value;
     const int k0 = kt * BN;
     __syncthreads();
     OP::store(stK, sK);
@@ -96,7 +99,7 @@ __global__ __launch_bounds__(64 * NW, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel
       stK.load_any(K, p.k.sr, k0 + BN, M, s.D, s.vec);
       stV.load_any(V, p.v.sr, k0 + BN, M, s.D, s.vec);
     }
-    if (CAUSAL && k0 > q0w + 32 * QT - 1) continue;  // tile entirely above this wave's diagonal
+    if (CAUSAL && k0 > q0w + 32 * QT - 1) return;  // tile entirely above this wave's diagonal
 
     f32x16_t sc[QT][NST];
 #pragma unroll
@@ -110,9 +113,8 @@ __global__ __launch_bounds__(64 * NW, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel
         for (int j = 0; j < QT; ++j) sc[j][t] = OP::mma(kfr, qf[j][c], sc[j][t]);
       }
     }
-    // Boundary tiles only (a uniform branch): masked scores become -inf, so P = 0 there. Interior
-    // tiles run the same code below with no per-element test.
-    if ((k0 + BN > M) || (CAUSAL && k0 + BN - 1 > q0w)) {
+    // masked scores become -inf, so P = 0 there
+    if (MASK && ((k0 + BN > M) || (CAUSAL && k0 + BN - 1 > q0w))) {
 #pragma unroll
       for (int j = 0; j < QT; ++j) {
         const int lim = CAUSAL ? min(M, q0w + 32 * j + li + 1) : M;  // first key this query cannot see
@@ -171,7 +173,14 @@ __global__ __launch_bounds__(64 * NW, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel
           for (int j = 0; j < QT; ++j) o[j][dt] = OP::mma(vfr, pf[j], o[j][dt]);
         }
       }
-  }
+  };
+  // Tiles with every key in range and visible to the block. Two copies of the loop pay in float32 only (16-bit D20 T1000
+  // 26.0 -> 27.0 us), and not in its two-wave workgroups above head dim 32, which spill.
+  constexpr bool PEEL = sizeof(T) == 4 && (NW == 4 || DP == 32);
+  const int nfull = PEEL ? (CAUSAL ? min(M / BN, qb * BM / BN) : M / BN) : 0;
+  int kt = 0;
+  for (; kt < min(nfull, nkt); ++kt) step(std::false_type{}, kt);
+  for (; kt < nkt; ++kt) step(std::true_type{}, kt);
 
 #pragma unroll
   for (int j = 0; j < QT; ++j) {

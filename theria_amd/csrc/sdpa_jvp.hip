@@ -35,7 +35,7 @@ namespace theria {
 
 // Tiles pass through registers into padded LDS rows. NW: waves per workgroup, four or two (at most 64 queries).
 template <typename T, int DP, bool CAUSAL, bool HAS_O, int NW = 4>
-__global__ __launch_bounds__(64 * NW) void jvp_kernel(const JvpParams p) {
+__global__ __launch_bounds__(64 * NW, sizeof(T) == 4 && DP == 32 ? 2 : 1) void jvp_kernel(const JvpParams p) {
   using OP = Ops<T, DP, (sizeof(T) == 4 && DP <= 64)>;
   using F = typename OP::F;
   constexpr int KC = OP::KC;
@@ -97,7 +97,8 @@ __global__ __launch_bounds__(64 * NW) void jvp_kernel(const JvpParams p) {
   if (CAUSAL) kend = min(s.M, qb * BM + BM);
   const int nkt = (kend + BN - 1) / BN;
   // The key tile kt held in (tK, tV, ttK, ttV).
-  auto compute = [&](int kt, const T* tK, const T* tV, const T* ttK, const T* ttV) {
+  auto compute = [&](auto mask_tag, int kt, const T* tK, const T* tV, const T* ttK, const T* ttV) __attribute__((always_inline)) {
+    constexpr bool MASK = decltype(mask_tag)::value;
     const int k0 = kt * BN;
     if (CAUSAL && k0 > q0w + 31) return;
 
@@ -114,13 +115,12 @@ __global__ __launch_bounds__(64 * NW) void jvp_kernel(const JvpParams p) {
         if (has_tk) gm[t] = OP::mma(OP::cols(ttK, t * 32 + li, c), qf[c], gm[t]);
       }
     }
-    const bool need_mask = (k0 + BN > s.M) || (CAUSAL && k0 + BN - 1 > q0w);
 #pragma unroll
     for (int t = 0; t < NST; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         float pv = fast_exp2(fmaf(sc[t][r], c2, -moff));
-        if (need_mask) {
+        if constexpr (MASK) {
           const int key = k0 + t * 32 + acc_row(r, g);
           if (key >= s.M || (CAUSAL && key > myq)) pv = 0.f;
         }
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(64 * NW) void jvp_kernel(const JvpParams p) {
       if (has_tv) gtV.load(TV, p.tv.sr, k0, s.M, s.D, s.vec);
     };
     if (nkt > 0) prefetch(0);
-    for (int kt = 0; kt < nkt; ++kt) {
+    auto step = [&](auto mask_tag, int kt) __attribute__((always_inline)) {
       __syncthreads();
       OP::store(gK, sK0);
       OP::store(gV, sV0);
@@ -171,8 +171,13 @@ __global__ __launch_bounds__(64 * NW) void jvp_kernel(const JvpParams p) {
       if (has_tv) OP::store(gtV, stV0);
       __syncthreads();
       if (kt + 1 < nkt) prefetch((kt + 1) * BN);
-      compute(kt, sK0, sV0, stK0, stV0);
-    }
+      compute(mask_tag, kt, sK0, sV0, stK0, stV0);
+    };
+    // the tiles with every key in range and visible to the block, then the others with the mask
+    const int nfull = min(nkt, CAUSAL ? min(s.M / BN, qb * BM / BN) : s.M / BN);
+    int kt = 0;
+    for (; kt < nfull; ++kt) step(std::false_type{}, kt);
+    for (; kt < nkt; ++kt) step(std::true_type{}, kt);
   }
 
   // normalize: P / L with L = sum_j P_j, i.e. every term below is divided by L (and a rebuilt O as well)
@@ -531,10 +536,12 @@ struct JvpLauncher {
       }
     }
     // at most 64 queries, and more workgroups than CUs (one four-wave workgroup per CU is resident): float32 B400 H4
-    // T64 D16 42 -> 34 us
-    if (p.s.T <= 64 && nblk > device_cu_count()) {
-      hipLaunchKernelGGL((jvp_kernel<T, DP, CAUSAL, HAS_O, 2>), dim3((unsigned)nblk), dim3(128), 0, st, p);
-      return hipGetLastError();
+    // T64 D16 42 -> 33 us. Not in float32 above head dim 64, where staging a tile with half the threads spills.
+    if constexpr (!(sizeof(T) == 4 && DP == 128)) {
+      if (p.s.T <= 64 && nblk > device_cu_count()) {
+        hipLaunchKernelGGL((jvp_kernel<T, DP, CAUSAL, HAS_O, 2>), dim3((unsigned)nblk), dim3(128), 0, st, p);
+        return hipGetLastError();
+      }
     }
     hipLaunchKernelGGL((jvp_kernel<T, DP, CAUSAL, HAS_O>), dim3((unsigned)nblk), dim3(256), 0, st, p);
     return hipGetLastError();
