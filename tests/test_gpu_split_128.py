@@ -54,3 +54,21 @@ def test_large_heads_on_strided_views(D, hip_device):
         got.append([_ops.jvp(*ts[:3], o, lse, *ts[4:], D**-0.5, True),
                     *_ops.bwd_bwd(*ts[:3], o, ts[3], lse, None, *ts[4:], D**-0.5, True)])
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("D", [96, 128])
+@pytest.mark.parametrize("T", [130, 600])
+def test_causal_dq_of_small_and_large_grids(T, D, hip_device):
+    """A causal grid of at most one workgroup per CU takes the peaked and common query blocks in one launch, a larger one
+    in two: the same head gives the same gradients bit for bit alone and as one of 160."""
+    print(f"[causal dq grids] T{T} D{D}", flush=True)
+    g = torch.Generator(device=hip_device).manual_seed(T + D)
+    q, k, v, do = (torch.randn(1, 1, T, D, generator=g, device=hip_device).to(BF16) for _ in range(4))
+    one = [q, k, v, do]
+    many = [t.expand(1, 160, T, D) for t in one]
+    got = []
+    for ts in (one, many):
+        o, lse = _ops.fwd(*ts[:3], D**-0.5, True)[:2]
+        got.append(_ops.bwd(*ts[:3], o, lse, ts[3], D**-0.5, True))
+    for a, b in zip(*got):
+        assert torch.equal(a[0, 0], b[0, 0]) and torch.equal(a[0, 0], b[0, 159])

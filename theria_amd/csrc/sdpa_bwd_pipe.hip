@@ -793,13 +793,23 @@ __global__ __launch_bounds__(64 * NW, WPS) void dq_pipe_kernel(const DqParams p)
 }
 
 // Launches with FD = (head dim == DP): one fused launch at head dim 64; at 128 the common launch (unless every
-// block takes the row-term pass), then the peaked launch.
+// block takes the row-term pass), then the peaked launch, or one fused launch on small causal grids.
 template <typename T, bool CAUSAL, int NW, int DP, bool OVERLAP, int WPS, int HALVES, bool FD>
 static void dq_go_fd(const DqParams& p, int64_t nblk, hipStream_t st) {
   if constexpr (DP <= 64) {
     hipLaunchKernelGGL((dq_pipe_kernel<T, CAUSAL, NW, DP, OVERLAP, WPS, HALVES, FD, 2>), dim3((unsigned)nblk),
                        dim3(64 * NW), 0, st, p);
   } else {
+    // Causal (every head's first rows are peaked) with at most one workgroup per CU: one launch, in which the peaked blocks
+    // run beside the common ones (backward, us: B2 H8 T1024 D128 122.9 -> 94.9, B1 H4 T2048 D128 168 -> 146). Without the
+    // mask the two launches stay (B2 H8 T1024 69.9 -> 71.4 in one).
+    if constexpr (CAUSAL) {
+      if (p.row_term < kRowFrozen && nblk <= device_cu_count()) {
+        hipLaunchKernelGGL((dq_pipe_kernel<T, CAUSAL, NW, DP, OVERLAP, WPS, HALVES, FD, 2>), dim3((unsigned)nblk),
+                           dim3(64 * NW), 0, st, p);
+        return;
+      }
+    }
     if (p.row_term < kRowFrozen)
       hipLaunchKernelGGL((dq_pipe_kernel<T, CAUSAL, NW, DP, OVERLAP, WPS, HALVES, FD, 0>), dim3((unsigned)nblk),
                          dim3(64 * NW), 0, st, p);
