@@ -76,8 +76,8 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
   int kend = s.M;
   if (CAUSAL) kend = min(s.M, qb * BM + BM);
   const int nkt = (kend + BN - 1) / BN;
-  // tiles that need no mask (their own copy of the loops; at float32 head dim 128, whose loop spills, only one copy)
-  const int nfull = sizeof(T) == 4 && DP == 128 ? 0 : min(nkt, CAUSAL ? min(s.M / BN, qb * BM / BN) : s.M / BN);
+  // tiles that need no mask (their own copy of the loops)
+  const int nfull = min(nkt, CAUSAL ? min(s.M / BN, qb * BM / BN) : s.M / BN);
   // 16-bit workgroups holding a row flagged peaked in lse take the exact form (uniform). Causal ones with at
   // most half the longest workgroup's key tiles run both of its passes in the first launch, inside that
   // launch's slack (every head's first query block holds such rows); the others are the second pass's.
@@ -87,7 +87,11 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
   bool flagged = false;
   if (EXACT || (LIGHT_OK && light)) flagged = __syncthreads_or(qvalid && lse_peaked(p.lse[row_id]));
   const bool exact = EXACT && flagged && !light;
-  const bool two_pass = !EXACT && LIGHT_OK && flagged && light;
+  // float32 at head dim 128 always takes the two passes: the one-pass form's four 128-wide accumulators and three operand
+  // sets spilled ~700 registers, the exact form's passes hold two (~100). Double backward with the column pass's reuse
+  // below, us: B4 H8 T700 D128 3560 -> 2694, B16 H16 T300 D128 causal 4248 -> 3254, B2 H16 T1000 D64 645 -> 627.
+  constexpr bool TWO = sizeof(T) == 4 && DP == 128;
+  const bool two_pass = TWO || (!EXACT && LIGHT_OK && flagged && light);
   if (EXACT && !exact) return;
 
   F qf[NKC], dof[NKC], gqf[NKC];
@@ -191,6 +195,18 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
         }
       }
       if constexpr (PRE) continue;
+      if constexpr (PASS == 3 && sizeof(T) == 4) {
+#pragma unroll
+        for (int cc = 0; cc < NPC; ++cc) {
+          const F gf = OP::acc(gm, cc), df = OP::acc(dpz, cc);
+#pragma unroll
+          for (int dt = 0; dt < NDT; ++dt) {
+            x13[dt] = OP::mma(OP::rows(tK, 32 * st, cc, dt * 32), gf, x13[dt]);
+            if (has_gk) yk[dt] = OP::mma(OP::rows(tgK, 32 * st, cc, dt * 32), df, yk[dt]);
+          }
+        }
+        continue;
+      }
       if constexpr (PASS == 3 && sizeof(T) == 2) {
 #pragma unroll
         for (int cc = 0; cc < NPC; ++cc) {
@@ -296,7 +312,7 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
         compute(pre_pass, std::true_type{}, 0, sK0, sV0, sgK0, sgV0);
         set_centre();
       }
-      sweep(full_pass);
+      if constexpr (!TWO) sweep(full_pass);
     }
   }
 
@@ -442,17 +458,11 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
       if (CAUSAL && kw0 > q0s + 31) continue;
 
       f32x16_t sc = zero16(), gm = zero16(), w = zero16(), dpz;
-      f32x4_t l4[4], z4[4], r4[4], t4[4], lo4[4];
 #pragma unroll
       for (int qd = 0; qd < 4; ++qd) {
-        const int o = 32 * sq + 8 * qd + 4 * g;
-        l4[qd] = *reinterpret_cast<const f32x4_t*>(sr + o);
-        z4[qd] = *reinterpret_cast<const f32x4_t*>(sr + BM + o);
-        r4[qd] = *reinterpret_cast<const f32x4_t*>(sr + 2 * BM + o);
-        t4[qd] = *reinterpret_cast<const f32x4_t*>(sr + 3 * BM + o);
-        if constexpr (OWN) lo4[qd] = *reinterpret_cast<const f32x4_t*>(sr + 4 * BM + o);
+        const f32x4_t z4 = *reinterpret_cast<const f32x4_t*>(sr + BM + 32 * sq + 8 * qd + 4 * g);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) dpz[4 * qd + e] = OWN ? 0.f : -z4[qd][e];
+        for (int e = 0; e < 4; ++e) dpz[4 * qd + e] = OWN ? 0.f : -z4[e];
       }
 #pragma unroll
       for (int c = 0; c < NKC; ++c) {
@@ -464,27 +474,40 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
         if (has_gk) gm = OP::template mma<true>(qfr, gkf[c], gm);
         if (has_gv) w = OP::template mma<true>(ofr, gvf[c], w);
       }
-      f32x16_t gdp, gs;
+      // the row terms are read here, four rows at a time, and the results take their operands' registers: gm <- Gbar_dP,
+      // w <- Gbar_S, dpz <- dS
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int qd = r >> 2, e = r & 3;
-        if constexpr (OWN) dpz[r] -= z4[qd][e];
-        float pv = OWN ? own_prob(sc[r], c2, l4[qd][e], lo4[qd][e]) : fast_exp2(fmaf(sc[r], c2, -l4[qd][e]));
-        if constexpr (DIAG)  // (a key past the end needs no mask: its lane's results are not stored)
-          if (mykey > q0s + acc_row(r, g)) pv = 0.f;
-        const float gam = s.scale * gm[r];
-        const float ds = pv * dpz[r];
-        const float e1 = fmaf(gam, dpz[r], w[r]);
-        gdp[r] = pv * (gam - r4[qd][e]);
-        gs[r] = pv * e1 - r4[qd][e] * ds - t4[qd][e] * pv;
-        dpz[r] = ds;
+      for (int qd = 0; qd < 4; ++qd) {
+        const int o = 32 * sq + 8 * qd + 4 * g;
+        const f32x4_t l4 = *reinterpret_cast<const f32x4_t*>(sr + o);
+        const f32x4_t r4 = *reinterpret_cast<const f32x4_t*>(sr + 2 * BM + o);
+        const f32x4_t t4 = *reinterpret_cast<const f32x4_t*>(sr + 3 * BM + o);
+        f32x4_t z4{}, lo4{};
+        if constexpr (OWN) {
+          z4 = *reinterpret_cast<const f32x4_t*>(sr + BM + o);
+          lo4 = *reinterpret_cast<const f32x4_t*>(sr + 4 * BM + o);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = 4 * qd + e;
+          if constexpr (OWN) dpz[r] -= z4[e];
+          float pv = OWN ? own_prob(sc[r], c2, l4[e], lo4[e]) : fast_exp2(fmaf(sc[r], c2, -l4[e]));
+          if constexpr (DIAG)  // (a key past the end needs no mask: its lane's results are not stored)
+            if (mykey > q0s + acc_row(r, g)) pv = 0.f;
+          const float gam = s.scale * gm[r];
+          const float ds = pv * dpz[r];
+          const float e1 = fmaf(gam, dpz[r], w[r]);
+          gm[r] = pv * (gam - r4[e]);
+          w[r] = pv * e1 - r4[e] * ds - t4[e] * pv;
+          dpz[r] = ds;
+        }
       }
       if constexpr (SPLIT && sizeof(T) == 2) {
 #pragma unroll
         for (int cc = 0; cc < NPC; ++cc) {
           F gdph, gdpl, gsh, gsl, dsh, dsl;
-          split_frag<T>(gdp, cc, gdph, gdpl);
-          split_frag<T>(gs, cc, gsh, gsl);
+          split_frag<T>(gm, cc, gdph, gdpl);
+          split_frag<T>(w, cc, gsh, gsl);
           split_frag<T>(dpz, cc, dsh, dsl);
 #pragma unroll
           for (int dt = 0; dt < NDT; ++dt) {
@@ -504,8 +527,8 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
       } else {
 #pragma unroll
         for (int cc = 0; cc < NPC; ++cc) {
-          const F gdpf = OP::acc(gdp, cc);
-          const F gsf = OP::acc(gs, cc);
+          const F gdpf = OP::acc(gm, cc);
+          const F gsf = OP::acc(w, cc);
           const F dsf = OP::acc(dpz, cc);
 #pragma unroll
           for (int dt = 0; dt < NDT; ++dt) {
