@@ -53,3 +53,29 @@ def test_largest_values_and_infinities(D):
     cols = [d for d in range(D) if d not in (2, 4)]
     torch.testing.assert_close(o[..., cols].double(), ref[..., cols], rtol=1e-5, atol=1e-5)
     torch.testing.assert_close(o[..., 2].double(), ref[..., 2], rtol=1e-4, atol=0.0)  # P of one key, scaled by 3.4e38
+
+
+@pytest.mark.parametrize("D", [64, 80, 128])
+@pytest.mark.parametrize("T,M,causal", [(20, 90, False), (130, 130, True)])
+def test_jvp_rounds_as_the_forward(T, M, causal, D, hip_device):
+    """Scores of up to ~20: lse and the JVP's scores round alike, so the tangent is no worse than PyTorch's float32
+    formula with its own softmax (bar: 1.5 times its error against float64; the kernel measured ~0.9 times, and 1.4 times
+    lse's rounding more when its scores were rounded in another order)."""
+    print(f"float32 split jvp T{T} M{M} D{D} causal={causal}", flush=True)
+    g = torch.Generator().manual_seed(D + T)
+    q, tq = (torch.randn(2, 4, T, D, generator=g) * s for s in (2.0, 1.0))
+    k, tk, v, tv = (torch.randn(2, 4, M, D, generator=g) * s for s in (2.0, 1.0, 1.0, 1.0))
+    mask = torch.ones(T, M, dtype=torch.bool).triu(1) if causal else torch.zeros(T, M, dtype=torch.bool)
+
+    def plain(dt):
+        a, b, c, ta, tb, tc = (t.to(dt) for t in (q, k, v, tq, tk, tv))
+        p = torch.softmax((a @ b.mT * D**-0.5).masked_fill(mask, -float("inf")), -1)
+        ds = p * ((ta @ b.mT + a @ tb.mT) * D**-0.5)
+        return (ds - p * ds.sum(-1, keepdim=True)) @ c + p @ tc
+
+    dev = [t.to(hip_device) for t in (q, k, v, tq, tk, tv)]
+    o, lse = _ops.fwd(*dev[:3], D**-0.5, causal)[:2]
+    got = _ops.jvp(*dev[:3], o, lse, *dev[3:], D**-0.5, causal).cpu()
+    ref = plain(torch.float64)
+    err, bar = (float((t.double() - ref).norm() / ref.norm()) for t in (got, plain(torch.float32)))
+    assert err <= 1.5 * bar, (err, bar)

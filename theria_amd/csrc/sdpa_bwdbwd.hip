@@ -43,7 +43,7 @@ namespace theria {
 // registers and schedule.
 template <typename T, int DP, bool CAUSAL, bool EXACT>
 __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdParams& p, const int blk, const int nblk) {
-  using OP = Ops<T, DP, (sizeof(T) == 4 && DP <= 64)>;
+  using OP = Ops<T, DP, sizeof(T) == 4>;
   using F = typename OP::F;
   constexpr int KC = OP::KC;
   constexpr int NW = 4, BM = 32 * NW, NT = 64 * NW;
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(256) void bwdbwd_rows_kernel(const BwdBwdParams p) 
 // Q, dO, gQ tiles staged as in the rows kernel, the row terms beside them.
 template <typename T, int DP, bool CAUSAL>
 __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdParams& p, const int blk, const int nblk) {
-  using OP = Ops<T, DP, (sizeof(T) == 4 && DP <= 64)>;
+  using OP = Ops<T, DP, sizeof(T) == 4>;
   using F = typename OP::F;
   constexpr int KC = OP::KC;
   constexpr int NW = 4, BN = 32 * NW, NT = 64 * NW;
