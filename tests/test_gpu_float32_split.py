@@ -79,3 +79,17 @@ def test_jvp_rounds_as_the_forward(T, M, causal, D, hip_device):
     ref = plain(torch.float64)
     err, bar = (float((t.double() - ref).norm() / ref.norm()) for t in (got, plain(torch.float32)))
     assert err <= 1.5 * bar, (err, bar)
+
+
+@pytest.mark.parametrize("D", [72, 96, 128])
+@pytest.mark.parametrize("T,M,causal", [(100, 1, False), (100, 100, True)])
+def test_one_visible_key_gives_no_curvature(T, M, causal, D, hip_device):
+    """A row that sees one key has P = 1 whatever its scores: its G_Q is 0 exactly where the row statistics, the row
+    kernel and the column kernel form S and dP by the same products, in the same order of rounding."""
+    print(f"float32 split one key T{T} M{M} D{D} causal={causal}", flush=True)
+    g = torch.Generator(device=hip_device).manual_seed(D + M)
+    q, do, tq = (torch.randn(1, 2, T, D, generator=g, device=hip_device) for _ in range(3))
+    k, v, tk, tv = (torch.randn(1, 2, M, D, generator=g, device=hip_device) for _ in range(4))
+    o, lse = _ops.fwd(q, k, v, D**-0.5, causal)[:2]
+    gq = _ops.bwd_bwd(q, k, v, o, do, lse, None, tq, tk, tv, D**-0.5, causal)[0]
+    assert (gq[:, :, 0 if causal else slice(None)] == 0).all()

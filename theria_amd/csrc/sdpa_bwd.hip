@@ -43,10 +43,9 @@
 
 namespace theria {
 
-// X3: float32 products by three-term bfloat16 splits (MfmaX3).
-template <typename T, int DP, bool CAUSAL, int QT, bool X3>
+template <typename T, int DP, bool CAUSAL, int QT>
 __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const DqParams p) {
-  using OP = Ops<T, DP, X3>;
+  using OP = Ops<T, DP>;
   using F = typename OP::F;
   constexpr int KC = OP::KC;
   constexpr int NW = 4, BM = 32 * NW * QT, BN = 32, NT = 64 * NW;
@@ -359,7 +358,7 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
 
 template <typename T, int DP, bool CAUSAL, int KT, bool DV_ONLY>
 __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(const DkdvParams p) {
-  using OP = Ops<T, DP, sizeof(T) == 4>;
+  using OP = Ops<T, DP>;
   using F = typename OP::F;
   constexpr int KC = OP::KC;
   constexpr int NW = 4, BN = 32 * NW * KT, NT = 64 * NW;
@@ -613,20 +612,11 @@ struct DqLauncher {
     if (nblk == 0) return hipSuccess;
     if constexpr (DP <= 64 && sizeof(T) == 2) {
       if (qt == 2) {
-        hipLaunchKernelGGL((dq_kernel<T, DP, CAUSAL, 2, false>), dim3((unsigned)nblk), dim3(256), 0, st, p);
+        hipLaunchKernelGGL((dq_kernel<T, DP, CAUSAL, 2>), dim3((unsigned)nblk), dim3(256), 0, st, p);
         return hipGetLastError();
       }
     }
-    // The row statistics of the double backward must come from the same products as its row and column kernels
-    // form (kRowOwnStats): native float32 ones at head dim 128, where the split fragments would not fit theirs.
-    if constexpr (sizeof(T) == 4) {
-      if (!(DP == 128 && p.row_term == kRowOwnStats)) {
-        hipLaunchKernelGGL((dq_kernel<T, DP, CAUSAL, 1, true>), dim3((unsigned)nblk), dim3(256), 0, st, p);
-        return hipGetLastError();
-      }
-    }
-    if constexpr (sizeof(T) == 2 || DP == 128)
-      hipLaunchKernelGGL((dq_kernel<T, DP, CAUSAL, 1, false>), dim3((unsigned)nblk), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((dq_kernel<T, DP, CAUSAL, 1>), dim3((unsigned)nblk), dim3(256), 0, st, p);
     return hipGetLastError();
   }
 };

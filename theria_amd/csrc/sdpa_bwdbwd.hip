@@ -43,7 +43,7 @@ namespace theria {
 // registers and schedule.
 template <typename T, int DP, bool CAUSAL, bool EXACT>
 __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdParams& p, const int blk, const int nblk) {
-  using OP = Ops<T, DP, sizeof(T) == 4>;
+  using OP = Ops<T, DP>;
   using F = typename OP::F;
   constexpr int KC = OP::KC;
   constexpr int NW = 4, BM = 32 * NW, NT = 64 * NW;
@@ -88,8 +88,11 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
   if (EXACT || (LIGHT_OK && light)) flagged = __syncthreads_or(qvalid && lse_peaked(p.lse[row_id]));
   const bool exact = EXACT && flagged && !light;
   // float32 at head dim 128 always takes the two passes: the one-pass form's four 128-wide accumulators and three operand
-  // sets spilled ~700 registers, the exact form's passes hold two (~100). Double backward with the column pass's reuse
-  // below, us: B4 H8 T700 D128 3560 -> 2694, B16 H16 T300 D128 causal 4248 -> 3254, B2 H16 T1000 D64 645 -> 627.
+  // sets spilled ~700 registers, the exact form's passes hold two. The split products spill more than v_mfma_f32_32x32x2_f32
+  // did (rows ~105 -> ~220 of 512 registers, columns ~200 -> ~330) and are faster all the same. HVP of <W, O>, us, the
+  // one-pass form with v_mfma_f32_32x32x2_f32 -> two passes with it -> two passes with split products: B4 H8 T700 D128
+  // 3713 -> 2593 -> 1790, B2 H16 T1000 D80 5333 -> 4027 -> 2635, causal 4584 -> 3099 -> 2249, B16 H16 T300 D128 causal
+  // 4573 -> 3301 -> 2202.
   constexpr bool TWO = sizeof(T) == 4 && DP == 128;
   const bool two_pass = TWO || (!EXACT && LIGHT_OK && flagged && light);
   if (EXACT && !exact) return;
@@ -142,7 +145,7 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
 
   // The key tile kt held in (tK, tV, tgK, tgV), as 32-key subtiles.
   // PASS: 0 the pre-pass (sums only: for the centres over the first tile, or for r and t over every tile),
-  // 1 the common pass, 3 the exact pass (Gbar_S from exact row terms r, t; 16-bit only).
+  // 1 the common pass, 3 the exact pass (Gbar_S from exact row terms r, t: 16-bit, and float32 at DP = 128).
   auto compute = [&](auto pass_tag, auto mask_tag, int kt, const T* tK, const T* tV, const T* tgK,
                      const T* tgV) __attribute__((always_inline)) {
     constexpr int PASS = decltype(pass_tag)::value;
@@ -351,7 +354,7 @@ __global__ __launch_bounds__(256) void bwdbwd_rows_kernel(const BwdBwdParams p) 
 // Q, dO, gQ tiles staged as in the rows kernel, the row terms beside them.
 template <typename T, int DP, bool CAUSAL>
 __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdParams& p, const int blk, const int nblk) {
-  using OP = Ops<T, DP, sizeof(T) == 4>;
+  using OP = Ops<T, DP>;
   using F = typename OP::F;
   constexpr int KC = OP::KC;
   constexpr int NW = 4, BN = 32 * NW, NT = 64 * NW;

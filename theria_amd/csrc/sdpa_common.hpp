@@ -2,9 +2,9 @@
 //
 // Tiling vocabulary used by every kernel:
 //  * All matrix products use 32x32 MFMA output tiles. For 16-bit inputs the instruction is
-//    v_mfma_f32_32x32x16_{bf16,f16} (k extent 16, 8 elements per lane); for float32 inputs it is either
-//    v_mfma_f32_32x32x2_f32 (k extent 2, 1 element per lane) or six v_mfma_f32_32x32x16_bf16 over operands split
-//    into three bfloat16 terms (MfmaX3 below). Accumulation is float32 in all.
+//    v_mfma_f32_32x32x16_{bf16,f16} (k extent 16, 8 elements per lane); float32 inputs take six
+//    v_mfma_f32_32x32x16_bf16 over operands split into three bfloat16 terms (MfmaX3 below). Accumulation is float32
+//    in all.
 //  * Operand fragment of lane l (li = l % 32, g = l / 32): the row (A) or column (B) index is li, and
 //    the k elements depend on g. Output ("accumulator") layout: register r of lane l holds the element
 //    at row acc_row(r, g) = 8*(r/4) + 4*g + r%4 and column li. These layouts were checked bit-exactly
@@ -68,23 +68,18 @@ template <> struct Mfma<_Float16> {
   }
 };
 
-template <> struct Mfma<float> {
-  using frag_t = float;
-  static constexpr int KC = 2;
-  static constexpr int EPL = 1;
-  __device__ __forceinline__ static f32x16_t mma(frag_t a, frag_t b, f32x16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-  }
-};
-
 // float32 products on the bfloat16 matrix pipe. Each operand is split into three bfloat16 terms, h = bf16(x),
 // m = bf16(x - h), l = bf16(x - h - m), which hold all 24 bits of it (rounding to nearest leaves |m| <= 2^-9 |x|
 // and |l| <= 2^-18 |x|), and a b is summed as the six products down to 2^-18: the three dropped ones (m l, l m,
 // l l) are below 2^-26 of it, under float32's own rounding. One 16-wide k chunk then takes 6 x 32 cycles of the
 // matrix pipe where eight v_mfma_f32_32x32x2_f32 take 8 x 64, and rounds the accumulator fewer times.
-// Measured against the native float32 products: forward + backward of B2 H16 T1000 D64 460 -> 297 us, the HVP of
-// B8 H8 T512 D64 783 -> 524 us; relative error against float64 7.4e-7 -> 6.4e-7 and 7.4e-7 -> 6.3e-7, and not
-// larger in any of 25 float32 calls over B 1..468, T and M 6..3638, D 16..128.
+// Every float32 kernel forms its products this way and in this order: the kernels of one call rebuild each other's
+// scores and probabilities (lse, the row statistics of the double backward), and differences of values rounded two
+// ways do not cancel (row statistics from v_mfma_f32_32x32x2_f32 beside split products here: G_V of a peaked D128
+// problem off by 9 times the 1e-5 bar). Ops below is the one place that chooses the product.
+// Measured against v_mfma_f32_32x32x2_f32 throughout: forward + backward of B2 H16 T1000 D64 458 -> 282 us, the HVP of
+// B8 H8 T512 D64 785 -> 512 us, of B4 H8 T700 D128 3713 -> 1790 us; relative error against float64 7.3e-7 -> 6.4e-7,
+// 7.4e-7 -> 6.2e-7 and 8.8e-7 -> 7.5e-7, and not larger in any of eight second-order calls at D 72..128.
 struct X3Frag {
   bf16x8_t h, m, l;
 };
@@ -154,17 +149,13 @@ __device__ __forceinline__ bool lse_peaked(float lse) {
 }
 
 // ----------------------------------------------------------------------------------------------
-// k-index mapping of fragment element 0 / element EPL/2 for 16-bit types, and the single element of
-// float32 fragments. c is the chunk index (KC wide), g the lane half.
+// k-index mapping of fragment element 0 / element EPL/2. c is the chunk index (KC wide), g the lane half.
 // ----------------------------------------------------------------------------------------------
 template <int ORDER> __device__ __forceinline__ int k16_first(int c, int g) {
   return ORDER == KLIN ? c * 16 + 8 * g : c * 16 + 4 * g;
 }
 template <int ORDER> __device__ __forceinline__ int k16_second(int c, int g) {
   return ORDER == KLIN ? c * 16 + 8 * g + 4 : c * 16 + 4 * g + 8;
-}
-template <int ORDER> __device__ __forceinline__ int k32(int c, int g) {
-  return ORDER == KLIN ? 2 * c + g : acc_row(c, g);
 }
 
 // ----------------------------------------------------------------------------------------------
@@ -174,20 +165,16 @@ template <int ORDER> __device__ __forceinline__ int k32(int c, int g) {
 template <typename T, int ORDER>
 __device__ __forceinline__ typename Mfma<T>::frag_t lds_cols(const T* base, int pitch, int row, int kbase, int c) {
   const int g = (threadIdx.x >> 5) & 1;
-  if constexpr (sizeof(T) == 2) {
-    using F = typename Mfma<T>::frag_t;
-    const T* p0 = base + row * pitch + kbase + k16_first<ORDER>(c, g);
-    if constexpr (ORDER == KLIN) {
-      return __builtin_bit_cast(F, *reinterpret_cast<const i16x8_t*>(p0));
-    } else {
-      const T* p1 = base + row * pitch + kbase + k16_second<ORDER>(c, g);
-      i16x4_t a = *reinterpret_cast<const i16x4_t*>(p0);
-      i16x4_t b = *reinterpret_cast<const i16x4_t*>(p1);
-      i16x8_t v = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-      return __builtin_bit_cast(F, v);
-    }
+  using F = typename Mfma<T>::frag_t;
+  const T* p0 = base + row * pitch + kbase + k16_first<ORDER>(c, g);
+  if constexpr (ORDER == KLIN) {
+    return __builtin_bit_cast(F, *reinterpret_cast<const i16x8_t*>(p0));
   } else {
-    return base[row * pitch + kbase + k32<ORDER>(c, g)];
+    const T* p1 = base + row * pitch + kbase + k16_second<ORDER>(c, g);
+    i16x4_t a = *reinterpret_cast<const i16x4_t*>(p0);
+    i16x4_t b = *reinterpret_cast<const i16x4_t*>(p1);
+    i16x8_t v = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    return __builtin_bit_cast(F, v);
   }
 }
 
@@ -202,46 +189,34 @@ template <typename T, int ORDER>
 __device__ __forceinline__ typename Mfma<T>::frag_t lds_rows(const T* base, int pitch, int kbase, int c, int col0) {
   const int lane = threadIdx.x & 63;
   const int g = lane >> 5;
-  if constexpr (sizeof(T) == 2) {
-    using F = typename Mfma<T>::frag_t;
-    const int s = lane & 15, hh = (lane >> 4) & 1;
-    const int col = col0 + 16 * hh + 4 * (s & 3);
-    const T* p0 = base + (kbase + k16_first<ORDER>(c, g) + (s >> 2)) * pitch + col;
-    const T* p1 = base + (kbase + k16_second<ORDER>(c, g) + (s >> 2)) * pitch + col;
-    i16x4_t a = ds_read_tr16(p0);
-    i16x4_t b = ds_read_tr16(p1);
-    i16x8_t v = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-    return __builtin_bit_cast(F, v);
-  } else {
-    return base[(kbase + k32<ORDER>(c, g)) * pitch + col0 + (lane & 31)];
-  }
+  using F = typename Mfma<T>::frag_t;
+  const int s = lane & 15, hh = (lane >> 4) & 1;
+  const int col = col0 + 16 * hh + 4 * (s & 3);
+  const T* p0 = base + (kbase + k16_first<ORDER>(c, g) + (s >> 2)) * pitch + col;
+  const T* p1 = base + (kbase + k16_second<ORDER>(c, g) + (s >> 2)) * pitch + col;
+  i16x4_t a = ds_read_tr16(p0);
+  i16x4_t b = ds_read_tr16(p1);
+  i16x8_t v = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  return __builtin_bit_cast(F, v);
 }
 
 // Accumulator tile -> operand fragment whose k index is the tile row (KACC order), chunk c.
 // c must be a compile-time constant after unrolling so the register indices stay static.
 template <typename T>
 __device__ __forceinline__ typename Mfma<T>::frag_t acc_frag(const f32x16_t& a, int c) {
-  if constexpr (sizeof(T) == 2) {
-    typename Mfma<T>::frag_t f;
+  typename Mfma<T>::frag_t f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = (T)a[c * 8 + e];
-    return f;
-  } else {
-    return a[c];
-  }
+  for (int e = 0; e < 8; ++e) f[e] = (T)a[c * 8 + e];
+  return f;
 }
 
 // Fragment with every element multiplied by x (in float32, rounded once to T).
 template <typename T>
 __device__ __forceinline__ typename Mfma<T>::frag_t scaled_frag(const typename Mfma<T>::frag_t& f, float x) {
-  if constexpr (sizeof(T) == 2) {
-    typename Mfma<T>::frag_t r;
+  typename Mfma<T>::frag_t r;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = (T)((float)f[e] * x);
-    return r;
-  } else {
-    return f * x;
-  }
+  for (int e = 0; e < 8; ++e) r[e] = (T)((float)f[e] * x);
+  return r;
 }
 
 // Two-term 16-bit split of accumulator chunk c (16-bit T only): hi = round(x), lo = round(x - hi), so
@@ -268,24 +243,19 @@ __device__ __forceinline__ typename Mfma<T>::frag_t gload_frag(const T* base, in
                                                               int D, bool vec) {
   using F = typename Mfma<T>::frag_t;
   const int g = (threadIdx.x >> 5) & 1;
-  if constexpr (sizeof(T) == 2) {
-    const int col = c * 16 + 8 * g;
-    i16x8_t v = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (row < nrows) {
-      const T* p = base + (int64_t)row * rs + col;
-      if (vec && col + 8 <= D) {
-        v = *reinterpret_cast<const i16x8_t*>(p);
-      } else {
-        const short* ps = reinterpret_cast<const short*>(p);
+  const int col = c * 16 + 8 * g;
+  i16x8_t v = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (row < nrows) {
+    const T* p = base + (int64_t)row * rs + col;
+    if (vec && col + 8 <= D) {
+      v = *reinterpret_cast<const i16x8_t*>(p);
+    } else {
+      const short* ps = reinterpret_cast<const short*>(p);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = (col + e < D) ? ps[e] : (short)0;
-      }
+      for (int e = 0; e < 8; ++e) v[e] = (col + e < D) ? ps[e] : (short)0;
     }
-    return __builtin_bit_cast(F, v);
-  } else {
-    const int col = 2 * c + g;
-    return (row < nrows && col < D) ? base[(int64_t)row * rs + col] : 0.f;
   }
+  return __builtin_bit_cast(F, v);
 }
 
 // Cooperative tile staging: a [ROWS][DP] tile of rows row0.. of a (rows, D) matrix, loaded into
@@ -474,10 +444,10 @@ __device__ __forceinline__ X3Frag split3(const float (&x)[8]) {
   return f;
 }
 
-// Tile layout, fragment access and product of a kernel over elements T at padded head dim DP. X3: float32 with
-// the split products; its LDS tiles hold each row as three bfloat16 planes of DP columns (h | m | l), split once
+// Tile layout, fragment access and product of a kernel over elements T at padded head dim DP. float32 has its own form
+// with the split products: its LDS tiles hold each row as three bfloat16 planes of DP columns (h | m | l), split once
 // when the tile is staged, so that fragments are read as a 16-bit tile's are (ds_read_b128, ds_read_b64_tr_b16).
-template <typename T, int DP, bool X3>
+template <typename T, int DP>
 struct Ops {
   using MM = Mfma<T>;
   using F = typename MM::frag_t;
@@ -508,7 +478,7 @@ struct Ops {
 };
 
 template <int DP>
-struct Ops<float, DP, true> {
+struct Ops<float, DP> {
   using MM = MfmaX3;
   using F = X3Frag;
   static constexpr int KC = MM::KC;

@@ -33,7 +33,7 @@ namespace theria {
 // SPLIT: one part of the keys per workgroup (FwdParams::nsplit), no causal mask.
 template <typename T, int DP, bool CAUSAL, int QT, int BN, int NW = 4, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NW, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel(const FwdParams p) {
-  using OP = Ops<T, DP, sizeof(T) == 4>;
+  using OP = Ops<T, DP>;
   using F = typename OP::F;
   constexpr int KC = OP::KC;
   constexpr int BM = 32 * NW * QT, NT = 64 * NW;

@@ -40,7 +40,7 @@ __global__ __launch_bounds__(64 * NW, sizeof(T) == 4 && DP == 32 ? 2 : 1) void j
   // another order of rounding don't cancel its error (T20 M90 D80 std 2, 2-norm against float64: 1.20e-6 -> 7.3e-7).
   // Above head dim 64 this also beats the float32 MFMA, ~40 spilled registers included (us: B4 H8 T700 D128 266 -> 191,
   // B16 H16 T300 D128 causal 367 -> 286, B300 H8 T20 M90 D80 426 -> 386).
-  using OP = Ops<T, DP, sizeof(T) == 4>;
+  using OP = Ops<T, DP>;
   using F = typename OP::F;
   constexpr int KC = OP::KC;
   constexpr int BM = 32 * NW, NT = 64 * NW;

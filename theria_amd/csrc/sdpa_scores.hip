@@ -11,8 +11,8 @@
 //  * one workgroup = 4 waves = 128 query rows of one (batch, head); each wave keeps its 32 queries' Q fragments
 //    in registers and the workgroup streams K in 64-key tiles through LDS (one global read of K per workgroup,
 //    register-prefetched one tile ahead);
-//  * scores are formed lane-per-query (S^T = K Q^T with MFMA, float32 accumulation: for float32 inputs
-//    v_mfma_f32_32x32x2_f32 forms exact float32 products and sums, the reference's "ieee" dot);
+//  * scores are formed lane-per-query (S^T = K Q^T with MFMA, float32 accumulation: float32 inputs
+//    take the split products, which keep float32's precision as the reference's "ieee" dot does);
 //  * each wave writes its 32 x 32 subtiles of results into its own padded LDS buffer and reads them back
 //    row-major, 16 bytes per lane, with non-temporal stores (the output is not read again by this kernel; K stays
 //    in L2). For 16-bit inputs up to head dim 64 the buffer holds four subtiles (16.5 KiB per wave), so that one
@@ -44,7 +44,7 @@ constexpr bool scores_wide() {
 
 template <typename T, int DP, int MODE>
 __global__ __launch_bounds__(256, (scores_wide<T, DP>() || DP > 64) ? 2 : 4) void scores_kernel(const ScoresParams p) {
-  using Tile = Ops<T, DP, sizeof(T) == 4>;
+  using Tile = Ops<T, DP>;
   using F = typename Tile::F;
   constexpr int NKC = DP / Tile::KC;
   constexpr int NW = 4, NT = 64 * NW, BN = 64, NU = BN / 32;

@@ -33,7 +33,7 @@ namespace theria {
 template <typename T, int DP>
 struct Small {
   static constexpr int R = 64, NT = 128;  // rows per tile, threads
-  using OP = Ops<T, DP, sizeof(T) == 4>;
+  using OP = Ops<T, DP>;
   using F = typename OP::F;
   using Stage = TileStage<T, R, DP, NT>;
   static constexpr int NKC = DP / OP::KC, NPC = 32 / OP::KC, NDT = DP < 32 ? 1 : DP / 32;
