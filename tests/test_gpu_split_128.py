@@ -72,3 +72,29 @@ def test_causal_dq_of_small_and_large_grids(T, D, hip_device):
         got.append(_ops.bwd(*ts[:3], o, lse, ts[3], D**-0.5, True))
     for a, b in zip(*got):
         assert torch.equal(a[0, 0], b[0, 0]) and torch.equal(a[0, 0], b[0, 159])
+
+
+def rounding(x, dt):
+    """2-norm error of rounding a float64 tensor to dt, relative to it."""
+    return float((x.to(dt).double() - x).norm() / x.norm())
+
+
+@pytest.mark.parametrize("std", [0.5, 1.0])
+@pytest.mark.parametrize("dt,D", [(BF16, 72), (BF16, 128), (F16, 96)])
+def test_jvp_error_is_the_rounding_of_its_output(dt, D, std, hip_device):
+    """Spread-out rows, few (two key groups) and many (one) blocks: P o G and P enter their products as two 16-bit terms,
+    2^-16 of the cancelling terms, so that of the tangents of Q and K only the output's own rounding shows (bar: 1.05
+    times it; one 16-bit term each gave 1.4 times)."""
+    for B, H, causal in ((1, 4, False), (1, 4, True), (16, 8, False)):
+        T, M = 200, 300
+        print(f"[split 128 jvp rounding] {dt} B{B}H{H} D{D} std{std} causal={causal}", flush=True)
+        g = torch.Generator().manual_seed(D + B)
+        q, tq = (torch.randn(B, H, T, D, generator=g).mul(x).to(dt) for x in (std, 1.0))
+        k, tk, v = (torch.randn(B, H, M, D, generator=g).mul(x).to(dt) for x in (std, 1.0, 1.0))
+        dev = [t.to(hip_device) for t in (q, k, v)]
+        o, lse = _ops.fwd(*dev, D**-0.5, causal)[:2]
+        got = _ops.jvp(*dev, o, lse, tq.to(hip_device), tk.to(hip_device), None, D**-0.5, causal).cpu().double()
+        ref = O.jvp(q, k, v, tq, tk, None, D**-0.5, causal)
+        err = float((got - ref).norm() / ref.norm())
+        print(f"    error {err:.3e}, rounding {rounding(ref, dt):.3e}", flush=True)
+        assert err <= 1.05 * rounding(ref, dt)

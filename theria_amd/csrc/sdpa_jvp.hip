@@ -12,8 +12,8 @@
 // amplified (a bfloat16-rounded P o G gave 0.03 absolute error on a row with four visible keys). Both
 // products are therefore formed from two-term 16-bit splits (hi + lo) of P o G and of P, and O is always
 // rebuilt in the pass from the same P (the saved O, rounded to 16 bits, is not used). The key-split kernel
-// (jvp_ksplit_kernel, below) takes the split only in waves holding a row flagged peaked in lse: elsewhere the
-// rounding of P o G and P spreads over many keys and one 16-bit term each suffices.
+// (jvp_ksplit_kernel, below) takes the split at head dims up to 64 only in waves holding a row flagged peaked in lse:
+// elsewhere the rounding of P o G and P spreads over many keys and one 16-bit term each keeps the 16-bit bar.
 // p.normalize divides P by its own row sum (every dtype): the JVP of the exact softmax for an lse this
 // library's forward wrote (a 16-bit forward's lse comes from rounded probabilities, so P rebuilt from it
 // sums to 1 only within ~2^-9). Without it P = exp(S - lse) is held exactly as given, which is the
@@ -227,8 +227,9 @@ __global__ __launch_bounds__(64 * NW, sizeof(T) == 4 && DP == 32 ? 2 : 1) void j
 // row sums) are exchanged through LDS at the end. DP = 128, whose accumulators take a whole SIMD per wave: G = 2 groups of
 // two waves (64 queries, 32-key tiles) where 128-query workgroups would leave CUs idle, else G = 1 group of four waves
 // (128 queries, no exchange), which reads each tile for twice the queries (us, the one-group kernel it replaced -> G = 2 /
-// G = 1, bfloat16: B2 H8 T1024 86 -> 32 / 46, B2 H16 T1024 90 -> 66 / 56, B1 H4 T8192 605 -> 405 / 356, B64 H8 T1000 M96
-// 250 -> 324 / 221, B2 H8 T1024 causal 86 -> 33). ALL: every tangent is given (the presence tests are then
+// G = 1, bfloat16 D128: B2 H8 T1024 84 -> 46 / 62, B2 H16 T1024 90 -> 84 / 74, B1 H4 T8192 601 -> 511 / 457, B64 H8 T1000
+// M96 250 -> 320 / 217, B2 H8 T1024 causal 84 -> 36 / 56; one 16-bit term instead of two would take 30 to 350 us of these
+// and raise the error 1.4 times). ALL: every tangent is given (the presence tests are then
 // constants, and the loop body has no branches between its products).
 template <typename T, bool CAUSAL, bool ALL, bool FD, int DP, int G>
 __global__ __launch_bounds__(DP == 64 ? 512 : 256, DP == 64 ? 2 : 1) void jvp_ksplit_kernel(const JvpParams p) {
@@ -288,10 +289,11 @@ __global__ __launch_bounds__(DP == 64 ? 512 : 256, DP == 64 ? 2 : 1) void jvp_ks
   const float lse2 = lse_raw * kLog2e;
   const float moff = lse2 == -THERIA_INF ? THERIA_INF : lse2;  // a row without visible keys has P = 0
   float cpart = 0.f, lpart = 0.f;
-  // The two-term products only in waves holding a row flagged peaked in lse (a dominant probability, which
+  // DP = 64: the two-term products only in waves holding a row flagged peaked in lse (a dominant probability, which
   // rows with few visible keys have): there (P o G) V and c o O cancel. Elsewhere the rounding of P o G and
-  // P spreads over many keys and one 16-bit term each suffices (uniform per wave).
-  const bool split = __any(lse_peaked(lse_raw));
+  // P spreads over many keys and one 16-bit term each keeps the bar (uniform per wave). DP = 128: every wave, so that
+  // nothing but the rounding of the output shows (and a caller's lse, which carries no flags, decides nothing).
+  const bool split = DP == 128 || __any(lse_peaked(lse_raw));
 
   int kend = s.M;
   if (CAUSAL) kend = min(s.M, qb * BM + BM);
@@ -412,10 +414,11 @@ __global__ __launch_bounds__(DP == 64 ? 512 : 256, DP == 64 ? 2 : 1) void jvp_ks
   else if (kt0 < kt1)
     issue_one(grp, kt0, 0);
   // The waves of a workgroup may take different copies of the loop: both meet the same barriers.
-  if (split)
+  if (DP == 128 || split) {
     sweep(std::integral_constant<bool, true>{});
-  else
-    sweep(std::integral_constant<bool, false>{});
+  } else {
+    if constexpr (DP == 64) sweep(std::integral_constant<bool, false>{});
+  }
 
   // Epilogue as jvp_kernel's (O rebuilt from the same P; normalize: P divided by its own row sum), for the N column tiles
   // from DT0 on.
