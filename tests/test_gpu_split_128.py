@@ -98,3 +98,23 @@ def test_jvp_error_is_the_rounding_of_its_output(dt, D, std, hip_device):
         err = float((got - ref).norm() / ref.norm())
         print(f"    error {err:.3e}, rounding {rounding(ref, dt):.3e}", flush=True)
         assert err <= 1.05 * rounding(ref, dt)
+
+
+@pytest.mark.parametrize("std", [0.5, 1.0])
+@pytest.mark.parametrize("dt,D", [(BF16, 72), (BF16, 128), (F16, 96)])
+def test_double_backward_of_dout_error_is_the_rounding_of_its_output(dt, D, std, hip_device):
+    """G_dO of the key-split row kernel, whose first pass also sums z and t from the same products: as the JVP above."""
+    T, M = 200, 300
+    for causal in (False, True):
+        print(f"[split 128 G_dO rounding] {dt} D{D} std{std} causal={causal}", flush=True)
+        g = torch.Generator().manual_seed(D)
+        q, tq = (torch.randn(2, 3, T, D, generator=g).mul(x).to(dt) for x in (std, 1.0))
+        k, tk, v = (torch.randn(2, 3, M, D, generator=g).mul(x).to(dt) for x in (std, 1.0, 1.0))
+        do = torch.randn(2, 3, T, D, generator=g).to(dt)
+        dq, dk, dv, ddo, dtq, dtk = (t.to(hip_device) for t in (q, k, v, do, tq, tk))
+        o, lse = _ops.fwd(dq, dk, dv, D**-0.5, causal)[:2]
+        got = _ops.bwd_bwd(dq, dk, dv, o, ddo, lse, None, dtq, dtk, None, D**-0.5, causal)[3].cpu().double()
+        ref = O.jvp(q, k, v, tq, tk, None, D**-0.5, causal)
+        err = float((got - ref).norm() / ref.norm())
+        print(f"    error {err:.3e}, rounding {rounding(ref, dt):.3e}", flush=True)
+        assert err <= 1.05 * rounding(ref, dt)

@@ -36,8 +36,8 @@ bool cols_qs_ok(const BwdBwdParams& p) {
 // multiple of 8, the tile columns past D zero-filled), as two key groups: at DP = 64 of four waves (eight-wave workgroups
 // of 128 queries, two waves per SIMD), at 128 of two (64 queries, 32-key tiles, one wave per SIMD at up to 512
 // registers; at 128 the general row kernel spilled and swept every key per wave, and the row terms and G_dO were launches
-// of their own. Double backward, bfloat16 D128, before -> here: B2 H8 T1024 474 -> 133 us, causal 383 -> 135, B1 H4 T8192
-// 3983 -> 1781, B8 H16 T512 597 -> 309, B64 H8 T65 236 -> 159). The keys of each query block are split between the
+// of their own. Double backward, bfloat16 D128, before -> here: B2 H8 T1024 472 -> 161 us, causal 383 -> 146, B1 H4 T8192
+// 3987 -> 1960, B8 H16 T512 596 -> 330, B64 H8 T65 236 -> 159). The keys of each query block are split between the
 // groups, whose partial sums meet in LDS. Each group makes two passes over its key tiles:
 //   1. with P from the forward's lse: L = sum_j P, sum_j P Gam and the largest P, and the D-wide products
 //      A = sum_j (P o Gam) V + sum_j P gV and O = sum_j P V, partial per group, then exchanged. Then
@@ -47,7 +47,11 @@ bool cols_qs_ok(const BwdBwdParams& p) {
 //      E1 = Gam (dP - z) + W, i.e. t = (dO . A - z sum_j P Gam) / L; and G_dO = (A - r O) / L, the JVP of O;
 //   2. G_Q = s sum_j (Gbar_S K + dS gK) with Gbar_S = P_c o ((Gam - r)(dP - z) + W - t), the exact form, in two
 //      D-wide accumulators.
-// Waves holding a row flagged peaked in the forward's lse enter P, P o Gam, Gbar_S and dS as two 16-bit terms.
+// P, P o Gam, Gbar_S and dS enter as two 16-bit terms each in waves holding a row flagged peaked in the forward's lse, and
+// at DP = 128 in every wave: the general kernel there summed z and t in float32, took the JVP's two-term products for G_dO,
+// and redid whole 128-row blocks holding a flagged row in two terms, and with one term in the other waves G_dO's error was
+// 1.4 times its rounding and G_Q's up to 1.09 times that kernel's (two terms: no output's error is larger, over 48 calls at
+// D 72..128 and std 0.5..2; they take 0 to 20 of the 146 to 330 us above).
 // Every row takes the exact form (no centring, no second launch for flagged rows, no separate row-term or JVP
 // pass); the gQ fragments sit in LDS, so that each pass's two accumulators, the per-wave Q and dO fragments and
 // the products fit 256 registers. Writes G_Q and G_dO, and r, t, z and lse + ln L (flagged peaked when the
@@ -109,7 +113,8 @@ __global__ __launch_bounds__(DP == 64 ? 512 : 256, DP == 64 ? 2 : 1) void bwdbwd
   const float lse2 = lse_raw * kLog2e;
   float moff = lse2 == -THERIA_INF ? THERIA_INF : lse2;  // a row without visible keys has P = 0; pass 2: P_c
   float z = 0.f;                                          // pass 2: the row term (pass 1 forms dP itself)
-  const bool split = __any(lse_peaked(lse_raw));  // uniform per wave (the forward's bound: a superset)
+  // two-term products (uniform per wave; the forward's bound: a superset of the peaked rows)
+  const bool split = DP == 128 || __any(lse_peaked(lse_raw));
 
   int kend = s.M;
   if (CAUSAL) kend = min(s.M, qb * BM + BM);
@@ -312,12 +317,14 @@ __global__ __launch_bounds__(DP == 64 ? 512 : 256, DP == 64 ? 2 : 1) void bwdbwd
   };
   float* buf = reinterpret_cast<float*>(smem);
 
-  if (split)
+  if (DP == 128 || split) {
     sweep([&](auto mask_tag, int kt, const char* a, const char* b_, const char* c, const char* d)
               __attribute__((always_inline)) { compute_sums(std::true_type{}, mask_tag, kt, a, b_, c, d); });
-  else
-    sweep([&](auto mask_tag, int kt, const char* a, const char* b_, const char* c, const char* d)
-              __attribute__((always_inline)) { compute_sums(std::false_type{}, mask_tag, kt, a, b_, c, d); });
+  } else {
+    if constexpr (DP == 64)
+      sweep([&](auto mask_tag, int kt, const char* a, const char* b_, const char* c, const char* d)
+                __attribute__((always_inline)) { compute_sums(std::false_type{}, mask_tag, kt, a, b_, c, d); });
+  }
   // dO . sum_j P V and dO . (sum_j (P o Gam) V + sum_j P gV) over this lane's columns of the accumulators
   float a_dot = 0.f, uw_dot = 0.f;
   if (qvalid) {
@@ -392,12 +399,14 @@ __global__ __launch_bounds__(DP == 64 ? 512 : 256, DP == 64 ? 2 : 1) void bwdbwd
   }
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) acc[dt] = accy[dt] = zero16();
-  if (split)
+  if (DP == 128 || split) {
     sweep([&](auto mask_tag, int kt, const char* a, const char* b_, const char* c, const char* d)
               __attribute__((always_inline)) { compute_exact(std::true_type{}, mask_tag, kt, a, b_, c, d); });
-  else
-    sweep([&](auto mask_tag, int kt, const char* a, const char* b_, const char* c, const char* d)
-              __attribute__((always_inline)) { compute_exact(std::false_type{}, mask_tag, kt, a, b_, c, d); });
+  } else {
+    if constexpr (DP == 64)
+      sweep([&](auto mask_tag, int kt, const char* a, const char* b_, const char* c, const char* d)
+                __attribute__((always_inline)) { compute_exact(std::false_type{}, mask_tag, kt, a, b_, c, d); });
+  }
 
   // group 1's accumulators to group 0 (element e of lane l of wave w at e * GT + w * 64 + l)
   if (grp == 1) {
