@@ -90,3 +90,32 @@ def test_split_forward_with_masked_keys(hip_device):
     for a, b in zip(got, want):
         torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
     assert (got[0][:, 1] == 0).all() and (got[1][:, 1] == -float("inf")).all()
+
+
+@pytest.mark.parametrize("dt", [F16, BF16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("T,D", [(1, 64), (65, 96), (100, 128), (128, 40), (60, 20)])
+def test_split_forward_sums_rows_in_float32(T, D, dt, hip_device):
+    """At most 128 queries: lse and the row sum are sums of float32 P, as they are unsplit, also where later keys' scores
+    are far above the first tiles' (float16 then moves the offset before a P leaves its range: 13 nats a tile). Bounds:
+    1e-5 for the sum of M float32 terms; in l's exponentials also the roundings of a score of size |S|: scale log2(e) (two),
+    the dot product (two), its product with that, the maximum in the log2 domain and back, and their difference, each
+    at most 2^-24 |S|: 8 of them. Rounded P gave 1e-4."""
+    M, scale = 1500, D**-0.5
+    print(f"[split forward row sums] {dt} T{T} D{D}", flush=True)
+    g = torch.Generator().manual_seed(T + D)
+    for std, rise in ((0.5, 0.0), (2.0, 0.0), (0.5, 300.0)):
+        q, k, v = (torch.randn(1, 3, n, D, generator=g) for n in (T, M, M))
+        q, k = q * std, k * std
+        if rise:  # scores climb by `rise` over the keys along one direction
+            q[..., 0] = 1.0
+            k[..., 0] = torch.linspace(0.0, rise / scale, M)
+        q, k, v = (t.to(dt) for t in (q, k, v))
+        assert _lib.load().theria_sdpa_fwd_ws_floats(ctypes.byref(_ops._problem(q, k, scale, False))) > 0
+        S = (q.double() @ k.double().transpose(-2, -1)) * scale
+        m = S.amax(-1)
+        l = torch.exp(S - m[..., None]).sum(-1)
+        got = _ops.fwd(*(t.to(hip_device) for t in (q, k, v)), scale, False, stats=True)
+        bars.close(got[0], torch.softmax(S, -1) @ v.double(), what="O", **bars.tol(dt))
+        bars.close(got[1], m + torch.log(l), what="lse", rtol=1e-5, atol=1e-5)
+        bars.close(got[2], m, what="m", rtol=1e-5, atol=1e-5)
+        bars.close(got[3], l, what="l", rtol=1e-5 + 8 * 2.0**-24 * float(S.abs().max()), atol=0.0)

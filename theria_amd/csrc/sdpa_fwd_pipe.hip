@@ -22,7 +22,9 @@
 //    than ~14 in the log2 domain) takes a slow path that recomputes S, moves m_use to the exact running
 //    max and rescales O and the row sum. lse = m_use + log2(l) does not depend on the offset.
 //  * Row sums are accumulated from the rounded 16-bit P values that feed the PV product (v_dot2), so
-//    numerator and denominator use the same probabilities.
+//    numerator and denominator use the same probabilities. FSUM (split keys, at most 128 queries): from the float32 P,
+//    as the general kernel that takes these problems whole, so that lse and the row sum do not lose 2^-9 by the split
+//    (lse of fp16 T65 M513 D96 std 2: off by 1.2e-6 on average, 9.4e-5 from rounded P).
 #include <type_traits>
 
 #include "fwd_split.hpp"
@@ -52,8 +54,8 @@ hipError_t tile_counts_fwd(unsigned long long* fwd, bool reset) {
 }
 #endif
 
-// SPLIT: one part of the keys per workgroup (FwdParams::nsplit), no causal mask.
-template <typename T, bool CAUSAL, bool STATS, int NW, int DP, int QT, bool FD, bool SPLIT = false>
+// SPLIT: one part of the keys per workgroup (FwdParams::nsplit), no causal mask. FSUM: row sums of float32 P.
+template <typename T, bool CAUSAL, bool STATS, int NW, int DP, int QT, bool FD, bool SPLIT = false, bool FSUM = false>
 __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p) {
   using MM = Mfma<T>;
   using F = typename MM::frag_t;
@@ -145,6 +147,9 @@ __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p)
       m_max[j] = -THERIA_INF;
       pk_max[j] = 0.f;
     }
+    // Largest lane partial row sum of a tile that keeps the offset. A P that float16 cannot hold makes a sum of rounded P
+    // infinite; a sum of float32 P has to stay below float16's largest value itself.
+    constexpr float kMaxSum = FSUM ? 0x1p15f : 0x1p20f;
     F pf[QT][2][2];  // P of the previous tile as MFMA B fragments: [query tile][32-key subtile][16-key chunk]
     bool pf_skip = false;
 
@@ -209,9 +214,14 @@ __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p)
           for (int cc = 0; cc < 2; ++cc) {
             F f;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) f[e] = (T)fast_exp2(fmaf(sc[j][t][8 * cc + e], c2, -off[j]));
+            for (int e = 0; e < 8; ++e) {
+              const float x = fast_exp2(fmaf(sc[j][t][8 * cc + e], c2, -off[j]));
+              f[e] = (T)x;
+              if constexpr (FSUM) acc += x;
+            }
             pn[j][t][cc] = f;
-            if constexpr (FINE) {
+            if constexpr (FSUM) {
+            } else if constexpr (FINE) {
               const float fs = frag_sum<T>(f, 0.f);
               acc += fs;
               mx = fmaxf(mx, fs);
@@ -231,9 +241,14 @@ __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p)
         for (int cc = 0; cc < 2; ++cc) {
           F f;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) f[e] = (T)fast_exp2(fmaf(st[j][8 * cc + e], c2, -m_use[j]));
+          for (int e = 0; e < 8; ++e) {
+            const float x = fast_exp2(fmaf(st[j][8 * cc + e], c2, -m_use[j]));
+            f[e] = (T)x;
+            if constexpr (FSUM) ps[j] += x;
+          }
           pn[j][t][cc] = f;
-          if constexpr (FINE) {
+          if constexpr (FSUM) {
+          } else if constexpr (FINE) {
             const float fs = frag_sum<T>(f, 0.f);
             ps[j] += fs;
             pk[j] = fmaxf(pk[j], fs);
@@ -346,7 +361,7 @@ __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p)
         }
         bool bad = false;
 #pragma unroll
-        for (int j = 0; j < QT; ++j) bad |= !(ps[j] <= 0x1p20f);
+        for (int j = 0; j < QT; ++j) bad |= !(ps[j] <= kMaxSum);
         if (__any(bad)) {
           f32x16_t sc2[QT][2];
           scores(kc, sc2);
@@ -382,7 +397,7 @@ __global__ __launch_bounds__(64 * NW, 2) void fwd_pipe_kernel(const FwdParams p)
             exps(sc, m_use, pn, ps, pk);
             bool bad = false;
 #pragma unroll
-            for (int j = 0; j < QT; ++j) bad |= !(ps[j] <= 0x1p20f);
+            for (int j = 0; j < QT; ++j) bad |= !(ps[j] <= kMaxSum);
             if (__any(bad)) {
               f32x16_t sc2[QT][2];
               scores(kc, sc2);
@@ -511,10 +526,14 @@ static void fwd_pipe_launch(const FwdParams& p0, hipStream_t st) {
   if constexpr (!CAUSAL) {
     if (p.nsplit > 1) {  // (the statistics kernel: the parts' row maxima are combined whether or not m is wanted)
       const dim3 grid((unsigned)((p.s.T + 127) / 128 * bh * p.nsplit)), block(256);
+      auto go = [&](auto fd_tag, auto fsum_tag) {
+        constexpr bool FD = decltype(fd_tag)::value, FSUM = decltype(fsum_tag)::value;
+        hipLaunchKernelGGL((fwd_pipe_kernel<T, false, true, 4, DP, 1, FD, true, FSUM>), grid, block, 0, st, p);
+      };
       if (p.s.D == DP)
-        hipLaunchKernelGGL((fwd_pipe_kernel<T, false, true, 4, DP, 1, true, true>), grid, block, 0, st, p);
+        p.s.T <= 128 ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
       else
-        hipLaunchKernelGGL((fwd_pipe_kernel<T, false, true, 4, DP, 1, false, true>), grid, block, 0, st, p);
+        p.s.T <= 128 ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
       return;
     }
   }
