@@ -80,3 +80,49 @@ def test_small_backward_equals_general_kernels(dt, D, std, hip_device):
             only_dv = _ops.bwd(q, k, v, o, lse, do, scale, causal, need_dq=False, need_dk=False)
             assert only_dv[0] is None and only_dv[1] is None
             assert torch.equal(only_dv[2], got[2]) and torch.equal(only_dv[3], got[3])
+
+
+@pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("T,M", [(50, 40), (70, 40)], ids=["small", "general"])
+def test_nan_key_reaches_the_rows_that_see_it(T, M, dt, hip_device):
+    """A NaN in one key, no cotangent of dQ (so that it enters the double backward through P alone): every row that sees
+    the key is NaN throughout, the causal rows before it are as without it."""
+    print(f"[small nan] {dt} T{T} M{M}", flush=True)
+    D, key = 16, 20
+    g = torch.Generator(device=hip_device).manual_seed(3)
+    q, do = (torch.randn(2, 2, T, D, generator=g, device=hip_device).to(dt) for _ in range(2))
+    k, v, tk, tv = (torch.randn(2, 2, M, D, generator=g, device=hip_device).to(dt) for _ in range(4))
+    bad = k.clone()
+    bad[:, :, key, 5] = float("nan")
+    for causal in (False, True):
+        outs = []
+        for kk in (bad, k):
+            o, lse = _ops.fwd(q, kk, v, D**-0.5, causal)[:2]
+            outs.append(_ops.bwd_bwd(q, kk, v, o, do, lse, None, None, tk, tv, D**-0.5, causal))
+        first = key if causal else 0
+        for i in (0, 3):  # G_Q, G_dO
+            assert torch.isnan(outs[0][i][:, :, first:]).all()
+            cols = [d for d in range(D) if i == 3 or d != 5]  # (0 times NaN in that column of G_Q)
+            assert torch.equal(outs[0][i][:, :, :first, cols], outs[1][i][:, :, :first, cols])
+
+
+@pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("T,M", [(50, 40), (96, 40)], ids=["small", "general"])
+def test_rows_without_a_visible_score(T, M, dt, hip_device):
+    """Every score is -infinity: P = 0, so nothing but the columns that meet an infinite key element (0 times infinity)
+    is anything but 0."""
+    print(f"[small masked rows] {dt} T{T} M{M}", flush=True)
+    D = 16
+    g = torch.Generator(device=hip_device).manual_seed(4)
+    q, do = (torch.randn(2, 2, T, D, generator=g, device=hip_device).to(dt) for _ in range(2))
+    k, v, tk, tv = (torch.randn(2, 2, M, D, generator=g, device=hip_device).to(dt) for _ in range(4))
+    q[..., 0] = 1.0
+    k[..., 0] = -float("inf")
+    for causal in (False, True):
+        o, lse = _ops.fwd(q, k, v, D**-0.5, causal)[:2]
+        assert (o == 0).all() and (lse == -float("inf")).all()
+        dq, dk, dv = _ops.bwd(q, k, v, o, lse, do, D**-0.5, causal)[:3]
+        gq, gk, gv, gdo = _ops.bwd_bwd(q, k, v, o, do, lse, None, None, tk, tv, D**-0.5, causal)
+        for name, x in (("dQ", dq[..., 1:]), ("dK", dk), ("dV", dv), ("G_Q", gq[..., 1:]), ("G_K", gk), ("G_V", gv),
+                        ("G_dO", gdo)):
+            assert (x == 0).all(), name

@@ -118,14 +118,15 @@ __global__ __launch_bounds__(128, (sizeof(T) == 4 ? DP <= 32 : DP <= 64) ? 2 : 1
   const float c2 = s.scale * kLog2e;
   const int w0 = 32 * wave, my = w0 + li;  // this wave's first row (query or key) and this lane's
 
-  // Every load of the row phase in flight together, and (PRE: where the registers allow) the column phase's tiles.
+  // Every load of the row phase in flight together, and (PRE: where the registers allow) the column phase's tiles. Query
+  // rows past the end repeat the last one: a score of a zero row against an infinite key would be NaN, and their P is 0.
   constexpr bool PRE = DP <= 32;
   typename K_::Stage qs, os, gs_;
   typename OP::Raw r0[NKC], r1[NKC], r2[NKC];
   auto load_q_side = [&]() {
-    qs.load(Q, p.q.sr, 0, s.T, s.D, s.vec);
-    os.load(dO, p.dout.sr, 0, s.T, s.D, s.vec);
-    if (has_gq) gs_.load(GQ, p.gq.sr, 0, s.T, s.D, s.vec);
+    qs.template load<true>(Q, p.q.sr, 0, s.T, s.D, s.vec);
+    os.template load<true>(dO, p.dout.sr, 0, s.T, s.D, s.vec);
+    if (has_gq) gs_.template load<true>(GQ, p.gq.sr, 0, s.T, s.D, s.vec);
   };
   {
     typename K_::Stage a, c, d, e;
@@ -178,19 +179,20 @@ __global__ __launch_bounds__(128, (sizeof(T) == 4 ? DP <= 32 : DP <= 64) ? 2 : 1
         m2 = fmaxf(m2, sc[t][r]);
       }
     }
-    m2 = pair_max(m2);  // finite unless a score is: every query sees at least one key
+    m2 = pair_max(m2);  // -inf: every visible score is (or is NaN, which the sums below keep)
     float l = 0.f, a = 0.f;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float pv = sc[t][r] > -THERIA_INF ? fast_exp2(sc[t][r] - m2) : 0.f;
+        const float pv = sc[t][r] == -THERIA_INF ? 0.f : fast_exp2(sc[t][r] - m2);
         sc[t][r] = pv;
         l += pv;
         a = fmaf(pv, dp[t][r], a);
       }
     l = pair_sum(l);
-    const float inv = 1.f / l, z = pair_sum(a) * inv;
+    const bool none = l == 0.f;  // no visible key: P = 0
+    const float inv = none ? 0.f : 1.f / l, z = pair_sum(a) * inv;
     float rr = 0.f, tt = 0.f;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -205,7 +207,7 @@ __global__ __launch_bounds__(128, (sizeof(T) == 4 ? DP <= 32 : DP <= 64) ? 2 : 1
     rr = pair_sum(rr);
     tt = pair_sum(tt);
     if (g == 0) {
-      const bool ok = my < s.T;  // rows past the end: P = exp2(-inf) = 0
+      const bool ok = my < s.T && !none;  // rows past the end or without a visible key: P = exp2(-inf) = 0
       sRow[0][my] = ok ? m2 : THERIA_INF;
       sRow[1][my] = ok ? inv : 0.f;
       sRow[2][my] = ok ? z : 0.f;
@@ -330,8 +332,8 @@ __global__ __launch_bounds__(128, (sizeof(T) == 4 ? DP <= 64 : true) ? 2 : 1) vo
   typename K_::Stage qs, os;
   typename OP::Raw r0[NKC], r1[NKC];
   auto load_q_side = [&]() {
-    qs.load(Q, p.q.sr, 0, s.T, s.D, s.vec);
-    os.load(dO, p.dout.sr, 0, s.T, s.D, s.vec);
+    qs.template load<true>(Q, p.q.sr, 0, s.T, s.D, s.vec);
+    os.template load<true>(dO, p.dout.sr, 0, s.T, s.D, s.vec);
   };
   const float lse = my < s.T ? p.lse[row_id] : THERIA_INF;
   {
