@@ -1,12 +1,16 @@
-"""float32 products formed on the bfloat16 matrix pipe from three-term splits (MfmaX3): operands of any magnitude,
-the largest float32, infinities, and tile and k-chunk edges.
+"""float32 products formed on the bfloat16 matrix pipe from three-term splits (MfmaX3): operands of 2^-20 to 2^20 in one
+row, the largest float32 and infinities against operands of either residual sign, and tile and k-chunk edges.
 
-Bound: S = sum of D products, the split keeping each to 2^-26 and the accumulator rounding at most once per term:
-|S - S64| <= (D + 8) 2^-24 sum |q| |k|, float32's own bound for a sum of D terms in any order."""
+Bound: S = sum of D products, the split keeping each to 2^-24 (2^-21 where both operands are large) and the accumulator
+rounding at most once per term: |S - S64| <= (D + 8) 2^-24 sum |q| |k|, float32's own bound for a sum of D terms in any
+order."""
+
+import math
 
 import pytest
 import torch
 
+from oracle import sdpa_oracle as O
 from theria_amd import _ops
 from theria_amd.attention.scores import triton_qk
 
@@ -93,3 +97,54 @@ def test_one_visible_key_gives_no_curvature(T, M, causal, D, hip_device):
     o, lse = _ops.fwd(q, k, v, D**-0.5, causal)[:2]
     gq = _ops.bwd_bwd(q, k, v, o, do, lse, None, tq, tk, tv, D**-0.5, causal)[0]
     assert (gq[:, :, 0 if causal else slice(None)] == 0).all()
+
+
+def masked_inputs(T, M, D, mask):
+    """Standard normal inputs, q's first element 1002.5 (its bfloat16 is 1004: the residual has the other sign) or 800; keys
+    3, M / 2 and M - 1 masked by `mask` in that element. Every other key has 0 there."""
+    g = torch.Generator().manual_seed(T + D)
+    q, do = (torch.randn(2, 2, T, D, generator=g) for _ in range(2))
+    k, v, tk, tv = (torch.randn(2, 2, M, D, generator=g) for _ in range(4))
+    q[..., 0] = torch.where(torch.arange(T) % 2 == 0, 1002.5, 800.0)
+    k[..., 0] = 0.0
+    gone = [3, M // 2, M - 1]
+    k[:, :, gone, 0] = mask
+    return q, k, v, do, tk, tv, [j for j in range(M) if j not in gone], gone
+
+
+@pytest.mark.parametrize("mask", [-float("inf"), float(torch.finfo(torch.float32).min), -1e37], ids=["inf", "lowest", "1e37"])
+@pytest.mark.parametrize("T,M,D", [(40, 50, 16), (64, 64, 64), (160, 150, 16), (128, 150, 64), (96, 90, 80), (160, 150, 128)])
+def test_keys_masked_by_value(T, M, D, mask, hip_device):
+    """Scores below the lowest float32 are -infinity, whatever the products' terms overflow to, in every kernel: the keys
+    are gone from O, the tangent and the gradients (1e-5 of the float64 results without them)."""
+    print(f"float32 split masked keys T{T} M{M} D{D} {mask}", flush=True)
+    q, k, v, do, tk, tv, keep, gone = masked_inputs(T, M, D, mask)
+    scale = D**-0.5
+    dq_, dk_, dv_, ddo, dtk, dtv = (t.to(hip_device) for t in (q, k, v, do, tk, tv))
+    k0, v0, tk0, tv0 = (t[:, :, keep] for t in (k, v, tk, tv))
+    cols = slice(1, None) if math.isinf(mask) else slice(None)  # (0 times infinity in dQ's and G_Q's first column)
+
+    def close(got, ref, what):
+        got = got.double().cpu()
+        assert torch.isfinite(got).all(), what
+        tol = 1e-5 * max(1.0, float(ref.abs().max()))
+        torch.testing.assert_close(got, ref, rtol=1e-5, atol=tol, msg=lambda m: f"{what}: {m}")
+
+    s = triton_qk(dq_, dk_)
+    assert (s[..., gone] == -float("inf")).all() or mask == -1e37
+    o, lse = _ops.fwd(dq_, dk_, dv_, scale, False)[:2]
+    close(o, O.forward(q, k0, v0, scale, False)[0], "O")
+    gq, gk, gv = _ops.bwd(dq_, dk_, dv_, o, lse, ddo, scale, False)[:3]
+    rq, rk, rv = O.backward(q, k0, v0, do, scale, False)
+    close(gq[..., cols], rq[..., cols], "dQ")
+    for name, x, r in (("dK", gk, rk), ("dV", gv, rv)):
+        close(x[:, :, keep], r, name)
+        close(x[:, :, gone], torch.zeros_like(r[:, :, :3]), name + " of the masked keys")
+    t = _ops.jvp(dq_, dk_, dv_, o, lse, None, dtk, dtv, scale, False)
+    close(t, O.jvp(q, k0, v0, None, tk0, tv0, scale, False), "tangent")
+    hq, hk, hv, hdo = _ops.bwd_bwd(dq_, dk_, dv_, o, ddo, lse, None, None, dtk, dtv, scale, False)
+    Hq, Hk, Hv, Hdo = O.double_backward(q, k0, v0, do, torch.zeros_like(q), tk0, tv0, scale, False)
+    close(hq[..., cols], Hq[..., cols], "G_Q")
+    close(hdo, Hdo, "G_dO")
+    for name, x, r in (("G_K", hk, Hk), ("G_V", hv, Hv)):
+        close(x[:, :, keep], r, name)

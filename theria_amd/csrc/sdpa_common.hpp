@@ -26,6 +26,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace theria {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -69,9 +71,9 @@ template <> struct Mfma<_Float16> {
 };
 
 // float32 products on the bfloat16 matrix pipe. Each operand is split into three bfloat16 terms, h = bf16(x),
-// m = bf16(x - h), l = bf16(x - h - m), which hold all 24 bits of it (rounding to nearest leaves |m| <= 2^-9 |x|
-// and |l| <= 2^-18 |x|), and a b is summed as the six products down to 2^-18: the three dropped ones (m l, l m,
-// l l) are below 2^-26 of it, under float32's own rounding. One 16-wide k chunk then takes 6 x 32 cycles of the
+// m = bf16(x - h), l = bf16(x - h - m), which hold all 24 bits of it (rounding to nearest leaves |m| <= 2^-8 |x|
+// and |l| <= 2^-17 |x|), and a b is summed as the six products down to 2^-16: the three dropped ones (m l, l m,
+// l l) are at most 2^-24 of it and 2^-27 on average, under float32's own rounding. One 16-wide k chunk then takes 6 x 32 cycles of the
 // matrix pipe where eight v_mfma_f32_32x32x2_f32 take 8 x 64, and rounds the accumulator fewer times.
 // Every float32 kernel forms its products this way and in this order: the kernels of one call rebuild each other's
 // scores and probabilities (lse, the row statistics of the double backward), and differences of values rounded two
@@ -413,32 +415,49 @@ __device__ __forceinline__ f32x4_t load4(const T* base, int64_t rs, int row, int
 // ----------------------------------------------------------------------------------------------
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
-// Element i of a register array of 8 floats -> element i of the three terms. CLAMP: values beyond bfloat16's
-// largest (a finite float32 there would round to infinity) take that value as their first term; an infinity then
-// ends up in l, which only meets the other operand's h, so that products with it stay infinite (NaN against 0)
-// as in float32, and a NaN reaches l the same way.
+// Element i of a register array of 8 floats -> element i of the three terms.
 // Two elements at a time, so that one v_cvt_pk_bf16_f32 rounds both and the rounded values are read back from its result
 // (element by element the compiler converts each value a second time for the residual: 56 conversions instead of 24 for
 // 16 elements).
+// LARGE: for operands that may hold a value of 2^9 or more (large_f32). A product that overflows has to be float32's
+// infinity, but a term of it such as a.h b.m may overflow with the other sign, and infinity - infinity is NaN (a key masked
+// by -3.4e38 against a query of 1002.5). So that no term can: from 2^9 on h is x truncated and m has x's sign, l rounded
+// (|l| <= 1/2 below 2^16, so that a.h b.l stays finite), from 2^16 on m is truncated too and l has x's sign; below 2^9,
+// |m| <= 1. An infinity is h = +-1, m = 0, l = +-inf: l only meets the other operand's h. The dropped products of two
+// operands between 2^9 and 2^16 are at most 2^-22 of theirs and 2^-25 on average (an emulation over two million pairs), of
+// two operands beyond 2^-21 and 2^-24; one rounding to float32 is 2^-24 and 2^-26.
+// Below 2^-110 l falls under bfloat16's smallest normal number and the split loses its low bits.
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
-template <bool CLAMP>
+__device__ __forceinline__ bool large_f32(float x) { return __builtin_fabsf(x) >= 0x1p9f; }
+// The larger of mx and |x| (mx if x is NaN) in one instruction; fmaxf would canonicalise x in another.
+__device__ __forceinline__ float max_abs(float mx, float x) {
+  return __builtin_amdgcn_fmed3f(mx, __builtin_fabsf(x), THERIA_INF);
+}
+template <bool LARGE>
 __device__ __forceinline__ void split3_pair(float x0, float x1, bf16x2_t& h, bf16x2_t& m, bf16x2_t& l) {
-  constexpr float kBig = 3.3895313892515355e38f;  // the largest finite bfloat16
-  auto big = [](float x) { return CLAMP ? __builtin_amdgcn_fmed3f(x, -kBig, kBig) : x; };
   auto lo = [](bf16x2_t p) { return __uint_as_float(__builtin_bit_cast(uint32_t, p) << 16); };
   auto hi = [](bf16x2_t p) { return __uint_as_float(__builtin_bit_cast(uint32_t, p) & 0xffff0000u); };
-  h = __builtin_convertvector((f32x2_t{big(x0), big(x1)}), bf16x2_t);
+  auto trunc = [](float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); };
+  auto first = [&](float x) {
+    if (!LARGE || !large_f32(x)) return x;
+    return __builtin_isinf(x) ? __builtin_copysignf(1.f, x) : trunc(x);
+  };
+  auto second = [&](float x, float r) {
+    if (!LARGE || !(__builtin_fabsf(x) >= 0x1p16f)) return r;
+    return __builtin_isinf(x) ? 0.f : trunc(r);
+  };
+  h = __builtin_convertvector((f32x2_t{first(x0), first(x1)}), bf16x2_t);
   const float r0 = x0 - lo(h), r1 = x1 - hi(h);
-  m = __builtin_convertvector((f32x2_t{big(r0), big(r1)}), bf16x2_t);
+  m = __builtin_convertvector((f32x2_t{second(x0, r0), second(x1, r1)}), bf16x2_t);
   l = __builtin_convertvector((f32x2_t{r0 - lo(m), r1 - hi(m)}), bf16x2_t);
 }
-template <bool CLAMP>
+template <bool LARGE>
 __device__ __forceinline__ X3Frag split3(const float (&x)[8]) {
   X3Frag f;
 #pragma unroll
   for (int e = 0; e < 8; e += 2) {
     bf16x2_t h, m, l;
-    split3_pair<CLAMP>(x[e], x[e + 1], h, m, l);
+    split3_pair<LARGE>(x[e], x[e + 1], h, m, l);
     f.h[e] = h[0], f.h[e + 1] = h[1];
     f.m[e] = m[0], f.m[e + 1] = m[1];
     f.l[e] = l[0], f.l[e + 1] = l[1];
@@ -526,8 +545,14 @@ struct Ops<float, DP> {
   }
   __device__ __forceinline__ static F frag(const Raw& r) {
     const float x[8] = {r.a[0], r.a[1], r.a[2], r.a[3], r.b[0], r.b[1], r.b[2], r.b[3]};
-    return split3<true>(x);
+    F f = split3<false>(x);
+    float mx = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mx = max_abs(mx, x[e]);
+    if (large_f32(mx)) f = split3<true>(x);
+    return f;
   }
+  // (P, dS and their like: not LARGE. An infinity among them gives NaN, as its sum with the row's other keys would.)
   __device__ __forceinline__ static F acc(const f32x16_t& a, int c) {
     float x[8];
 #pragma unroll
@@ -541,27 +566,33 @@ struct Ops<float, DP> {
   template <int ROWS, int NT>
   __device__ __forceinline__ static void store(const TileStage<float, ROWS, DP, NT>& st, float* lds) {
     using S = TileStage<float, ROWS, DP, NT>;
+    float mx = 0.f;
+    auto put = [&](auto large_tag) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < S::PER; ++i) {
-      const int ch = (int)threadIdx.x + i * NT;
-      if (S::NCH % NT == 0 || ch < S::NCH) {
-        const int row = ch / S::CPR, col = (ch % S::CPR) * S::VEC;
-        const f32x4_t x = __builtin_bit_cast(f32x4_t, st.r[i]);
-        bf16x4_t h, m, l;
+      for (int i = 0; i < S::PER; ++i) {
+        const int ch = (int)threadIdx.x + i * NT;
+        if (S::NCH % NT == 0 || ch < S::NCH) {
+          const int row = ch / S::CPR, col = (ch % S::CPR) * S::VEC;
+          const f32x4_t x = __builtin_bit_cast(f32x4_t, st.r[i]);
+          bf16x4_t h, m, l;
 #pragma unroll
-        for (int e = 0; e < 4; e += 2) {
-          bf16x2_t h2, m2, l2;
-          split3_pair<true>(x[e], x[e + 1], h2, m2, l2);
-          h[e] = h2[0], h[e + 1] = h2[1];
-          m[e] = m2[0], m[e + 1] = m2[1];
-          l[e] = l2[0], l[e + 1] = l2[1];
+          for (int e = 0; e < 4; e += 2) {
+            bf16x2_t h2, m2, l2;
+            split3_pair<decltype(large_tag)::value>(x[e], x[e + 1], h2, m2, l2);
+            h[e] = h2[0], h[e + 1] = h2[1];
+            m[e] = m2[0], m[e + 1] = m2[1];
+            l[e] = l2[0], l[e + 1] = l2[1];
+            if constexpr (!decltype(large_tag)::value) mx = max_abs(max_abs(mx, x[e]), x[e + 1]);
+          }
+          char* p = reinterpret_cast<char*>(lds + row * PITCH) + 2 * col;
+          *reinterpret_cast<i16x4_t*>(p) = __builtin_bit_cast(i16x4_t, h);
+          *reinterpret_cast<i16x4_t*>(p + 2 * DP) = __builtin_bit_cast(i16x4_t, m);
+          *reinterpret_cast<i16x4_t*>(p + 4 * DP) = __builtin_bit_cast(i16x4_t, l);
         }
-        char* p = reinterpret_cast<char*>(lds + row * PITCH) + 2 * col;
-        *reinterpret_cast<i16x4_t*>(p) = __builtin_bit_cast(i16x4_t, h);
-        *reinterpret_cast<i16x4_t*>(p + 2 * DP) = __builtin_bit_cast(i16x4_t, m);
-        *reinterpret_cast<i16x4_t*>(p + 4 * DP) = __builtin_bit_cast(i16x4_t, l);
       }
-    }
+    };
+    put(std::false_type{});
+    if (large_f32(mx)) put(std::true_type{});  // the same places again
   }
 };
 
