@@ -69,11 +69,7 @@ def test_small_backward_equals_general_kernels(dt, D, std, hip_device):
             dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
             delta = torch.empty_like(lse)
             prob = _ops._problem(q, k, scale, causal)
-            if dt == F32:  # the general entry forms dO . O from a given O: take the row term the combined one wrote
-                delta.copy_(got[3])
-                _ops.bwd_dq(prob, q, k, v, None, False, do, lse, delta, dq)
-            else:
-                _ops.bwd_dq(prob, q, k, v, o, o_f32, do, lse, delta, dq)
+            _ops.bwd_dq(prob, q, k, v, o, o_f32, do, lse, delta, dq)
             _ops.bwd_dkdv(prob, q, k, v, do, lse, delta, dk, dv)
             for name, a, b in zip(("dQ", "dK", "dV", "delta"), got, (dq, dk, dv, delta)):
                 bars.close(a, b.double().cpu(), what=f"{name} causal={causal} o_f32={o_f32}", **bars.tol(dt))
