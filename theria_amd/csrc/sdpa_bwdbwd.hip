@@ -282,10 +282,7 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
     auto sweep = [&](auto pass_tag) __attribute__((always_inline)) {
       auto step = [&](auto mask_tag, int kt) __attribute__((always_inline)) {
         __syncthreads();
-        OP::store(gsK, sK0);
-        OP::store(gsV, sV0);
-        if (has_gk) OP::store(gsgK, sgK0);
-        if (has_gv) OP::store(gsgV, sgV0);
+        OP::store(gsK, sK0, gsV, sV0, gsgK, has_gk ? sgK0 : nullptr, gsgV, has_gv ? sgV0 : nullptr);
         __syncthreads();
         if (kt + 1 < nkt) prefetch((kt + 1) * BN);
         compute(pass_tag, mask_tag, kt, sK0, sV0, sgK0, sgV0);
@@ -307,10 +304,7 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
     } else {
       if (sizeof(T) == 2 && nkt > 0) {
         // centre pre-pass over tile 0 (the loop stages the same registers again)
-        OP::store(gsK, sK0);
-        OP::store(gsV, sV0);
-        if (has_gk) OP::store(gsgK, sgK0);
-        if (has_gv) OP::store(gsgV, sgV0);
+        OP::store(gsK, sK0, gsV, sV0, gsgK, has_gk ? sgK0 : nullptr, gsgV, has_gv ? sgV0 : nullptr);
         __syncthreads();
         compute(pre_pass, std::true_type{}, 0, sK0, sV0, sgK0, sgV0);
         set_centre();
@@ -596,9 +590,7 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
     if (nqt > 0) prefetch(0);
     auto step = [&](auto diag_tag, int it) __attribute__((always_inline)) {
       __syncthreads();
-      OP::store(gsQ, sQ0);
-      OP::store(gsO, sdO0);
-      if (has_gq) OP::store(gsgQ, sgQ0);
+      OP::store(gsQ, sQ0, gsO, sdO0, gsgQ, has_gq ? sgQ0 : nullptr);
       store_rows(sRow0);
       __syncthreads();
       if (it + 1 < nqt) prefetch(it + 1);
@@ -611,9 +603,7 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
     if (pk_any)
       peaked_tiles([&](int it) __attribute__((always_inline)) {
         prefetch(it);
-        OP::store(gsQ, sQ0);
-        OP::store(gsO, sdO0);
-        if (has_gq) OP::store(gsgQ, sgQ0);
+        OP::store(gsQ, sQ0, gsO, sdO0, gsgQ, has_gq ? sgQ0 : nullptr);
         store_rows(sRow0);
       });
   }

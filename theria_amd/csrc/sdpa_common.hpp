@@ -26,8 +26,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <type_traits>
-
 namespace theria {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -265,6 +263,7 @@ __device__ __forceinline__ typename Mfma<T>::frag_t gload_frag(const T* base, in
 // Out-of-range rows and columns are zero, so every LDS column < DP is defined.
 template <typename T, int ROWS, int DP, int NT>
 struct TileStage {
+  static constexpr int THREADS = NT;
   static constexpr int VEC = 16 / (int)sizeof(T);
   static constexpr int CPR = DP / VEC;
   static constexpr int NCH = ROWS * CPR;
@@ -492,9 +491,11 @@ struct Ops {
   __device__ __forceinline__ static f32x16_t mma(const F& a, const F& b, f32x16_t c) {
     return MM::mma(a, b, c);
   }
-  template <int ROWS, int NT>
-  __device__ __forceinline__ static void store(const TileStage<T, ROWS, DP, NT>& st, T* lds) {
-    st.store(lds, PITCH);
+  // store(t1, lds1, t2, lds2, ...): staged tiles to LDS. A null lds is left out.
+  template <typename S, typename... A>
+  __device__ __forceinline__ static void store(const S& st, T* lds, A&&... more) {
+    if (lds) st.store(lds, PITCH);
+    if constexpr (sizeof...(more) > 0) store(more...);
   }
 };
 
@@ -563,26 +564,34 @@ struct Ops<float, DP> {
   __device__ __forceinline__ static f32x16_t mma(const F& a, const F& b, f32x16_t c) {
     return MM::template mma<SW>(a, b, c);
   }
-  template <int ROWS, int NT>
-  __device__ __forceinline__ static void store(const TileStage<float, ROWS, DP, NT>& st, float* lds) {
-    using S = TileStage<float, ROWS, DP, NT>;
+  // All the tiles as they are (their splits interleave), then again, to the same places, for a thread that met a large
+  // value in any of them.
+  template <typename... A>
+  __device__ __forceinline__ static void store(A&&... tiles) {
+    if (large_f32(put<false>(tiles...))) put<true>(tiles...);
+  }
+
+ private:
+  // Returns the largest |x| (0 if LARGE).
+  template <bool LARGE, typename S, typename... A>
+  __device__ __forceinline__ static float put(const S& st, float* lds, A&&... more) {
     float mx = 0.f;
-    auto put = [&](auto large_tag) __attribute__((always_inline)) {
+    if (lds) {
 #pragma unroll
       for (int i = 0; i < S::PER; ++i) {
-        const int ch = (int)threadIdx.x + i * NT;
-        if (S::NCH % NT == 0 || ch < S::NCH) {
+        const int ch = (int)threadIdx.x + i * S::THREADS;
+        if (S::NCH % S::THREADS == 0 || ch < S::NCH) {
           const int row = ch / S::CPR, col = (ch % S::CPR) * S::VEC;
           const f32x4_t x = __builtin_bit_cast(f32x4_t, st.r[i]);
           bf16x4_t h, m, l;
 #pragma unroll
           for (int e = 0; e < 4; e += 2) {
             bf16x2_t h2, m2, l2;
-            split3_pair<decltype(large_tag)::value>(x[e], x[e + 1], h2, m2, l2);
+            split3_pair<LARGE>(x[e], x[e + 1], h2, m2, l2);
             h[e] = h2[0], h[e + 1] = h2[1];
             m[e] = m2[0], m[e + 1] = m2[1];
             l[e] = l2[0], l[e + 1] = l2[1];
-            if constexpr (!decltype(large_tag)::value) mx = max_abs(max_abs(mx, x[e]), x[e + 1]);
+            if constexpr (!LARGE) mx = max_abs(max_abs(mx, x[e]), x[e + 1]);
           }
           char* p = reinterpret_cast<char*>(lds + row * PITCH) + 2 * col;
           *reinterpret_cast<i16x4_t*>(p) = __builtin_bit_cast(i16x4_t, h);
@@ -590,9 +599,9 @@ struct Ops<float, DP> {
           *reinterpret_cast<i16x4_t*>(p + 4 * DP) = __builtin_bit_cast(i16x4_t, l);
         }
       }
-    };
-    put(std::false_type{});
-    if (large_f32(mx)) put(std::true_type{});  // the same places again
+    }
+    if constexpr (sizeof...(more) > 0) mx = max_abs(mx, put<LARGE>(more...));
+    return mx;
   }
 };
 
