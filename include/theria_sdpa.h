@@ -167,20 +167,25 @@ int theria_sdpa_jvp(const theria_sdpa_problem_t* p, const theria_tensor_t* q, co
  * with cotangents (gq, gk, gv) of (dQ, dK, dV). Outputs out_gq, out_gk, out_gv, out_gdout.
  * The reference has no kernel for this: its HVP is a finite difference of the VJP
  * (theria/attention/hvp_utils.py:30-49) or autograd-in-backward (theria/autograd/sdpa_custom_function.py:32-53).
- * delta (the row term written by theria_sdpa_bwd) is not read and may be NULL: a pass over the keys recomputes
- * the row term into the workspace. Any cotangent may have data == NULL (zero).
- * For float32 inputs that pass also forms each row's own statistics from its float32 scores, m2 = max_j fl(S c)
- * and L2 = log2 sum_j exp2(fl(S c) - m2) with c = scale log2(e), and the row and column kernels rebuild
- * P = exp2((fl(S c) - m2) - L2) with dP formed as in that pass (lse is read only by the G_dO pass): on rows
- * whose probability sits on one key the second-order terms are differences (dP - z, Gam - r, E1 - t) that
- * P from a rounded lse would leave at ~1e-5.
- * For 16-bit inputs a pass over the keys recomputes, into the workspace, the row normaliser
- * lse + ln(sum_j P_ij) (a 16-bit forward's lse comes from rounded probabilities, so P rebuilt from it sums to
- * one only within ~2^-9) and the row term sum_j P_ij dP_ij / sum_j P_ij in float32 (delta from the 16-bit O
- * differs from it by the rounding of O); the second-order terms amplify both where they cancel. delta is
- * then not read. Query blocks holding a row flagged peaked in lse are redone by a second row pass (run as
- * part of the column kernel's grid) that forms G_Q's score-gradient in float32 from the first pass's row
- * terms; those blocks and tiles enter the G_Q, G_K, G_V products as two 16-bit terms.
+ * delta (the row term written by theria_sdpa_bwd) is not read and may be NULL: the row term is formed anew.
+ * Any cotangent may have data == NULL (zero).
+ * At most 64 queries and 64 keys (float32: head dim up to 64): one launch, every row's statistics from its own
+ * scores (lse is not read). Otherwise:
+ * For float32 inputs a pass over the keys forms the row term and each row's own statistics from its float32
+ * scores, m2 = max_j fl(S c) and L2 = log2 sum_j exp2(fl(S c) - m2) with c = scale log2(e), and the row and
+ * column kernels rebuild P = exp2((fl(S c) - m2) - L2) from the same products, in the same order of rounding,
+ * with dP formed as in that pass (lse is read only by the G_dO pass): on rows whose probability sits on one key
+ * the second-order terms are differences (dP - z, Gam - r, E1 - t) that P from a rounded lse, or scores rounded
+ * another way, would leave at ~1e-5.
+ * For 16-bit inputs the row normaliser lse + ln(sum_j P_ij) (a 16-bit forward's lse comes from rounded
+ * probabilities, so P rebuilt from it sums to one only within ~2^-9) and the row term sum_j P_ij dP_ij /
+ * sum_j P_ij are formed anew into the workspace (delta from the 16-bit O differs from it by the rounding of O);
+ * the second-order terms amplify both where they cancel. Head dims that are a multiple of 8 with 16-byte-aligned
+ * views: by the first of two passes of the row kernel, which forms G_Q in the exact form for every row and G_dO
+ * (two launches in all; P, P o Gam, Gbar_S and dS as two 16-bit terms on rows flagged peaked, and on every row
+ * above head dim 64). Others: by a pass over the keys; query blocks holding a row flagged peaked are redone by a
+ * second row pass (run as part of the column kernel's grid) that forms G_Q's score gradient in float32 from the
+ * first pass's row terms; those blocks and tiles enter the G_Q, G_K, G_V products as two 16-bit terms.
  * row_ws is a caller-owned float32 workspace of 5*batch*heads*tq elements.
  */
 int theria_sdpa_bwd_bwd(const theria_sdpa_problem_t* p, const theria_tensor_t* q, const theria_tensor_t* k,

@@ -91,8 +91,8 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
   // sets spilled ~700 registers, the exact form's passes hold two. The split products spill more than v_mfma_f32_32x32x2_f32
   // did (rows ~105 -> ~220 of 512 registers, columns ~200 -> ~330) and are faster all the same. HVP of <W, O>, us, the
   // one-pass form with v_mfma_f32_32x32x2_f32 -> two passes with it -> two passes with split products: B4 H8 T700 D128
-  // 3713 -> 2593 -> 1790, B2 H16 T1000 D80 5333 -> 4027 -> 2635, causal 4584 -> 3099 -> 2249, B16 H16 T300 D128 causal
-  // 4573 -> 3301 -> 2202.
+  // 3708 -> 2593 -> 1683, B2 H16 T1000 D80 5323 -> 4027 -> 2514, causal 4578 -> 3099 -> 2281, B16 H16 T300 D128 causal
+  // 4560 -> 3301 -> 2224.
   constexpr bool TWO = sizeof(T) == 4 && DP == 128;
   const bool two_pass = TWO || (!EXACT && LIGHT_OK && flagged && light);
   if (EXACT && !exact) return;

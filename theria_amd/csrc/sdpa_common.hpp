@@ -75,11 +75,11 @@ template <> struct Mfma<_Float16> {
 // matrix pipe where eight v_mfma_f32_32x32x2_f32 take 8 x 64, and rounds the accumulator fewer times.
 // Every float32 kernel forms its products this way and in this order: the kernels of one call rebuild each other's
 // scores and probabilities (lse, the row statistics of the double backward), and differences of values rounded two
-// ways do not cancel (row statistics from v_mfma_f32_32x32x2_f32 beside split products here: G_V of a peaked D128
-// problem off by 9 times the 1e-5 bar). Ops below is the one place that chooses the product.
-// Measured against v_mfma_f32_32x32x2_f32 throughout: forward + backward of B2 H16 T1000 D64 458 -> 282 us, the HVP of
-// B8 H8 T512 D64 785 -> 512 us, of B4 H8 T700 D128 3713 -> 1790 us; relative error against float64 7.3e-7 -> 6.4e-7,
-// 7.4e-7 -> 6.2e-7 and 8.8e-7 -> 7.5e-7, and not larger in any of eight second-order calls at D 72..128.
+// ways do not cancel (row statistics from v_mfma_f32_32x32x2_f32 beside split products here: G_Q of a peaked D96 problem
+// off by 2.0e-4 where float32 PyTorch is off by 4.9e-5). Ops below is the one place that chooses the product.
+// Measured against v_mfma_f32_32x32x2_f32 throughout: forward + backward of B2 H16 T1000 D64 461 -> 285 us, the HVP of
+// B8 H8 T512 D64 786 -> 525 us, of B4 H8 T700 D128 3708 -> 1683 us; relative error against float64 7.4e-7 -> 6.4e-7,
+// 7.4e-7 -> 6.2e-7 and 8.7e-7 -> 7.5e-7, and not larger in any of eight second-order calls at D 72..128.
 struct X3Frag {
   bf16x8_t h, m, l;
 };

@@ -29,7 +29,7 @@ constexpr int FWD_MAX_SPLITS = 64;  // what the combining kernel takes
 namespace theria {
 
 // NW waves per workgroup: four, or two for at most 64 queries (QT = 1), where two of four would have no rows (us, four
-// -> two waves: float32 B400 H4 T64 D16 18.6 -> 17.3, B128 H8 T32 D32 12.6 -> 9.5, bfloat16 B64 H8 T64 D128 13.2 -> 9.4).
+// -> two waves: float32 B400 H4 T64 D16 17.9 -> 13.8, B128 H8 T32 D32 11.7 -> 8.1, bfloat16 B64 H8 T64 D128 13.5 -> 9.1).
 // SPLIT: one part of the keys per workgroup (FwdParams::nsplit), no causal mask.
 template <typename T, int DP, bool CAUSAL, int QT, int BN, int NW = 4, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NW, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel(const FwdParams p) {
@@ -339,11 +339,11 @@ template <int DP> constexpr int fwd_qt(int T) { return (FWD_QT_MAX >= 2 && DP <=
 // take three times as long: half), in parts of at least two 64-key tiles, one part per idle CU. The split costs the
 // partial rows' round trip and a launch, 5-8 us, so short sweeps stay whole: at 16-bit head dims up to 64 a tile takes
 // ~0.7 us and the lines cross at 20 tiles (us, whole -> split: B1 H8 T1024 M1024 D64 14.1 -> 16.2, B1 H4 T2048 M2048 D64
-// 24.0 -> 19.1), at larger ones at 10 (B1 H2 T1024 M700 D128 16.3 -> 12.8), and for float32 and the general kernel's 16-bit
-// blocks (up to 128 queries) at 8 (float32 B1 H4 T300 M500 D32 19.8 -> 11.1, B1 H16 T100 M500 D128 18.7 -> 11.6). Two parts
-// only pay in float32 (bfloat16 B1 H8 T2048 M2048 D128 36.5 -> 37.8, float32 B1 H16 T700 M700 D128 78.6 -> 56.2).
-// B1 H16 T100 M6000 D128 bfloat16: 169 -> 21.6 us (16 workgroups -> 256; 50 MB read once, 10 us at a copy's rate); B1 H4
-// T512 M8192 D64 81.6 -> 18.9 us.
+// 24.0 -> 19.8), at larger ones at 10 (B1 H2 T1024 M700 D128 16.0 -> 13.4), and for float32 and the general kernel's 16-bit
+// blocks (up to 128 queries) at 8 (float32 B1 H4 T300 M500 D32 18.5 -> 11.6, B1 H16 T100 M500 D128 18.6 -> 12.0). Two parts
+// only pay in float32 (bfloat16 B1 H8 T2048 M2048 D128 36.5 -> 37.8, float32 B1 H16 T700 M700 D128 71.6 -> 53.1).
+// B1 H16 T100 M6000 D128 bfloat16: 148-168 -> 21 us (16 workgroups -> 256; 50 MB read once, 10 us at a copy's rate); B1 H4
+// T512 M8192 D64 81.0 -> 18.6 us.
 int fwd_splits(const Shape& s) {
   if (s.causal || s.T < 1) return 1;
   const int64_t blocks = (int64_t)((s.T + 127) / 128) * s.B * s.H, tiles = (s.M + 63) / 64, cus = device_cu_count();
@@ -392,7 +392,7 @@ struct FwdLauncher {
     // Two query tiles per wave only for 16-bit inputs: with float32 fragments (twice the registers)
     // that variant spills ~150 VGPRs and runs at half the one-tile rate.
     // Two-wave workgroups where four-wave ones (two of whose waves have no rows) would not all be resident at once;
-    // below that the wider workgroup stages its tiles sooner (float32 D64 B24 H16 T52: 12.0 against 14.5 us).
+    // below that the wider workgroup stages its tiles sooner (float32 D64 B24 H16 T52: 10.7 against 13.0 us).
     const int64_t nbh = (int64_t)p.s.B * p.s.H;
     if (p.s.T >= 1 && p.s.T <= 64 && nbh > (int64_t)device_cu_count() * (DP <= 64 ? 2 : 1)) {
       hipLaunchKernelGGL((fwd_kernel<T, DP, CAUSAL, 1, 64, 2>), dim3((unsigned)nbh), dim3(128), 0, st, p);

@@ -38,8 +38,8 @@ template <typename T, int DP, bool CAUSAL, bool HAS_O, int NW = 4>
 __global__ __launch_bounds__(64 * NW, sizeof(T) == 4 && DP == 32 ? 2 : 1) void jvp_kernel(const JvpParams p) {
   // float32 forms its scores as the forward does, from split operands: lse was rounded with those scores, and scores of
   // another order of rounding don't cancel its error (T20 M90 D80 std 2, 2-norm against float64: 1.20e-6 -> 7.3e-7).
-  // Above head dim 64 this also beats the float32 MFMA, ~40 spilled registers included (us: B4 H8 T700 D128 266 -> 191,
-  // B16 H16 T300 D128 causal 367 -> 286, B300 H8 T20 M90 D80 426 -> 386).
+  // Above head dim 64 this also beats the float32 MFMA, ~40 spilled registers included (us: B4 H8 T700 D128 276 -> 188,
+  // B16 H16 T300 D128 causal 381 -> 282, B300 H8 T20 M90 D80 438 -> 394).
   using OP = Ops<T, DP>;
   using F = typename OP::F;
   constexpr int KC = OP::KC;
@@ -225,8 +225,8 @@ __global__ __launch_bounds__(64 * NW, sizeof(T) == 4 && DP == 32 ? 2 : 1) void j
 // two waves (64 queries, 32-key tiles) where 128-query workgroups would leave CUs idle, else G = 1 group of four waves
 // (128 queries, no exchange), which reads each tile for twice the queries (us, the one-group kernel it replaced -> G = 2 /
 // G = 1, bfloat16 D128: B2 H8 T1024 84 -> 46 / 62, B2 H16 T1024 90 -> 84 / 74, B1 H4 T8192 601 -> 511 / 457, B64 H8 T1000
-// M96 250 -> 320 / 217, B2 H8 T1024 causal 84 -> 36 / 56; one 16-bit term instead of two would take 30 to 350 us of these
-// and raise the error 1.4 times). ALL: every tangent is given (the presence tests are then
+// M96 250 -> 320 / 217, B2 H8 T1024 causal 84 -> 36 / 56; with one 16-bit term instead of two the better of each took 39, 59,
+// 354, 217 and 30 us, at 1.4 times the error). ALL: every tangent is given (the presence tests are then
 // constants, and the loop body has no branches between its products).
 template <typename T, bool CAUSAL, bool ALL, bool FD, int DP, int G>
 __global__ __launch_bounds__(DP == 64 ? 512 : 256, DP == 64 ? 2 : 1) void jvp_ksplit_kernel(const JvpParams p) {
@@ -540,7 +540,7 @@ struct JvpLauncher {
       }
     }
     // at most 64 queries, and more workgroups than CUs (one four-wave workgroup per CU is resident): float32 B400 H4
-    // T64 D16 42 -> 33 us. Not in float32 above head dim 64, where staging a tile with half the threads spills.
+    // T64 D16 37.4 -> 26.9 us. Not in float32 above head dim 64, where staging a tile with half the threads spills.
     if constexpr (!(sizeof(T) == 4 && DP == 128)) {
       if (p.s.T <= 64 && nblk > device_cu_count()) {
         hipLaunchKernelGGL((jvp_kernel<T, DP, CAUSAL, HAS_O, 2>), dim3((unsigned)nblk), dim3(128), 0, st, p);
