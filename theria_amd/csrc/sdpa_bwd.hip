@@ -157,7 +157,7 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
       constexpr bool MASK = decltype(mask_tag)::value;
       const int k0 = kt * BN;
       __syncthreads();
-      OP::store(pK, sK, pV, sV);
+      OP::store(pK, sK, true, pV, sV, true);
       __syncthreads();
       if (kt + 1 < nkt) {
         pK.load(K, p.k.sr, k0 + BN, s.M, s.D, s.vec);
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DQ_MINW : 1)) void dq_kernel(const
     constexpr bool MASK = decltype(mask_tag)::value;
     const int k0 = kt * BN;
     __syncthreads();
-    OP::store(stK, sK, stV, sV);
+    OP::store(stK, sK, true, stV, sV, true);
     __syncthreads();
     if (kt + 1 < nkt) {
       stK.load(K, p.k.sr, k0 + BN, s.M, s.D, s.vec);
@@ -471,7 +471,7 @@ __global__ __launch_bounds__(256, (DP <= 64 ? DKDV_MINW : 1)) void dkdv_kernel(c
   auto step = [&](auto mask_tag, int it) __attribute__((always_inline)) {
     const int q0 = qbeg + it * BM;
     __syncthreads();
-    OP::store(stQ, sQ, stO, sdO);
+    OP::store(stQ, sQ, true, stO, sdO, true);
     if (tid < BM) {
       sLse[tid] = pre_lse;
       sDel[tid] = pre_del;

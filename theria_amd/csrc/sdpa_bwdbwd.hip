@@ -91,8 +91,8 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
   // sets spilled ~700 registers, the exact form's passes hold two. The split products spill more than v_mfma_f32_32x32x2_f32
   // did (rows ~105 -> ~220 of 512 registers, columns ~200 -> ~330) and are faster all the same. HVP of <W, O>, us, the
   // one-pass form with v_mfma_f32_32x32x2_f32 -> two passes with it -> two passes with split products: B4 H8 T700 D128
-  // 3708 -> 2593 -> 1683, B2 H16 T1000 D80 5323 -> 4027 -> 2514, causal 4578 -> 3099 -> 2281, B16 H16 T300 D128 causal
-  // 4560 -> 3301 -> 2224.
+  // 3724 -> 2593 -> 1666, B2 H16 T1000 D80 5333 -> 4027 -> 2447, causal 4586 -> 3099 -> 2193, B16 H16 T300 D128 causal
+  // 4572 -> 3301 -> 2132.
   constexpr bool TWO = sizeof(T) == 4 && DP == 128;
   const bool two_pass = TWO || (!EXACT && LIGHT_OK && flagged && light);
   if (EXACT && !exact) return;
@@ -282,7 +282,7 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
     auto sweep = [&](auto pass_tag) __attribute__((always_inline)) {
       auto step = [&](auto mask_tag, int kt) __attribute__((always_inline)) {
         __syncthreads();
-        OP::store(gsK, sK0, gsV, sV0, gsgK, has_gk ? sgK0 : nullptr, gsgV, has_gv ? sgV0 : nullptr);
+        OP::store(gsK, sK0, true, gsV, sV0, true, gsgK, sgK0, has_gk, gsgV, sgV0, has_gv);
         __syncthreads();
         if (kt + 1 < nkt) prefetch((kt + 1) * BN);
         compute(pass_tag, mask_tag, kt, sK0, sV0, sgK0, sgV0);
@@ -304,7 +304,7 @@ __device__ __attribute__((always_inline)) inline void rows_block(const BwdBwdPar
     } else {
       if (sizeof(T) == 2 && nkt > 0) {
         // centre pre-pass over tile 0 (the loop stages the same registers again)
-        OP::store(gsK, sK0, gsV, sV0, gsgK, has_gk ? sgK0 : nullptr, gsgV, has_gv ? sgV0 : nullptr);
+        OP::store(gsK, sK0, true, gsV, sV0, true, gsgK, sgK0, has_gk, gsgV, sgV0, has_gv);
         __syncthreads();
         compute(pre_pass, std::true_type{}, 0, sK0, sV0, sgK0, sgV0);
         set_centre();
@@ -590,7 +590,7 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
     if (nqt > 0) prefetch(0);
     auto step = [&](auto diag_tag, int it) __attribute__((always_inline)) {
       __syncthreads();
-      OP::store(gsQ, sQ0, gsO, sdO0, gsgQ, has_gq ? sgQ0 : nullptr);
+      OP::store(gsQ, sQ0, true, gsO, sdO0, true, gsgQ, sgQ0, has_gq);
       store_rows(sRow0);
       __syncthreads();
       if (it + 1 < nqt) prefetch(it + 1);
@@ -603,7 +603,7 @@ __device__ __attribute__((always_inline)) inline void cols_block(const BwdBwdPar
     if (pk_any)
       peaked_tiles([&](int it) __attribute__((always_inline)) {
         prefetch(it);
-        OP::store(gsQ, sQ0, gsO, sdO0, gsgQ, has_gq ? sgQ0 : nullptr);
+        OP::store(gsQ, sQ0, true, gsO, sdO0, true, gsgQ, sgQ0, has_gq);
         store_rows(sRow0);
       });
   }

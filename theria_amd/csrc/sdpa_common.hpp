@@ -77,9 +77,9 @@ template <> struct Mfma<_Float16> {
 // scores and probabilities (lse, the row statistics of the double backward), and differences of values rounded two
 // ways do not cancel (row statistics from v_mfma_f32_32x32x2_f32 beside split products here: G_Q of a peaked D96 problem
 // off by 2.0e-4 where float32 PyTorch is off by 4.9e-5). Ops below is the one place that chooses the product.
-// Measured against v_mfma_f32_32x32x2_f32 throughout: forward + backward of B2 H16 T1000 D64 461 -> 285 us, the HVP of
-// B8 H8 T512 D64 786 -> 525 us, of B4 H8 T700 D128 3708 -> 1683 us; relative error against float64 7.4e-7 -> 6.4e-7,
-// 7.4e-7 -> 6.2e-7 and 8.7e-7 -> 7.5e-7, and not larger in any of eight second-order calls at D 72..128.
+// Measured against v_mfma_f32_32x32x2_f32 throughout: forward + backward of B2 H16 T1000 D64 461 -> 281 us, the HVP of
+// B8 H8 T512 D64 786 -> 504 us, of B4 H8 T700 D128 3724 -> 1666 us; relative error against float64 7.4e-7 -> 6.4e-7,
+// 7.4e-7 -> 6.2e-7 and 8.8e-7 -> 7.5e-7, and not larger in any of eight second-order calls at D 72..128.
 struct X3Frag {
   bf16x8_t h, m, l;
 };
@@ -418,7 +418,7 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 // Two elements at a time, so that one v_cvt_pk_bf16_f32 rounds both and the rounded values are read back from its result
 // (element by element the compiler converts each value a second time for the residual: 56 conversions instead of 24 for
 // 16 elements).
-// LARGE: for operands that may hold a value of 2^9 or more (large_f32). A product that overflows has to be float32's
+// LV: 0 for |x| below 2^9, 1 below 2^16, 2 for every x; a value is split alike at every level that takes it. A product that overflows has to be float32's
 // infinity, but a term of it such as a.h b.m may overflow with the other sign, and infinity - infinity is NaN (a key masked
 // by -3.4e38 against a query of 1002.5). So that no term can: from 2^9 on h is x truncated and m has x's sign, l rounded
 // (|l| <= 1/2 below 2^16, so that a.h b.l stays finite), from 2^16 on m is truncated too and l has x's sign; below 2^9,
@@ -427,36 +427,38 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 // two operands beyond 2^-21 and 2^-24; one rounding to float32 is 2^-24 and 2^-26.
 // Below 2^-110 l falls under bfloat16's smallest normal number and the split loses its low bits.
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ bool large_f32(float x) { return __builtin_fabsf(x) >= 0x1p9f; }
+constexpr float kLarge1 = 0x1p9f, kLarge2 = 0x1p16f;
 // The larger of mx and |x| (mx if x is NaN) in one instruction; fmaxf would canonicalise x in another.
 __device__ __forceinline__ float max_abs(float mx, float x) {
   return __builtin_amdgcn_fmed3f(mx, __builtin_fabsf(x), THERIA_INF);
 }
-template <bool LARGE>
+template <int LV>
 __device__ __forceinline__ void split3_pair(float x0, float x1, bf16x2_t& h, bf16x2_t& m, bf16x2_t& l) {
   auto lo = [](bf16x2_t p) { return __uint_as_float(__builtin_bit_cast(uint32_t, p) << 16); };
   auto hi = [](bf16x2_t p) { return __uint_as_float(__builtin_bit_cast(uint32_t, p) & 0xffff0000u); };
   auto trunc = [](float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); };
   auto first = [&](float x) {
-    if (!LARGE || !large_f32(x)) return x;
-    return __builtin_isinf(x) ? __builtin_copysignf(1.f, x) : trunc(x);
+    if (LV == 0) return x;
+    if (LV == 2 && __builtin_isinf(x)) return __builtin_copysignf(1.f, x);
+    return __builtin_fabsf(x) >= kLarge1 ? trunc(x) : x;
   };
   auto second = [&](float x, float r) {
-    if (!LARGE || !(__builtin_fabsf(x) >= 0x1p16f)) return r;
-    return __builtin_isinf(x) ? 0.f : trunc(r);
+    if (LV < 2) return r;
+    if (__builtin_isinf(x)) return 0.f;
+    return __builtin_fabsf(x) >= kLarge2 ? trunc(r) : r;
   };
   h = __builtin_convertvector((f32x2_t{first(x0), first(x1)}), bf16x2_t);
   const float r0 = x0 - lo(h), r1 = x1 - hi(h);
   m = __builtin_convertvector((f32x2_t{second(x0, r0), second(x1, r1)}), bf16x2_t);
   l = __builtin_convertvector((f32x2_t{r0 - lo(m), r1 - hi(m)}), bf16x2_t);
 }
-template <bool LARGE>
+template <int LV>
 __device__ __forceinline__ X3Frag split3(const float (&x)[8]) {
   X3Frag f;
 #pragma unroll
   for (int e = 0; e < 8; e += 2) {
     bf16x2_t h, m, l;
-    split3_pair<LARGE>(x[e], x[e + 1], h, m, l);
+    split3_pair<LV>(x[e], x[e + 1], h, m, l);
     f.h[e] = h[0], f.h[e + 1] = h[1];
     f.m[e] = m[0], f.m[e + 1] = m[1];
     f.l[e] = l[0], f.l[e + 1] = l[1];
@@ -491,10 +493,11 @@ struct Ops {
   __device__ __forceinline__ static f32x16_t mma(const F& a, const F& b, f32x16_t c) {
     return MM::mma(a, b, c);
   }
-  // store(t1, lds1, t2, lds2, ...): staged tiles to LDS. A null lds is left out.
+  // store(t1, lds1, has1, t2, lds2, has2, ...): the staged tiles that are there to LDS. (Flags, not null pointers: the
+  // address of an LDS array is compared at run time.)
   template <typename S, typename... A>
-  __device__ __forceinline__ static void store(const S& st, T* lds, A&&... more) {
-    if (lds) st.store(lds, PITCH);
+  __device__ __forceinline__ static void store(const S& st, T* lds, bool has, A&&... more) {
+    if (has) st.store(lds, PITCH);
     if constexpr (sizeof...(more) > 0) store(more...);
   }
 };
@@ -546,37 +549,45 @@ struct Ops<float, DP> {
   }
   __device__ __forceinline__ static F frag(const Raw& r) {
     const float x[8] = {r.a[0], r.a[1], r.a[2], r.a[3], r.b[0], r.b[1], r.b[2], r.b[3]};
-    F f = split3<false>(x);
     float mx = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) mx = max_abs(mx, x[e]);
-    if (large_f32(mx)) f = split3<true>(x);
+    F f = split3<0>(x);
+    if (__builtin_expect(__any(mx >= kLarge1), 0)) f = split3<2>(x);
     return f;
   }
-  // (P, dS and their like: not LARGE. An infinity among them gives NaN, as its sum with the row's other keys would.)
+  // (P, dS and their like: always at level 0. An infinity among them gives NaN, as its sum with the row's other keys would.)
   __device__ __forceinline__ static F acc(const f32x16_t& a, int c) {
     float x[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) x[e] = a[8 * c + e];
-    return split3<false>(x);
+    return split3<0>(x);
   }
   template <bool SW = false>
   __device__ __forceinline__ static f32x16_t mma(const F& a, const F& b, f32x16_t c) {
     return MM::template mma<SW>(a, b, c);
   }
-  // All the tiles as they are (their splits interleave), then again, to the same places, for a thread that met a large
-  // value in any of them.
+  // All the tiles of a step in one call, so that their splits interleave: at level 0, then again, to the same places, for a
+  // thread that met a larger value in any of them, in a block out of the loop's line. Operands of 2^9 and more throughout
+  // cost 1 to 20% (forward B2 H16 T1000 D64 59 -> 69 us, double backward 630 -> 716); splitting at the right level at once
+  // would save most of that and costs the usual operands 2 to 4%, since nothing can start before the look is done.
   template <typename... A>
   __device__ __forceinline__ static void store(A&&... tiles) {
-    if (large_f32(put<false>(tiles...))) put<true>(tiles...);
+    const float mx = put<0>(tiles...);
+    if (__builtin_expect(__any(mx >= kLarge1), 0)) {  // uniform
+      if (mx >= kLarge2)
+        put<2>(tiles...);
+      else if (mx >= kLarge1)
+        put<1>(tiles...);
+    }
   }
 
  private:
-  // Returns the largest |x| (0 if LARGE).
-  template <bool LARGE, typename S, typename... A>
-  __device__ __forceinline__ static float put(const S& st, float* lds, A&&... more) {
+  // Returns the largest |x| (level 0).
+  template <int LV, typename S, typename... A>
+  __device__ __forceinline__ static float put(const S& st, float* lds, bool has, A&&... more) {
     float mx = 0.f;
-    if (lds) {
+    if (has) {
 #pragma unroll
       for (int i = 0; i < S::PER; ++i) {
         const int ch = (int)threadIdx.x + i * S::THREADS;
@@ -587,11 +598,11 @@ struct Ops<float, DP> {
 #pragma unroll
           for (int e = 0; e < 4; e += 2) {
             bf16x2_t h2, m2, l2;
-            split3_pair<LARGE>(x[e], x[e + 1], h2, m2, l2);
+            split3_pair<LV>(x[e], x[e + 1], h2, m2, l2);
             h[e] = h2[0], h[e + 1] = h2[1];
             m[e] = m2[0], m[e + 1] = m2[1];
             l[e] = l2[0], l[e + 1] = l2[1];
-            if constexpr (!LARGE) mx = max_abs(max_abs(mx, x[e]), x[e + 1]);
+            if constexpr (LV == 0) mx = max_abs(max_abs(mx, x[e]), x[e + 1]);
           }
           char* p = reinterpret_cast<char*>(lds + row * PITCH) + 2 * col;
           *reinterpret_cast<i16x4_t*>(p) = __builtin_bit_cast(i16x4_t, h);
@@ -600,7 +611,7 @@ struct Ops<float, DP> {
         }
       }
     }
-    if constexpr (sizeof...(more) > 0) mx = max_abs(mx, put<LARGE>(more...));
+    if constexpr (sizeof...(more) > 0) mx = max_abs(mx, put<LV>(more...));
     return mx;
   }
 };

@@ -92,7 +92,7 @@ __global__ __launch_bounds__(64 * NW, (DP <= 64 ? FWD_MINW : 1)) void fwd_kernel
     constexpr bool MASK = decltype(mask_tag)::value;
     const int k0 = kt * BN;
     __syncthreads();
-    OP::store(stK, sK, stV, sV);
+    OP::store(stK, sK, true, stV, sV, true);
     __syncthreads();
     if (kt + 1 < nkt) {
       stK.load_any(K, p.k.sr, k0 + BN, M, s.D, s.vec);

@@ -169,7 +169,7 @@ __global__ __launch_bounds__(64 * NW, sizeof(T) == 4 && DP == 32 ? 2 : 1) void j
     if (nkt > 0) prefetch(0);
     auto step = [&](auto mask_tag, int kt) __attribute__((always_inline)) {
       __syncthreads();
-      OP::store(gK, sK0, gV, sV0, gtK, has_tk ? stK0 : nullptr, gtV, has_tv ? stV0 : nullptr);
+      OP::store(gK, sK0, true, gV, sV0, true, gtK, stK0, has_tk, gtV, stV0, has_tv);
       __syncthreads();
       if (kt + 1 < nkt) prefetch((kt + 1) * BN);
       compute(mask_tag, kt, sK0, sV0, stK0, stV0);

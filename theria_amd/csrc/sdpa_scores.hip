@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256, (scores_wide<T, DP>() || DP > 64) ? 2 : 4) voi
   // Stages key tile kt (two barriers) and prefetches the next one.
   auto stage = [&](int kt) {
     __syncthreads();  // every wave is done with the previous tile
-    Tile::store(stK, sK);
+    Tile::store(stK, sK, true);
     __syncthreads();
     if (kt + 1 < nkt) stK.load_any(K, p.k.sr, (kt + 1) * BN, s.M, s.D, s.vec);
   };

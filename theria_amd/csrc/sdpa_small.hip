@@ -141,7 +141,7 @@ __global__ __launch_bounds__(128, (sizeof(T) == 4 ? DP <= 32 : DP <= 64) ? 2 : 1
       r2[c_] = has_gq ? OP::raw(GQ, p.gq.sr, my, s.T, c_, s.D, s.vec) : typename OP::Raw{};
     }
     if (PRE) load_q_side();
-    OP::store(a, tile[0], c, tile[1], d, has_gk ? tile[2] : nullptr, e, has_gv ? tile[3] : nullptr);
+    OP::store(a, tile[0], true, c, tile[1], true, d, tile[2], has_gk, e, tile[3], has_gv);
   }
   __syncthreads();
 
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(128, (sizeof(T) == 4 ? DP <= 32 : DP <= 64) ? 2 : 1
     gvf[c_] = has_gv ? OP::cols(tile[3], my, c_) : F{};
   }
   __syncthreads();  // both waves are done with the key-side tiles
-  OP::store(qs, tile[0], os, tile[1], gs_, has_gq ? tile[2] : nullptr);
+  OP::store(qs, tile[0], true, os, tile[1], true, gs_, tile[2], has_gq);
   __syncthreads();
   if (w0 >= s.M) return;
 
@@ -341,7 +341,7 @@ __global__ __launch_bounds__(128, (sizeof(T) == 4 ? DP <= 64 : true) ? 2 : 1) vo
       r1[c_] = OP::raw(dO, p.dout.sr, my, s.T, c_, s.D, s.vec);
     }
     if (PRE) load_q_side();
-    OP::store(a, tile[0], c, tile[1]);
+    OP::store(a, tile[0], true, c, tile[1], true);
   }
   // (a barrier of the workgroup either way)
   bool exact = true;
@@ -438,7 +438,7 @@ __global__ __launch_bounds__(128, (sizeof(T) == 4 ? DP <= 64 : true) ? 2 : 1) vo
     vf[c_] = OP::cols(tile[1], my, c_);
   }
   __syncthreads();  // both waves are done with the key-side tiles
-  OP::store(qs, tile[0], os, tile[1]);
+  OP::store(qs, tile[0], true, os, tile[1], true);
   __syncthreads();
   if (w0 >= s.M) return;
   f32x16_t accK[NDT], accV[NDT];
