@@ -291,8 +291,6 @@ struct TileStage {
       load(base, rs, row0, nrows, D, vec);
   }
 
-  // REPEAT: rows past the end read as the last one (nrows > 0) in place of zero.
-  template <bool REPEAT = false>
   __device__ __forceinline__ void load(const T* base, int64_t rs, int row0, int nrows, int D, bool vec) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -300,7 +298,7 @@ struct TileStage {
       i16x8_t v = {0, 0, 0, 0, 0, 0, 0, 0};
       if (NCH % NT == 0 || ch < NCH) {
         const int row = ch / CPR, col = (ch % CPR) * VEC;
-        const int grow = REPEAT ? min(row0 + row, nrows - 1) : row0 + row;
+        const int grow = row0 + row;
         if (grow < nrows && col < D) {
           const T* p = base + (int64_t)grow * rs + col;
           if (vec && col + VEC <= D) {

@@ -118,15 +118,14 @@ __global__ __launch_bounds__(128, (sizeof(T) == 4 ? DP <= 32 : DP <= 64) ? 2 : 1
   const float c2 = s.scale * kLog2e;
   const int w0 = 32 * wave, my = w0 + li;  // this wave's first row (query or key) and this lane's
 
-  // Every load of the row phase in flight together, and (PRE: where the registers allow) the column phase's tiles. Query
-  // rows past the end repeat the last one: a score of a zero row against an infinite key would be NaN, and their P is 0.
+  // Every load of the row phase in flight together, and (PRE: where the registers allow) the column phase's tiles.
   constexpr bool PRE = DP <= 32;
   typename K_::Stage qs, os, gs_;
   typename OP::Raw r0[NKC], r1[NKC], r2[NKC];
   auto load_q_side = [&]() {
-    qs.template load<true>(Q, p.q.sr, 0, s.T, s.D, s.vec);
-    os.template load<true>(dO, p.dout.sr, 0, s.T, s.D, s.vec);
-    if (has_gq) gs_.template load<true>(GQ, p.gq.sr, 0, s.T, s.D, s.vec);
+    qs.load(Q, p.q.sr, 0, s.T, s.D, s.vec);
+    os.load(dO, p.dout.sr, 0, s.T, s.D, s.vec);
+    if (has_gq) gs_.load(GQ, p.gq.sr, 0, s.T, s.D, s.vec);
   };
   {
     typename K_::Stage a, c, d, e;
@@ -289,6 +288,11 @@ __global__ __launch_bounds__(128, (sizeof(T) == 4 ? DP <= 32 : DP <= 64) ? 2 : 1
         dp[r] = pv * dz;                           // dS
       }
     }
+    if (32 * t + 32 > s.T) {  // rows past the end: P = 0, but the score of their zeros against an infinite key is NaN
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (32 * t + acc_row(r, g) >= s.T) gm[r] = w[r] = dp[r] = 0.f;
+    }
 #pragma unroll
     for (int cc = 0; cc < NPC; ++cc) {
       const auto gs = K_::terms(w, cc), ds = K_::terms(dp, cc), gd = K_::terms(gm, cc);
@@ -327,8 +331,8 @@ __global__ __launch_bounds__(128, (sizeof(T) == 4 ? DP <= 64 : true) ? 2 : 1) vo
   typename K_::Stage qs, os;
   typename OP::Raw r0[NKC], r1[NKC];
   auto load_q_side = [&]() {
-    qs.template load<true>(Q, p.q.sr, 0, s.T, s.D, s.vec);
-    os.template load<true>(dO, p.dout.sr, 0, s.T, s.D, s.vec);
+    qs.load(Q, p.q.sr, 0, s.T, s.D, s.vec);
+    os.load(dO, p.dout.sr, 0, s.T, s.D, s.vec);
   };
   const float lse = my < s.T ? p.lse[row_id] : THERIA_INF;
   {
@@ -463,6 +467,11 @@ __global__ __launch_bounds__(128, (sizeof(T) == 4 ? DP <= 64 : true) ? 2 : 1) vo
         sc[r] = pv;
         dp[r] = pv * (dp[r] - z4[e]);
       }
+    }
+    if (32 * t + 32 > s.T) {  // as in small_bwdbwd_kernel
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (32 * t + acc_row(r, g) >= s.T) sc[r] = dp[r] = 0.f;
     }
 #pragma unroll
     for (int cc = 0; cc < NPC; ++cc) {
