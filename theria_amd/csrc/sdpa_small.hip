@@ -17,9 +17,9 @@
 // terms (hi + lo), as the general kernels do on peaked rows. P = exp2(fl(S c) - max) / sum from the row's own scores
 // in the double backward (the given lse is not needed there), exp(S - lse) in the backward.
 // GPU time, general kernels (their float32 products still on v_mfma_f32_32x32x2_f32) -> here (us; backward / double
-// backward): float32 B400 H4 T64 D16 93 / 278 -> 30 / 54, float32 B64 H8 T64 D64 65 / 188 -> 31 / 89, float32 B2 H2 T16 D8
-// 13.8 / 30.8 -> 8.4 / 12.0, bfloat16 B64 H8 T64 D64 32 / 49 -> 20 / 29, bfloat16 B512 H8 T64 D128 causal 510 / 1257 ->
-// 169 / 397, bfloat16 B1 H1 T64 D64 17.7 / 23.4 -> 11.2 / 18.8 (faster at every one of 20 shapes tried). What bounds it: one workgroup's chain of loads, products and
+// backward): float32 B400 H4 T64 D16 94 / 279 -> 29 / 54, float32 B64 H8 T64 D64 65 / 188 -> 30 / 80, float32 B2 H2 T16 D8
+// 13.5 / 31.0 -> 8.5 / 11.7, bfloat16 B64 H8 T64 D64 32 / 49 -> 21 / 27, bfloat16 B512 H8 T64 D128 causal 509 / 1268 ->
+// 148 / 386, bfloat16 B1 H1 T64 D64 17.7 / 23.2 -> 11.2 / 18.3 (faster at every one of 20 shapes tried). What bounds it: one workgroup's chain of loads, products and
 // exchanges (~12 us) times the rounds the registers and LDS leave (2 waves per SIMD; float32 D64, 104 KB, one workgroup
 // per CU).
 // DP = 16 exists only here: one k chunk, and half of the 32-wide output tile unused.
